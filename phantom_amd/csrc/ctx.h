@@ -115,6 +115,10 @@ struct phsph_ctx {
   DBuf<int32_t> nd_lo, nd_hi;  // inoderange (0-based positions, inclusive)
   DBuf<int32_t> leaf_flag;   // leaf_is_active
   DBuf<int32_t> leaves;      // leaf node ids
+  DBuf<int32_t> tg_lo;       // tile groups: first tree position of each (one more: nlive)
+  DBuf<int32_t> tg_t;        // the same as indexes into the active list
+  DBuf<int32_t> tg_big;      // tile groups that need the large tile
+  int ntg = 0, tg_max = 0;   // tile groups, particles of the largest
   DBuf<int32_t> pleaf;       // tree position -> index into leaves
   DBuf<int32_t> iparts;      // inodeparts: signed 1-based original index
   DBuf<double> tx, ty, tz, th;  // treecache x, y, z, h (tree order)
@@ -134,6 +138,7 @@ struct phsph_ctx {
   // ---- neighbour search ----
   DBuf<uint32_t> gcand;      // candidate leaves per group [ngroups*caps.gcand]
   DBuf<int32_t> gncand;      // count per group
+  DBuf<double> gbox;         // bounding box and largest search h of each group (8 doubles)
   DBuf<int64_t> goff;        // exact per-group offsets into gcand (after an overflow)
   const int64_t *goff_p = nullptr;  // goff.p when the last walk used exact offsets
   DBuf<int64_t> loff;        // per-group offsets of the force lists (after an overflow)
@@ -143,6 +148,7 @@ struct phsph_ctx {
   // the density lists also serve as force lists while positions, h and the
   // active set are those of the last densityiterate
   bool dlist_reuse = false;
+  bool dlist_tile = false;          // their slots are the active list without padding
   int dlist_nact = 0, dlist_cap = 0;
   int dlist_nretry = 0;             // particles of the first attempt run again
   // first search radius of densityiterate (units of radkern*h at entry):

@@ -25,13 +25,14 @@
 // Every neighbour membership test computes r^2 = ((dx*dx + dy*dy) + dz*dz)
 // and q^2 = r^2 * (1/h)^2 with separately rounded FP64 operations, exactly
 // as the reference, so neighbour counts agree bit for bit.
-#include "stream.h"
+#include "dens_tile.h"
 
 #include <algorithm>
 #include <vector>
 #include <cstdlib>
 
-enum { DFL_CAND = 1, DFL_LIST = 2, DFL_REWALK = 4, DFL_NOCONV = 8, DFL_NEGH = 16, DFL_STACK = 32 };
+// c->counters: particles that outgrew their lists, groups for the large tile
+constexpr int CNT_REWALK = 8, CNT_BIG = 9;
 
 struct DensIn {
   const double4 *tp;  // x, y, z (treecache) and h at entry
@@ -128,29 +129,38 @@ __global__ void k_walk(DevConst dc, double rfac, const phsph_kdnode *__restrict_
 __global__ void __launch_bounds__(64)
 k_group_walk(DevConst dc, int mode, double rfac, const phsph_kdnode *__restrict__ nd,
              const double *__restrict__ hmaxn, const int32_t *__restrict__ leaf_flag,
-             const int32_t *__restrict__ act, int nact, const double *__restrict__ tx,
+             const int32_t *__restrict__ act, int nact, const int32_t *__restrict__ gt,
+             const double *__restrict__ tx,
              const double *__restrict__ ty, const double *__restrict__ tz, const double *__restrict__ hsrc,
              int ngroups, uint32_t *__restrict__ gcand, int32_t *__restrict__ gncand, const int64_t *goff,
-             int capg, int32_t *__restrict__ flags) {
+             int capg, double *__restrict__ gbox, int32_t *__restrict__ flags) {
   __shared__ int stk[WALK_STACK];
   const int g = xcd_block(blockIdx.x, gridDim.x);
   if (g >= ngroups) return;
   const size_t gbase = cand_base(goff, g, capg);
   const int gcap = cand_cap(goff, g, capg);
   const int lane = threadIdx.x;
-  const int t = g * GROUP + lane;
+  const int t0 = gt ? gt[g] : g * GROUP, t1 = gt ? gt[g + 1] : min(nact, t0 + GROUP);
+  if (t0 >= t1) {  // a tile without active particles
+    if (lane == 0) gncand[g] = 0;
+    return;
+  }
   double xl = PH_HUGE64, yl = PH_HUGE64, zl = PH_HUGE64, xh = -PH_HUGE64, yh = -PH_HUGE64, zh = -PH_HUGE64;
   double hm = 0.;
-  if (t < nact && act[t] >= 0) {
+  for (int t = t0 + lane; t < t1; t += 64) {
     const int p = act[t];
-    xl = xh = tx[p];
-    yl = yh = ty[p];
-    zl = zh = tz[p];
-    hm = hsrc[p];
+    if (p < 0) continue;
+    xl = fmin(xl, tx[p]); xh = fmax(xh, tx[p]);
+    yl = fmin(yl, ty[p]); yh = fmax(yh, ty[p]);
+    zl = fmin(zl, tz[p]); zh = fmax(zh, tz[p]);
+    hm = fmax(hm, hsrc[p]);
   }
   xl = wave_min(xl); yl = wave_min(yl); zl = wave_min(zl);
   xh = wave_max(xh); yh = wave_max(yh); zh = wave_max(zh);
   hm = wave_max(hm);
+  if (gbox && lane < GBOX)  // the box and search h for the tile kernels
+    gbox[(size_t)g * GBOX + lane] = (lane < 3) ? (lane == 0 ? xl : lane == 1 ? yl : zl)
+                                   : (lane < 6) ? (lane == 3 ? xh : lane == 4 ? yh : zh) : hm;
   const double bx = 0.5 * (xl + xh), by = 0.5 * (yl + yh), bz = 0.5 * (zl + zh);
   // half extents, rounded up so that every particle lies inside
   const double ex = 0.5 * (xh - xl) * (1. + 1e-12) + 1e-300, ey = 0.5 * (yh - yl) * (1. + 1e-12) + 1e-300,
@@ -1038,9 +1048,9 @@ int dens_trial_stats(phsph_ctx *c) {
 }
 
 // ------------------------------------------------------------------------
-int walk_groups(phsph_ctx *c, int mode, double rfac, const double *d_hsrc, const double *d_hmaxn) {
+int walk_groups(phsph_ctx *c, int mode, double rfac, const double *d_hsrc, const double *d_hmaxn, bool tiles) {
   hipStream_t s = c->stream;
-  const int ng = (c->nact + GROUP - 1) / GROUP;
+  const int ng = tiles ? c->ntg : (c->nact + GROUP - 1) / GROUP;
   c->ngroups = ng;
   c->goff_p = nullptr;
   while (c->caps.gcand > 16 && !list_fits(c, (size_t)(ng + 1) * c->caps.gcand)) c->caps.gcand /= 2;
@@ -1052,13 +1062,15 @@ int walk_groups(phsph_ctx *c, int mode, double rfac, const double *d_hsrc, const
     const int64_t *goff = exact ? c->goff.p : nullptr;
     if (!exact) PH_HIPCHECK(c, c->gcand.ensure((size_t)(ng + 1) * c->caps.gcand));
     PH_HIPCHECK(c, c->gncand.ensure(ng + 1));
+    PH_HIPCHECK(c, c->gbox.ensure((size_t)(ng + 1) * GBOX));
     int32_t zero = 0;
     PH_HIPCHECK(c, dev_set(c, c->counters.p, &zero, sizeof(int32_t)));
     if (ng > 0) {
       LaunchTimer lt(c, mode == 0 ? "walk_density" : "walk_force");
       hipLaunchKernelGGL(k_group_walk, dim3(xcd_grid(ng)), dim3(64), 0, s, c->dc, mode, rfac, c->nd.p, d_hmaxn,
-                         c->leaf_flag.p, c->act.p, c->nact, c->tx.p, c->ty.p, c->tz.p, d_hsrc, ng, c->gcand.p,
-                         c->gncand.p, goff, c->caps.gcand, c->counters.p);
+                         c->leaf_flag.p, c->act.p, c->nact, tiles ? c->tg_t.p : nullptr, c->tx.p, c->ty.p, c->tz.p,
+                         d_hsrc, ng, c->gcand.p,
+                         c->gncand.p, goff, c->caps.gcand, c->gbox.p, c->counters.p);
     }
     PH_HIPCHECK(c, hipGetLastError());
     int32_t fl = 0;
@@ -1265,6 +1277,27 @@ __global__ void k_check_hbound(int nact, const int32_t *__restrict__ act, const 
   }
   if (__ballot(bad) != 0ull && (threadIdx.x & 63) == 0) atomicOr(flag, 1);
 }
+
+// tile groups as ranges of the active list: the first active particle at or
+// after each group's first tree position
+__global__ void k_tile_ranges(int ntg, const int32_t *__restrict__ tg_lo, const int32_t *__restrict__ act, int nact,
+                              int32_t *__restrict__ tg_t) {
+  const int g = blockIdx.x * blockDim.x + threadIdx.x;
+  if (g > ntg) return;
+  const int lo = tg_lo[g];
+  int a = 0, b = nact;  // first a with act[a] >= lo
+  if (lo < nact && act[lo] == lo) {  // every particle up to here is active
+    a = lo;
+  } else {
+    while (a < b) {
+      const int m = (a + b) >> 1;
+      if (act[m] < lo) a = m + 1;
+      else b = m;
+    }
+  }
+  tg_t[g] = a;
+}
+
 int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
   hipStream_t s = c->stream;
   const int n = c->nlive;
@@ -1337,18 +1370,35 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
     rc = leaf_hmax_run(c, c->th_in.p, c->hmax0.p);
     if (rc) return rc;
   }
-  rc = pad_groups(c);
-  if (rc) return rc;
   // list capacity: it grows for the particles run again (the list memory is
   // that of the retried particles); a grown capacity is kept for later calls
   // while the lists of every active particle fit in the list budget
   // 12 bytes per entry: the entry and its squared separation
   while (c->caps.dlist > 16 && !list_fits(c, (size_t)list_cap(c->caps.dlist) * nact * 3)) c->caps.dlist /= 2;
+  // Dense active sets are searched by tiles (dens_tile.hip).  Every particle
+  // of the region that 64 active particles span is a candidate, so the tests
+  // grow with the inverse of the active fraction, while the list kernel's
+  // lanes visit only the leaves in their own reach; from half of the
+  // particles active on the tile is the faster one.  Not with a list capacity
+  // below a tile's own.
+  const bool tile = 2 * (int64_t)nact >= n && c->caps.dlist >= dens_tile_list_cap(c);
+  const bool tile_tune = tile && c->tune_mode == TUNE_PENDING && nact >= TUNE_MIN_ACTIVE;
+  if (tile) {
+    PH_HIPCHECK(c, c->tg_t.ensure((size_t)c->ntg + 1));
+    hipLaunchKernelGGL(k_tile_ranges, dim3(nblocks((size_t)c->ntg + 1, 256)), dim3(256), 0, s, c->ntg, c->tg_lo.p,
+                       c->act.p, nact, c->tg_t.p);
+  }
+  if (!tile || tile_tune) {
+    rc = pad_groups(c);
+    if (rc) return rc;
+  }
+  c->dlist_tile = tile;
   int dlist = c->caps.dlist;
   const int dlist0 = dlist;
   bool tuned_now = false, retune = false;
+  int nrewalk = 0;  // particles of the first attempt that outgrew their lists
   for (int attempt = 0; attempt < 12; attempt++) {
-    const int na = c->nact;  // active slots, padding included
+    int na = c->nact;  // active slots, padding included
     if (na == 0) break;
     // the first attempt writes the lists the force pass may use; retries
     // write buffers of their own so that those stay intact
@@ -1362,18 +1412,18 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
     PH_HIPCHECK(c, THF.ensure((size_t)na + 1));
     // only the first attempt's lists serve the force pass
     const bool widen = attempt == 0 && reusable;
-    rc = walk_groups(c, 0, rfac * lmargin, c->th_in.p, widen ? c->hmax0.p : nullptr);
-    if (rc) return rc;
-    const int ng = c->ngroups;
+    const bool by_tile = tile && attempt == 0;
     PH_HIPCHECK(c, LB.ensure((size_t)list_cap(dlist) * na + 1));
     DBuf<double> &R2B = attempt == 0 ? c->nr2 : c->nr2_r;
     if (c->tune.r2 || c->tune_mode == TUNE_PENDING) PH_HIPCHECK(c, R2B.ensure((size_t)list_cap(dlist) * na + 2));
-    hipLaunchKernelGGL(k_zero_i32, dim3(nblocks(n, 256)), dim3(256), 0, s, c->tmpi.p, n, 0);
-    int32_t zero = 0;
-    PH_HIPCHECK(c, dev_set(c, c->counters.p, &zero, sizeof(int32_t)));
-    {
-      const IterLaunch L{c, s, ng, icall, rfac, na, lmargin, dlist, widen, LB.p, R2B.p, TNL.p, THS.p, THF.p};
-      if (attempt == 0 && c->tune_mode == TUNE_PENDING && na >= TUNE_MIN_ACTIVE) {
+    int32_t zero = 0, tfl = 0;  // tfl: list overflow seen by the autotuner
+    if (!by_tile || (tile_tune && attempt == 0)) {
+      rc = walk_groups(c, 0, rfac * lmargin, c->th_in.p, widen ? c->hmax0.p : nullptr);
+      if (rc) return rc;
+      hipLaunchKernelGGL(k_zero_i32, dim3(nblocks(n, 256)), dim3(256), 0, s, c->tmpi.p, n, 0);
+      PH_HIPCHECK(c, dev_set(c, c->counters.p, &zero, sizeof(int32_t)));
+      const IterLaunch L{c, s, c->ngroups, icall, rfac, na, lmargin, dlist, widen, LB.p, R2B.p, TNL.p, THS.p, THF.p};
+      if (attempt == 0 && c->tune_mode == TUNE_PENDING && (tile_tune || na >= TUNE_MIN_ACTIVE)) {
         tuned_now = true;
         rc = tune_density_iter(c, L);  // times every configuration, keeps the fastest
         if (rc) return rc;
@@ -1381,6 +1431,29 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
         LaunchTimer lt(c, "density_iter");
         launch_dens_iter(c->tune, L);
       }
+    }
+    if (tile_tune && attempt == 0) {
+      // the configuration is for the particles that tiles leave to the list
+      // kernels; the tiles start from the unpadded active list again
+      PH_HIPCHECK(c, hipMemcpyAsync(&tfl, c->counters.p, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+      PH_HIPCHECK(c, hipMemcpyAsync(c->act.p, c->act_dens.p, sizeof(int32_t) * nact, hipMemcpyDeviceToDevice, s));
+      PH_HIPCHECK(c, hipStreamSynchronize(s));
+      c->nact = na = nact;
+      hipLaunchKernelGGL(k_zero_i32, dim3(nblocks(c->nleaves, 256)), dim3(256), 0, s, c->leaf_nits.p, c->nleaves, 0);
+    }
+    if (by_tile) {
+      rc = walk_groups(c, 0, rfac * lmargin, c->th_in.p, widen ? c->hmax0.p : nullptr, true);
+      if (rc) return rc;
+      hipLaunchKernelGGL(k_zero_i32, dim3(nblocks(n, 256)), dim3(256), 0, s, c->tmpi.p, n, 0);
+      PH_HIPCHECK(c, dev_set(c, c->counters.p, &zero, sizeof(int32_t)));
+      PH_HIPCHECK(c, dev_set(c, c->counters.p + CNT_REWALK, &zero, sizeof(int32_t)));
+      PH_HIPCHECK(c, dev_set(c, c->counters.p + CNT_BIG, &zero, sizeof(int32_t)));
+      PH_HIPCHECK(c, c->tg_big.ensure((size_t)c->ntg + 1));
+      const DensIterOut o{LB.p, list_cap(dlist), TNL.p, widen ? c->t_nlj.p : nullptr, THS.p, THF.p, c->p_nits.p, c->leaf_nits.p,
+                          c->tmpi.p, c->counters.p + CNT_REWALK, c->htraj.p, (size_t)c->htraj_stride, c->hconv.p, c->tg_big.p,
+                          c->counters.p + CNT_BIG};
+      LaunchTimer lt(c, "density_iter");
+      launch_dens_tile(c, icall, rfac, lmargin, widen ? c->hmax0.p : nullptr, o);
     }
     {
       LaunchTimer lt(c, "density_sums");
@@ -1403,20 +1476,21 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
 #undef DFIN
     }
     PH_HIPCHECK(c, hipGetLastError());
-    int32_t fl = 0;
-    PH_HIPCHECK(c, hipMemcpyAsync(&fl, c->counters.p, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+    int32_t cnt[CNT_REWALK + 1];
+    PH_HIPCHECK(c, hipMemcpyAsync(cnt, c->counters.p, sizeof(cnt), hipMemcpyDeviceToHost, s));
     PH_HIPCHECK(c, hipStreamSynchronize(s));
+    const int32_t fl = cnt[0];
     if (dbg) {
       size_t fr = 0, tot = 0;
       (void)hipMemGetInfo(&fr, &tot);
       fprintf(stderr, "phsph densityiterate: attempt %d particles %d groups %d rfac %g list %d flags %d free %.1f GiB\n",
-              attempt, na, ng, rfac, dlist, fl, fr / 1073741824.0);
+              attempt, na, c->ngroups, rfac, dlist, fl, fr / 1073741824.0);
     }
     if (fl & DFL_NOCONV) PH_RET(c, PHSPH_ERR_NOCONVERGE, "densityiterate: could not converge in density");
     // a tuning attempt whose lists overflowed (the first call on a context
     // grows the list capacity) times unrepresentative work: tune again on
     // the next large call if that call's capacity is larger
-    if (attempt == 0 && tuned_now && (fl & DFL_LIST)) retune = true;
+    if (attempt == 0 && tuned_now && ((fl | tfl) & DFL_LIST)) retune = true;
     if (fl & DFL_NEGH) PH_RET(c, PHSPH_ERR_INPUT, "densityiterate: setting negative h from hrho");
     if (attempt == 0) {
       rewalk0 = (fl & DFL_REWALK) != 0;
@@ -1430,7 +1504,7 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
         PH_HIPCHECK(c, hipMemcpyAsync(c->dretry0.p, c->tmpi.p, sizeof(int32_t) * n, hipMemcpyDeviceToDevice, s));
       }
     }
-    if (!(fl & (DFL_REWALK | DFL_LIST))) {
+    if (!(fl & (DFL_REWALK | DFL_LIST | DFL_TILE))) {
       c->nact = 0;
       break;
     }
@@ -1438,7 +1512,10 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
     if (fl & DFL_LIST) dlist *= 2;
     rc = compact_active(c, c->tmpi.p, n);
     if (rc) return rc;
-    if (attempt == 0) c->dlist_nretry = c->nact;
+    if (attempt == 0) {
+      c->dlist_nretry = c->nact;
+      nrewalk = by_tile ? cnt[CNT_REWALK] : c->nact;
+    }
     rc = pad_groups(c);
     if (rc) return rc;
   }
@@ -1459,7 +1536,7 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
   // or the lists could not serve the force pass, one level narrower when
   // none outgrew them
   if (nact > 0) {
-    const bool outgrown = rewalk0 && c->dlist_nretry * 200 > nact;
+    const bool outgrown = rewalk0 && (int64_t)nrewalk * 200 > nact;
     if (outgrown || (reusable && !c->dlist_reuse)) {
       if (c->rfac_level < 2) {
         c->rfac_floor = std::max(c->rfac_floor, c->rfac_level + 1);

@@ -1051,8 +1051,11 @@ int force_run(phsph_ctx *c, int icall, const ForceIOArgs &a, double *dtc_out, do
     PH_HIPCHECK(c, hipStreamSynchronize(s));
     reuse = (bad == 0);
   }
-  rc = pad_groups(c);
-  if (rc) return rc;
+  if (reuse && c->dlist_tile && c->nact != c->dlist_nact) reuse = false;
+  if (!(reuse && c->dlist_tile)) {  // the slots of tile lists are not padded
+    rc = pad_groups(c);
+    if (rc) return rc;
+  }
   if (reuse && c->nact != c->dlist_nact) reuse = false;
   c->force_reused_lists = reuse;
   // node hmax of the final smoothing lengths for the h_j search radius

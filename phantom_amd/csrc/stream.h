@@ -158,7 +158,9 @@ __device__ __forceinline__ int leaf_relist_hmax(int lo, int hi, double hcell, co
 // Candidate leaves of each group of 64 active particles, into c->gcand at
 // c->goff_p (exact per-group offsets after an overflow, else nullptr and the
 // uniform capacity c->caps.gcand).
-int walk_groups(phsph_ctx *c, int mode, double rfac, const double *d_hsrc, const double *d_hmaxn);
+// tiles: the groups are the tile groups of the active list (c->tg_t).
+int walk_groups(phsph_ctx *c, int mode, double rfac, const double *d_hsrc, const double *d_hmaxn,
+                bool tiles = false);
 
 // Neighbour lists: entry k of active slot t lives in segment k/16 of that
 // slot, a run of 16 entries (64 bytes) that the slot's lane fills on its own;

@@ -22,12 +22,15 @@
 //  * Children are numbered 2n, 2n+1 (Gafton & Rosswog indexing, :820-823).
 #include "stream.h"
 
+#include <algorithm>
+
 #define SUB_MAX TREE_SUB_MAX  // particles per LDS subtree
 #define SUB_BS 256
 #define SUB_QMAX 192  // >= 2*floor(SUB_MAX/(MINPART+1)) nodes per level
 
 enum { CNT_NEXT = 0, CNT_ERR = 1, CNT_FALLBACK = 2, CNT_MAXLEVEL = 3, CNT_MINLEVEL = 4, CNT_NAN = 5,
-       CNT_NLEAF = 6, CNT_LIVE = 7, CNT_NCHUNK = 8, CNT_NBIG = 9, CNT_SEQMAX = 10, CNT_N = 11 };
+       CNT_NLEAF = 6, CNT_LIVE = 7, CNT_NCHUNK = 8, CNT_NBIG = 9, CNT_SEQMAX = 10, CNT_TGMAX = 11, CNT_NTG = 12,
+       CNT_N = 13 };
 enum { TERR_NODEID = 1, TERR_QUEUE = 2, TERR_COUNT = 4 };
 
 // ------------------------------------------------------------------------
@@ -1149,13 +1152,37 @@ __global__ void k_leaf_count(const int32_t *leaf_flag, int64_t ncells, int32_t *
   block_excl_scan<256>(b, shi, &tot);
   if (threadIdx.x == 0) bcount[blockIdx.x] = tot;
 }
-__global__ void k_leaf_fill(const int32_t *leaf_flag, int64_t ncells, const int32_t *bcount, int32_t *leaves) {
+// Tile groups (tile.h): the leaf that begins its highest ancestor of at most
+// gmax particles marks that node's first tree position.
+__global__ void k_leaf_fill(const int32_t *leaf_flag, int64_t ncells, const int32_t *bcount, int32_t *leaves,
+                            const int32_t *nd_lo, const int32_t *nd_hi, int gmax, int32_t *tflag, int32_t *tmax) {
   __shared__ int shi[8];
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x + 1;
   int b = (i <= ncells) ? (leaf_flag[i] != 0) : 0;
   int tot;
   int pre = block_excl_scan<256>(b, shi, &tot);
-  if (b) leaves[bcount[blockIdx.x] + pre] = (int32_t)i;
+  int m = 0;
+  if (b) {
+    leaves[bcount[blockIdx.x] + pre] = (int32_t)i;
+    int n = (int)i;
+    while (n > 1 && nd_hi[n >> 1] - nd_lo[n >> 1] < gmax) n >>= 1;
+    if (nd_lo[n] == nd_lo[i]) {
+      tflag[nd_lo[n]] = 1;
+      m = nd_hi[n] - nd_lo[n] + 1;
+    }
+  }
+  for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o, 64));
+  if ((threadIdx.x & 63) == 0 && m > 0) atomicMax(tmax, m);
+}
+// first positions of the tile groups in tree order, and the end
+__global__ void k_tile_fill(const int32_t *tflag, int n, const int32_t *bcount, const int32_t *ntg, int32_t *tg_lo) {
+  __shared__ int shi[8];
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int b = (i < n) ? tflag[i] : 0;
+  int tot;
+  const int pre = block_excl_scan<256>(b, shi, &tot);
+  if (b) tg_lo[bcount[blockIdx.x] + pre] = i;
+  if (i == 0) tg_lo[*ntg] = n;
 }
 __global__ void k_pleaf(const int32_t *leaves, int nleaves, const int32_t *nd_lo, const int32_t *nd_hi,
                         int32_t *pleaf) {
@@ -1212,7 +1239,7 @@ int tree_build(phsph_ctx *c, double *d_xyzh, int ld, int np, const int8_t *d_iph
   // the reference seeds the bounds with particle 1 before wrapping it
   double x0[3];
   PH_HIPCHECK(c, hipMemcpyAsync(x0, d_xyzh, 3 * sizeof(double), hipMemcpyDeviceToHost, s));
-  int32_t hc[CNT_N] = {0, 0, 0, 0, 1 << 30, 0, 0, 0, 0, 0, 0};
+  int32_t hc[CNT_N] = {0, 0, 0, 0, 1 << 30, 0, 0, 0, 0, 0, 0, 0, 0};
   PH_HIPCHECK(c, dev_set(c, c->counters.p, hc, sizeof(hc)));
   PH_HIPCHECK(c, hipStreamSynchronize(s));
   {
@@ -1317,20 +1344,37 @@ int tree_build(phsph_ctx *c, double *d_xyzh, int ld, int np, const int8_t *d_iph
   c->tree_fallbacks = cnt[CNT_FALLBACK];
   // leaves in node-id order
   const unsigned nbl = nblocks(c->ncells, 256);
-  PH_HIPCHECK(c, c->tmpi2.ensure((size_t)nbl + 1));
+  const unsigned nbt = nblocks(c->nlive, 256);
+  PH_HIPCHECK(c, c->tmpi2.ensure((size_t)std::max(nbl, nbt) + 1));
+  // Nodes of a level hold about nlive / 2^level particles: the tile limit of
+  // 64 or 80 that fills wavefronts of 16 better (a mean of 60 to 76 mostly
+  // passes 64, and half nodes of 30 to 38 would leave part of a third
+  // wavefront idle; any other mean, or its half, stays below 64)
+  double mean = (double)c->nlive;
+  while (mean > 76.) mean *= 0.5;
+  const int gmax = (mean > 60.) ? 80 : 64;
+  // at most one group per leaf
+  PH_HIPCHECK(c, c->tg_lo.ensure((size_t)c->nlive + 2));
   PH_HIPCHECK(c, c->leaves.ensure(c->nlive + 1));
   PH_HIPCHECK(c, c->pleaf.ensure(c->nlive + 1));
   {
     LaunchTimer lt(c, "tree_leaves");
+    hipLaunchKernelGGL(k_fill_i32, dim3(nbt), dim3(256), 0, s, c->tmpi.p, (int64_t)c->nlive, 0);
     hipLaunchKernelGGL(k_leaf_count, dim3(nbl), dim3(256), 0, s, c->leaf_flag.p, c->ncells, c->tmpi2.p);
     hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(1024), 0, s, c->tmpi2.p, (int)nbl,
                        c->counters.p + CNT_NLEAF);
     hipLaunchKernelGGL(k_leaf_fill, dim3(nbl), dim3(256), 0, s, c->leaf_flag.p, c->ncells, c->tmpi2.p,
-                       c->leaves.p);
+                       c->leaves.p, c->nd_lo.p, c->nd_hi.p, gmax, c->tmpi.p, c->counters.p + CNT_TGMAX);
+    hipLaunchKernelGGL(k_count_blocks, dim3(nbt), dim3(256), 0, s, c->tmpi.p, c->nlive, c->tmpi2.p);
+    hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(1024), 0, s, c->tmpi2.p, (int)nbt, c->counters.p + CNT_NTG);
+    hipLaunchKernelGGL(k_tile_fill, dim3(nbt), dim3(256), 0, s, c->tmpi.p, c->nlive, c->tmpi2.p,
+                       c->counters.p + CNT_NTG, c->tg_lo.p);
   }
   PH_HIPCHECK(c, hipMemcpyAsync(cnt, c->counters.p, sizeof(cnt), hipMemcpyDeviceToHost, s));
   PH_HIPCHECK(c, hipStreamSynchronize(s));
   c->nleaves = cnt[CNT_NLEAF];
+  c->ntg = cnt[CNT_NTG];
+  c->tg_max = cnt[CNT_TGMAX];
   hipLaunchKernelGGL(k_pleaf, dim3(nblocks(c->nleaves, 256)), dim3(256), 0, s, c->leaves.p, c->nleaves,
                      c->nd_lo.p, c->nd_hi.p, c->pleaf.p);
   PH_HIPCHECK(c, hipGetLastError());
