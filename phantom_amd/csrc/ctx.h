@@ -118,6 +118,10 @@ struct phsph_ctx {
   DBuf<int32_t> tg_lo;       // tile groups: first tree position of each (one more: nlive)
   DBuf<int32_t> tg_t;        // the same as indexes into the active list
   DBuf<int32_t> tg_big;      // tile groups that need the large tile
+  DBuf<uint32_t> tl_cand, tl_bcand;  // tile lists (TileLists, tile.h)
+  DBuf<uint16_t> tl_list, tl_blist;
+  DBuf<int32_t> tl_nc, tl_bnc;
+  DBuf<double2> t_sums;      // sums of the last h iteration per active slot
   int ntg = 0, tg_max = 0;   // tile groups, particles of the largest
   DBuf<int32_t> pleaf;       // tree position -> index into leaves
   DBuf<int32_t> iparts;      // inodeparts: signed 1-based original index

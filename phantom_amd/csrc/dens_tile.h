@@ -4,6 +4,87 @@
 #include "tile.h"
 
 enum { DFL_CAND = 1, DFL_LIST = 2, DFL_REWALK = 4, DFL_NOCONV = 8, DFL_NEGH = 16, DFL_STACK = 32, DFL_TILE = 64 };
+// c->counters: particles that outgrew their lists, groups for the large tile
+constexpr int CNT_REWALK = 8, CNT_BIG = 9;
+
+struct DensIn {
+  const double4 *tp;  // x, y, z (treecache) and h at entry
+  const double4 *tv;  // vx, vy, vz
+  const double4 *tf;  // fxyzu + fext (null: zero)
+  const double4 *tB;  // Bevol x, y, z and rho(h at entry) (MHD)
+};
+struct DensOut {
+  double *xyzh;  int ldx;
+  float *divcurlv; int lddcv;
+  float *divcurlB;
+  float *alphaind;
+  float *gradh; int ldgradh;
+  float *dvdx;
+};
+
+// store_results (dens.F90:1511-1681) at the final h from the sums taken at
+// the h of the last iteration
+template <bool MHD>
+__device__ __forceinline__ void dens_store(const DevConst &dc, int p, double hfin, double rs_rho, double rs_gh,
+                                           double rs_gs, double rs_divv, double rs_divB, const double *dv,
+                                           const double *da, const double *rr, const double *dB,
+                                           const int32_t *__restrict__ iparts, double *__restrict__ th_out,
+                                           const DensOut &out, int32_t *__restrict__ p_nneigh, int nneigh,
+                                           int32_t *__restrict__ flags) {
+  const double pm = dc.pmass;
+  const double hf1 = 1. / hfin, hf21 = hf1 * hf1, hf31 = hf1 * hf21, hf41 = hf21 * hf21;
+  const double rhoi = dc.cnormk * (rs_rho + dc.wab0 * pm) * hf31;
+  const double gradhs = dc.cnormk * (rs_gh + dc.gradh0 * pm) * hf41;
+  const double dhdrhoi = -hfin / (3. * rhoh_d(hfin, dc.hfact, pm));
+  const double omegai = 1. - dhdrhoi * gradhs;
+  const double gradhi = 1. / omegai;
+  const double gradsofti = ((rs_gs + dc.dphidh0 * pm) * hf21) * dhdrhoi;
+  const double hnew = hrho_d(rhoi, dc.hfact, pm);
+  if (hnew < 0.) atomicOr(flags, DFL_NEGH);
+  const int o = abs(iparts[p]) - 1;
+  out.xyzh[(size_t)o * out.ldx + 3] = hnew;
+  th_out[p] = hnew;
+  const float gh32 = (float)gradhi;
+  out.gradh[(size_t)o * out.ldgradh] = gh32;
+  if (dc.gravity && out.ldgradh > 1) out.gradh[(size_t)o * out.ldgradh + 1] = (float)gradsofti;
+  const double rho1i = 1. / rhoi;
+  const double term = dc.cnormk * (double)gh32 * rho1i * hf41;
+  out.divcurlv[(size_t)o * out.lddcv] = (float)(-rs_divv * term);
+  // exact-linear gradients (dens.F90:866-967, 997-1052, 1086-1101)
+  const double rxx = rr[0], rxy = rr[1], rxz = rr[2], ryy = rr[3], ryz = rr[4], rzz = rr[5];
+  const double denom = rxx * ryy * rzz + 2. * rxy * rxz * ryz - rxx * ryz * ryz - ryy * rxz * rxz - rzz * rxy * rxy;
+  const double rm0 = ryy * rzz - ryz * ryz, rm1 = rxz * ryz - rzz * rxy, rm2 = rxy * ryz - rxz * ryy;
+  const double rm3 = rzz * rxx - rxz * rxz, rm4 = rxy * rxz - rxx * ryz, rm5 = rxx * ryy - rxy * rxy;
+  double gv[9], div_a;
+  if (fabs(denom) > PH_TINY64) {
+    const double dd = 1. / denom;
+    for (int cpt = 0; cpt < 3; cpt++) {
+      const double ax = dv[3 * cpt], ay = dv[3 * cpt + 1], az = dv[3 * cpt + 2];
+      gv[3 * cpt] = -((ax * rm0 + ay * rm1 + az * rm2) * dd);
+      gv[3 * cpt + 1] = -((ax * rm1 + ay * rm3 + az * rm4) * dd);
+      gv[3 * cpt + 2] = -((ax * rm2 + ay * rm4 + az * rm5) * dd);
+    }
+    const double gax = (da[0] * rm0 + da[1] * rm1 + da[2] * rm2) * dd;
+    const double gay = (da[3] * rm1 + da[4] * rm3 + da[5] * rm4) * dd;
+    const double gaz = (da[6] * rm2 + da[7] * rm4 + da[8] * rm5) * dd;
+    div_a = -(gax + gay + gaz);
+  } else {
+    for (int k = 0; k < 9; k++) gv[k] = -dv[k] * term;
+    div_a = -term * (da[0] + da[4] + da[8]);
+  }
+  const double d5 = div_a - (gv[0] * gv[0] + gv[4] * gv[4] + gv[8] * gv[8] +
+                             2. * (gv[1] * gv[3] + gv[2] * gv[6] + gv[5] * gv[7]));
+  if (out.alphaind) out.alphaind[(size_t)o * 3 + 2] = (float)d5;
+  if (out.dvdx)
+    for (int k = 0; k < 9; k++) out.dvdx[(size_t)o * 9 + k] = (float)gv[k];
+  if (MHD && out.divcurlB) {
+    out.divcurlB[(size_t)o * 4 + 0] = (float)(-rs_divB * term);
+    out.divcurlB[(size_t)o * 4 + 1] = (float)(-(dB[7] - dB[5]) * term);
+    out.divcurlB[(size_t)o * 4 + 2] = (float)(-(dB[2] - dB[6]) * term);
+    out.divcurlB[(size_t)o * 4 + 3] = (float)(-(dB[3] - dB[1]) * term);
+  }
+  p_nneigh[p] = nneigh;
+}
 
 // outputs of the search and h iteration, by active slot (t_), tree position
 // (p_, retry, htraj, hconv) and leaf
@@ -16,7 +97,7 @@ struct DensIterOut {
   double *htraj;
   size_t hstride;
   double *hconv;
-  int32_t *big, *nbig;  // groups that need the large tile
+  double2 *t_sums;  // sum of w m and of -(q w' + 3 w) m at the last iteration
 };
 
 // The kernels in the form w = sum_k c_k max(k - q, 0)^n (kernel_cubic.f90:34-60:
@@ -70,21 +151,9 @@ struct IterSums {
   }
 };
 
-// sqrt of a squared separation: reciprocal square root estimate and one
-// coupled Newton step for the root and its half reciprocal, then the residual
-// (to about one unit in the last place; zero and denormal squares give about
-// 1e-145, far below any h)
-__device__ __forceinline__ double sqrt_sep(double r2) {
-  const double a = fmax(r2, 1e-290);
-  const double y = __builtin_amdgcn_rsq(a);
-  double g = a * y, h = 0.5 * y;
-  const double e = fma(-h, g, 0.5);
-  g = fma(g, e, g);
-  h = fma(h, e, h);
-  const double d = fma(-g, g, a);
-  return fma(d, h, g);
-}
-
 void launch_dens_tile(phsph_ctx *c, int icall, double rfac, double lmargin, const double *hmax0,
-                      const DensIterOut &out);
+                      const DensIterOut &out, const TileLists &tl);
+void launch_dens_sums(phsph_ctx *c, const TileLists &tl, bool mhd, bool mixed, const DensIn &in, const DensOut &out);
+// the list buffers for the context's tile groups
+int tile_lists(phsph_ctx *c, TileLists &tl);
 int dens_tile_list_cap(const phsph_ctx *c);

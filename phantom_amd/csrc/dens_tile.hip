@@ -6,6 +6,8 @@
 // does not fit a tile and for the particles that are run again.
 #include "dens_tile.h"
 
+#include <algorithm>
+
 // One particle's neighbour distances live in the registers of its four
 // lanes, entry k in lane k mod 4, so a Newton iteration reads no memory.
 //
@@ -41,7 +43,7 @@ k_dens_tile(DevConst dc, int icall, double rfac, double lmargin, const int32_t *
             const double *__restrict__ gbox, const int32_t *__restrict__ pleaf, const uint32_t *__restrict__ gcand,
             const int32_t *__restrict__ gncand, const int64_t *goff, int capg, const int32_t *__restrict__ nd_lo,
             const int32_t *__restrict__ nd_hi, const phsph_kdnode *__restrict__ nd, const double4 *__restrict__ tp,
-            const double *__restrict__ hmax0, DensIterOut out, int32_t *__restrict__ flags) {
+            const double *__restrict__ hmax0, DensIterOut out, TileLists tl, int32_t *__restrict__ flags) {
   constexpr bool BIG = TileCap<K, V>::BIG;
   constexpr int W = TileCap<K, V>::W, NC = TileCap<K, V>::NC, LC = TileCap<K, V>::LC, NE = BIG ? 1 : LC / TILE_L;
   constexpr int LEAVES = 64 * W;  // leaves staged at a time
@@ -60,9 +62,12 @@ k_dens_tile(DevConst dc, int icall, double rfac, double lmargin, const int32_t *
   __shared__ int wcnt[2][W];
   __shared__ double wred[W][2];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  auto group = [&](const int g) {
+  auto group = [&](const int g, const int b) {  // b: its place in the large arrays
   const int t0 = gt[g], t1 = gt[g + 1];
-  if (t0 >= t1) return;  // no active particle in the node
+  if (t0 >= t1) {  // no active particle in the node
+    if (!BIG && threadIdx.x == 0) tl.nc[g] = -1;
+    return;
+  }
   const double *gb = gbox + (size_t)g * GBOX;
   const double bx = 0.5 * (gb[0] + gb[3]), by = 0.5 * (gb[1] + gb[4]), bz = 0.5 * (gb[2] + gb[5]);
   const double ex = 0.5 * (gb[3] - gb[0]) * (1. + 1e-12) + 1e-300, ey = 0.5 * (gb[4] - gb[1]) * (1. + 1e-12) + 1e-300,
@@ -107,13 +112,7 @@ k_dens_tile(DevConst dc, int icall, double rfac, double lmargin, const int32_t *
           const int j = U.leaf.lo[r + li] + lk, code = cc >> 8;
           const double4 v = tp[j];
           x = v.x; y = v.y; z = v.z;
-          if (code != SEP_PLAIN) {
-            int sx, sy, sz;
-            off_decode(code, sx, sy, sz);
-            if (sx) x = xadd(x, copysign(dc.dxbound, (double)sx));
-            if (sy) y = xadd(y, copysign(dc.dybound, (double)sy));
-            if (sz) z = xadd(z, copysign(dc.dzbound, (double)sz));
-          }
+          offset_pos(dc, code, x, y, z);
           if (hmax0) rj2 = (float)((rl * v.w) * (rl * v.w) * (1. + 1.2e-7));
           const double qx = fmax(fabs(x - bx) - ex, 0.), qy = fmax(fabs(y - by) - ey, 0.),
                        qz = fmax(fabs(z - bz) - ez, 0.);
@@ -151,7 +150,12 @@ k_dens_tile(DevConst dc, int icall, double rfac, double lmargin, const int32_t *
     const double need = (rl * hmx + 3. * smax) * (1. + 1e-9);
     bad = bad || ex + need >= dc.hdlx || ey + need >= dc.hdly || ez + need >= dc.hdlz;
   }
-  if (bad && !BIG && nc > NC && tid == 0) out.big[atomicAdd(out.nbig, 1)] = g;  // the large form next
+  if (bad && !BIG && nc > NC && tid == 0) tl.big[atomicAdd(tl.nbig, 1)] = g;  // the large form next
+  uint32_t *gcl = BIG ? tl.bcand + (size_t)b * tl.bncap : tl.cand + (size_t)g * tl.ncap;
+  uint16_t *gll = BIG ? tl.blist + (size_t)b * TILE_BW * tl.blc * TILE_P : tl.list + (size_t)g * tl.lw * tl.lc * TILE_P;
+  if (!bad)
+    for (int k = tid; k < nc; k += 64 * W) gcl[k] = cj[k];
+  if (tid == 0) (BIG ? tl.bnc[b] : tl.nc[g]) = bad ? -1 : nc;
   const int pi = lane / TILE_L, sl = lane % TILE_L;
   const int lcap = min(LC, out.capl);
   bool redo = false;  // a list of this group did not fit
@@ -250,12 +254,19 @@ k_dens_tile(DevConst dc, int icall, double rfac, double lmargin, const int32_t *
     nmax = __builtin_amdgcn_readfirstlane(nmax);
     auto dist = [&](int s) {
       const double dx = xi - cx[s], dy = yi - cy[s], dz = zi - cz[s];
-      return sqrt_sep(dx * dx + dy * dy + dz * dz);
+      double rr, r1;
+      sqrt_rsqrt_sep(dx * dx + dy * dy + dz * dz, 0., rr, r1);
+      return rr;
     };
     double r[NE];
     if constexpr (BIG) {
-      for (int k = sl; k < nl; k += TILE_L) out.nlist[list_at(nact, t, k)] = cj[L[k][pi]];
+      uint16_t *ll = gll + (size_t)((wt - t0) / TILE_P) * tl.blc * TILE_P;
+      for (int k = sl; k < nl; k += TILE_L) {
+        out.nlist[list_at(nact, t, k)] = cj[L[k][pi]];
+        ll[k * TILE_P + pi] = L[k][pi];
+      }
     } else {
+      uint16_t *ll = gll + (size_t)w * LC * TILE_P;
 #pragma unroll
       for (int e = 0; e < NE; e++) {
         r[e] = PH_HUGE64;
@@ -264,6 +275,7 @@ k_dens_tile(DevConst dc, int icall, double rfac, double lmargin, const int32_t *
           if (k < nl) {
             const int s = L[k][pi];
             r[e] = dist(s);
+            ll[k * TILE_P + pi] = (uint16_t)s;
             out.nlist[((size_t)(TILE_L * e / LSEG) * nact + t) * LSEG + TILE_L * e % LSEG + sl] = cj[s];
           }
         }
@@ -335,6 +347,7 @@ k_dens_tile(DevConst dc, int icall, double rfac, double lmargin, const int32_t *
           if (out.hconv) out.hconv[p] = hi;  // the h of the last summation (cell%h once converged)
           out.t_nl[t] = n;
           if (out.t_nlj) out.t_nlj[t] = 0;
+          out.t_sums[t] = make_double2(srho, sgh);
           out.t_hsum[t] = hi;
           out.t_hfin[t] = hfin;
           out.p_nits[p] = nit;
@@ -348,30 +361,40 @@ k_dens_tile(DevConst dc, int icall, double rfac, double lmargin, const int32_t *
   } else {
     if (t0 + w * TILE_P < t1) wave16(t0 + w * TILE_P);
     // a list of any wavefront too long: the group again in the large form
-    if (!bad && __syncthreads_or(redo) && tid == 0) out.big[atomicAdd(out.nbig, 1)] = g;
+    if (!bad && __syncthreads_or(redo) && tid == 0) {
+      tl.nc[g] = -1;
+      tl.big[atomicAdd(tl.nbig, 1)] = g;
+    }
   }
   };
   if constexpr (BIG) {  // the listed groups in turn
-    const int nbig = *out.nbig;
+    const int nbig = *tl.nbig;
     for (int k = blockIdx.x; k < nbig; k += gridDim.x) {
-      group(out.big[k]);
-      __syncthreads();
+      const int g = tl.big[k];
+      if (k < tl.bcap) {
+        group(g, k);
+        __syncthreads();
+      } else {  // no room for its lists
+        for (int t = gt[g] + tid; t < gt[g + 1]; t += 64 * W) out.retry[act[t]] = 1;
+        if (tid == 0) atomicOr(flags, DFL_TILE);
+      }
     }
   } else {
     const int g = xcd_block(blockIdx.x, gridDim.x);
-    if (g < ngroups) group(g);
+    if (g < ngroups) group(g, 0);
   }
 }
 
 void launch_dens_tile(phsph_ctx *c, int icall, double rfac, double lmargin, const double *hmax0,
-                      const DensIterOut &out) {
+                      const DensIterOut &out, const TileLists &tl) {
   const int ng = c->ngroups;
   // the large form: as many workgroups as the CUs hold
   const dim3 gr(xcd_grid(ng)), gb((unsigned)(c->ncu > 0 ? c->ncu : 256));
 #define DT(KK, VV, GG)                                                                                             \
   hipLaunchKernelGGL((k_dens_tile<KK, VV>), GG, dim3(64 * TileCap<KK, VV>::W), 0, c->stream, c->dc, icall, rfac,   \
                      lmargin, c->act.p, c->nact, ng, c->tg_t.p, c->gbox.p, c->pleaf.p, c->gcand.p, c->gncand.p,     \
-                     c->goff_p, c->caps.gcand, c->nd_lo.p, c->nd_hi.p, c->nd.p, c->tp4.p, hmax0, out, c->counters.p)
+                     c->goff_p, c->caps.gcand, c->nd_lo.p, c->nd_hi.p, c->nd.p, c->tp4.p, hmax0, out, tl,        \
+                     c->counters.p)
   const bool w4 = c->tg_max <= 4 * TILE_P;
   if (c->p.kernel == PHSPH_KERNEL_CUBIC) {
     if (w4) DT(PHSPH_KERNEL_CUBIC, TILE_4, gr); else DT(PHSPH_KERNEL_CUBIC, TILE_5, gr);
@@ -381,6 +404,41 @@ void launch_dens_tile(phsph_ctx *c, int icall, double rfac, double lmargin, cons
     DT(PHSPH_KERNEL_QUINTIC, TILE_BIG, gb);
   }
 #undef DT
+}
+
+// The arrays of a context are sized for its tile groups and kept.  A thirtieth
+// of the groups and 1024 have room in the large form.
+template <int K>
+static void tile_caps(const phsph_ctx *c, TileLists &tl) {
+  const bool w4 = c->tg_max <= 4 * TILE_P;
+  tl.lw = w4 ? TileCap<K, TILE_4>::W : TileCap<K, TILE_5>::W;
+  tl.ncap = w4 ? TileCap<K, TILE_4>::NC : TileCap<K, TILE_5>::NC;
+  tl.lc = TileCap<K, TILE_4>::LC;
+  tl.bncap = TileCap<K, TILE_BIG>::NC;
+  tl.blc = TileCap<K, TILE_BIG>::LC;
+}
+int tile_lists(phsph_ctx *c, TileLists &tl) {
+  const size_t ng = c->ntg;
+  if (c->p.kernel == PHSPH_KERNEL_CUBIC) tile_caps<PHSPH_KERNEL_CUBIC>(c, tl);
+  else tile_caps<PHSPH_KERNEL_QUINTIC>(c, tl);
+  tl.bcap = (int)std::min(ng, 1024 + ng / 32);
+  PH_HIPCHECK(c, c->tl_cand.ensure(ng * tl.ncap));
+  PH_HIPCHECK(c, c->tl_list.ensure(ng * tl.lw * tl.lc * TILE_P));
+  PH_HIPCHECK(c, c->tl_nc.ensure(ng + 1));
+  PH_HIPCHECK(c, c->tg_big.ensure(ng + 1));
+  PH_HIPCHECK(c, c->tl_bcand.ensure((size_t)tl.bcap * tl.bncap));
+  PH_HIPCHECK(c, c->tl_blist.ensure((size_t)tl.bcap * TILE_BW * tl.blc * TILE_P));
+  PH_HIPCHECK(c, c->tl_bnc.ensure(tl.bcap + 1));
+  tl.gt = c->tg_t.p;
+  tl.cand = c->tl_cand.p;
+  tl.list = c->tl_list.p;
+  tl.nc = c->tl_nc.p;
+  tl.big = c->tg_big.p;
+  tl.nbig = c->counters.p + CNT_BIG;
+  tl.bcand = c->tl_bcand.p;
+  tl.blist = c->tl_blist.p;
+  tl.bnc = c->tl_bnc.p;
+  return PHSPH_OK;
 }
 
 int dens_tile_list_cap(const phsph_ctx *c) {

@@ -31,24 +31,6 @@
 #include <vector>
 #include <cstdlib>
 
-// c->counters: particles that outgrew their lists, groups for the large tile
-constexpr int CNT_REWALK = 8, CNT_BIG = 9;
-
-struct DensIn {
-  const double4 *tp;  // x, y, z (treecache) and h at entry
-  const double4 *tv;  // vx, vy, vz
-  const double4 *tf;  // fxyzu + fext (null: zero)
-  const double4 *tB;  // Bevol x, y, z and rho(h at entry) (MHD)
-};
-struct DensOut {
-  double *xyzh;  int ldx;
-  float *divcurlv; int lddcv;
-  float *divcurlB;
-  float *alphaind;
-  float *gradh; int ldgradh;
-  float *dvdx;
-};
-
 // ------------------------------------------------------------------------
 // per-leaf walk of the reference (trial-neighbour statistics only)
 // ------------------------------------------------------------------------
@@ -527,70 +509,6 @@ k_dens_iter(DevConst dc, int icall, double rfac, const int32_t *__restrict__ act
       }
     }
   }
-}
-
-// store_results (dens.F90:1511-1681) at the final h from the sums taken at
-// the h of the last iteration
-template <bool MHD>
-__device__ __forceinline__ void dens_store(const DevConst &dc, int p, double hfin, double rs_rho, double rs_gh,
-                                           double rs_gs, double rs_divv, double rs_divB, const double *dv,
-                                           const double *da, const double *rr, const double *dB,
-                                           const int32_t *__restrict__ iparts, double *__restrict__ th_out,
-                                           const DensOut &out, int32_t *__restrict__ p_nneigh, int nneigh,
-                                           int32_t *__restrict__ flags) {
-  const double pm = dc.pmass;
-  const double hf1 = 1. / hfin, hf21 = hf1 * hf1, hf31 = hf1 * hf21, hf41 = hf21 * hf21;
-  const double rhoi = dc.cnormk * (rs_rho + dc.wab0 * pm) * hf31;
-  const double gradhs = dc.cnormk * (rs_gh + dc.gradh0 * pm) * hf41;
-  const double dhdrhoi = -hfin / (3. * rhoh_d(hfin, dc.hfact, pm));
-  const double omegai = 1. - dhdrhoi * gradhs;
-  const double gradhi = 1. / omegai;
-  const double gradsofti = ((rs_gs + dc.dphidh0 * pm) * hf21) * dhdrhoi;
-  const double hnew = hrho_d(rhoi, dc.hfact, pm);
-  if (hnew < 0.) atomicOr(flags, DFL_NEGH);
-  const int o = abs(iparts[p]) - 1;
-  out.xyzh[(size_t)o * out.ldx + 3] = hnew;
-  th_out[p] = hnew;
-  const float gh32 = (float)gradhi;
-  out.gradh[(size_t)o * out.ldgradh] = gh32;
-  if (dc.gravity && out.ldgradh > 1) out.gradh[(size_t)o * out.ldgradh + 1] = (float)gradsofti;
-  const double rho1i = 1. / rhoi;
-  const double term = dc.cnormk * (double)gh32 * rho1i * hf41;
-  out.divcurlv[(size_t)o * out.lddcv] = (float)(-rs_divv * term);
-  // exact-linear gradients (dens.F90:866-967, 997-1052, 1086-1101)
-  const double rxx = rr[0], rxy = rr[1], rxz = rr[2], ryy = rr[3], ryz = rr[4], rzz = rr[5];
-  const double denom = rxx * ryy * rzz + 2. * rxy * rxz * ryz - rxx * ryz * ryz - ryy * rxz * rxz - rzz * rxy * rxy;
-  const double rm0 = ryy * rzz - ryz * ryz, rm1 = rxz * ryz - rzz * rxy, rm2 = rxy * ryz - rxz * ryy;
-  const double rm3 = rzz * rxx - rxz * rxz, rm4 = rxy * rxz - rxx * ryz, rm5 = rxx * ryy - rxy * rxy;
-  double gv[9], div_a;
-  if (fabs(denom) > PH_TINY64) {
-    const double dd = 1. / denom;
-    for (int cpt = 0; cpt < 3; cpt++) {
-      const double ax = dv[3 * cpt], ay = dv[3 * cpt + 1], az = dv[3 * cpt + 2];
-      gv[3 * cpt] = -((ax * rm0 + ay * rm1 + az * rm2) * dd);
-      gv[3 * cpt + 1] = -((ax * rm1 + ay * rm3 + az * rm4) * dd);
-      gv[3 * cpt + 2] = -((ax * rm2 + ay * rm4 + az * rm5) * dd);
-    }
-    const double gax = (da[0] * rm0 + da[1] * rm1 + da[2] * rm2) * dd;
-    const double gay = (da[3] * rm1 + da[4] * rm3 + da[5] * rm4) * dd;
-    const double gaz = (da[6] * rm2 + da[7] * rm4 + da[8] * rm5) * dd;
-    div_a = -(gax + gay + gaz);
-  } else {
-    for (int k = 0; k < 9; k++) gv[k] = -dv[k] * term;
-    div_a = -term * (da[0] + da[4] + da[8]);
-  }
-  const double d5 = div_a - (gv[0] * gv[0] + gv[4] * gv[4] + gv[8] * gv[8] +
-                             2. * (gv[1] * gv[3] + gv[2] * gv[6] + gv[5] * gv[7]));
-  if (out.alphaind) out.alphaind[(size_t)o * 3 + 2] = (float)d5;
-  if (out.dvdx)
-    for (int k = 0; k < 9; k++) out.dvdx[(size_t)o * 9 + k] = (float)gv[k];
-  if (MHD && out.divcurlB) {
-    out.divcurlB[(size_t)o * 4 + 0] = (float)(-rs_divB * term);
-    out.divcurlB[(size_t)o * 4 + 1] = (float)(-(dB[7] - dB[5]) * term);
-    out.divcurlB[(size_t)o * 4 + 2] = (float)(-(dB[2] - dB[6]) * term);
-    out.divcurlB[(size_t)o * 4 + 3] = (float)(-(dB[3] - dB[1]) * term);
-  }
-  p_nneigh[p] = nneigh;
 }
 
 // ------------------------------------------------------------------------
@@ -1396,6 +1314,7 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
   int dlist = c->caps.dlist;
   const int dlist0 = dlist;
   bool tuned_now = false, retune = false;
+  TileLists tl{};
   int nrewalk = 0;  // particles of the first attempt that outgrew their lists
   for (int attempt = 0; attempt < 12; attempt++) {
     int na = c->nact;  // active slots, padding included
@@ -1448,12 +1367,13 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
       PH_HIPCHECK(c, dev_set(c, c->counters.p, &zero, sizeof(int32_t)));
       PH_HIPCHECK(c, dev_set(c, c->counters.p + CNT_REWALK, &zero, sizeof(int32_t)));
       PH_HIPCHECK(c, dev_set(c, c->counters.p + CNT_BIG, &zero, sizeof(int32_t)));
-      PH_HIPCHECK(c, c->tg_big.ensure((size_t)c->ntg + 1));
+      rc = tile_lists(c, tl);
+      if (rc) return rc;
+      PH_HIPCHECK(c, c->t_sums.ensure((size_t)na + 1));
       const DensIterOut o{LB.p, list_cap(dlist), TNL.p, widen ? c->t_nlj.p : nullptr, THS.p, THF.p, c->p_nits.p, c->leaf_nits.p,
-                          c->tmpi.p, c->counters.p + CNT_REWALK, c->htraj.p, (size_t)c->htraj_stride, c->hconv.p, c->tg_big.p,
-                          c->counters.p + CNT_BIG};
+                          c->tmpi.p, c->counters.p + CNT_REWALK, c->htraj.p, (size_t)c->htraj_stride, c->hconv.p, c->t_sums.p};
       LaunchTimer lt(c, "density_iter");
-      launch_dens_tile(c, icall, rfac, lmargin, widen ? c->hmax0.p : nullptr, o);
+      launch_dens_tile(c, icall, rfac, lmargin, widen ? c->hmax0.p : nullptr, o, tl);
     }
     {
       LaunchTimer lt(c, "density_sums");
@@ -1465,7 +1385,9 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
   hipLaunchKernelGGL((k_dens_final_mixed<KK>), dim3(xcd_grid(nblocks(na, 256))), dim3(256), 0, s, c->dc, c->act.p, \
                      na, LB.p, TNL.p, THS.p, THF.p, c->tmpi.p, c->iparts.p, c->tp4.p,                               \
                      c->tv4.p, have_f ? c->tf4.p : nullptr, c->th.p, out, c->p_nneigh.p, c->counters.p)
-      if (mixed) {
+      if (by_tile) {
+        launch_dens_sums(c, tl, mhd, mixed, in, out);
+      } else if (mixed) {
         if (c->p.kernel == PHSPH_KERNEL_CUBIC) DMIX(PHSPH_KERNEL_CUBIC); else DMIX(PHSPH_KERNEL_QUINTIC);
       } else if (c->p.kernel == PHSPH_KERNEL_CUBIC) {
         if (mhd) DFIN(PHSPH_KERNEL_CUBIC, true); else DFIN(PHSPH_KERNEL_CUBIC, false);

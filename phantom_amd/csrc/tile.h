@@ -43,6 +43,99 @@ struct TileCap {
   static constexpr int LC = BIG ? 1024 : CU ? 96 : 160;
   static constexpr int WPE = BIG ? 1 : V == TILE_5 ? (CU ? 3 : 2) : (CU ? 4 : 3);
 };
+// adds the periodic offset of a separation code to a position (get_sep,
+// kdtree.F90:1468-1501)
+__device__ __forceinline__ void offset_pos(const DevConst &dc, int code, double &x, double &y, double &z) {
+  if (code == SEP_PLAIN) return;
+  int sx, sy, sz;
+  off_decode(code, sx, sy, sz);
+  if (sx) x = xadd(x, copysign(dc.dxbound, (double)sx));
+  if (sy) y = xadd(y, copysign(dc.dybound, (double)sy));
+  if (sz) z = xadd(z, copysign(dc.dzbound, (double)sz));
+}
+
+// The lists that the density tile kernel leaves for the sums and for the force
+// pass: the candidates of each group (tree position and offset code) and, per
+// 16 particles (one wavefront), the entries of their lists as 16-bit slots of
+// the group's candidates, entry k of the 16 particles in 32 consecutive bytes.
+// Groups in the large form have arrays of their own, by position in big.
+struct TileLists {
+  const int32_t *gt;  // group ranges of the active list
+  uint32_t *cand;     // ncap per group
+  uint16_t *list;     // lw wavefronts of lc entries per group
+  int32_t *nc;        // candidates per group; -1: large form, or handed back
+  int ncap, lc, lw;
+  int32_t *big, *nbig;  // groups in the large form
+  uint32_t *bcand;
+  uint16_t *blist;
+  int32_t *bnc;
+  int bncap, blc, bcap;  // bcap: groups the arrays hold (more are handed back)
+};
+constexpr int TILE_BW = 5;  // wavefronts of 16 particles of a group in the large form
+
+// the group of a workgroup of a launch over all groups and the large ones
+struct TileGroup {
+  int g, t0, t1, nc, lc;
+  const uint32_t *cand;
+  const uint16_t *list;
+  __device__ __forceinline__ bool find(const TileLists &tl, int ngroups) {
+    const int ngr = (ngroups + 7) / 8 * 8;  // blocks of the ordinary groups
+    if ((int)blockIdx.x < ngr) {
+      g = xcd_block(blockIdx.x, ngr);
+      if (g >= ngroups) return false;
+      nc = tl.nc[g];
+      lc = tl.lc;
+      cand = tl.cand + (size_t)g * tl.ncap;
+      list = tl.list + (size_t)g * tl.lw * tl.lc * TILE_P;
+    } else {
+      const int b = blockIdx.x - ngr;
+      if (b >= *tl.nbig) return false;
+      g = tl.big[b];
+      nc = tl.bnc[b];
+      lc = tl.blc;
+      cand = tl.bcand + (size_t)b * tl.bncap;
+      list = tl.blist + (size_t)b * TILE_BW * tl.blc * TILE_P;
+    }
+    t0 = tl.gt[g];
+    t1 = tl.gt[g + 1];
+    return nc >= 0 && t0 < t1;
+  }
+};
+static inline unsigned tile_grid(int ngroups, const TileLists &tl) { return xcd_grid(ngroups) + (unsigned)tl.bcap; }
+
+// r and 1/(r + eps) of a squared separation, from a reciprocal square root
+// estimate: one coupled Newton step for the root and its half reciprocal, the
+// residual of the root, and one step for the reciprocal (each to about one unit
+// in the last place; zero and denormal squares give about 1e-145, far below
+// any h)
+__device__ __forceinline__ void sqrt_rsqrt_sep(double r2, double eps, double &r, double &r1) {
+  const double a = fmax(r2, 1e-290);
+  const double y = __builtin_amdgcn_rsq(a);
+  double g = a * y, h = 0.5 * y;
+  const double e = fma(-h, g, 0.5);
+  g = fma(g, e, g);
+  h = fma(h, e, h);
+  const double d = fma(-g, g, a);
+  r = fma(d, h, g);
+  h = h + h;
+  const double e1 = fma(-(r + eps), h, 1.);
+  r1 = fma(h, e1, h);
+}
+
+// dw/dq without branches: sums of max(k - q, 0)^n (kernel_cubic.f90:34-60,
+// kernel_quintic.f90:34-75)
+template <int K>
+__device__ __forceinline__ double kern_grad(double q) {
+  if (K == PHSPH_KERNEL_CUBIC) {
+    const double a = fmax(2. - q, 0.), b = fmax(1. - q, 0.);
+    return fma(-0.75 * a, a, 3. * (b * b));
+  } else {
+    const double a = fmax(3. - q, 0.), b = fmax(2. - q, 0.), c = fmax(1. - q, 0.);
+    const double a2 = a * a, b2 = b * b, c2 = c * c;
+    return fma(-5. * a2, a2, fma(30. * b2, b2, -75. * (c2 * c2)));
+  }
+}
+
 constexpr int GBOX = 8;                  // doubles per group: bounding box, largest search h
 
 // exchange within the four lanes of a particle

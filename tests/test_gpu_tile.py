@@ -1,0 +1,70 @@
+"""The tile kernels (one workgroup per tree node, candidates in LDS) against
+the oracle at the sizes where their forms change: sets whose nodes hold other
+than 64 particles, boxes too small for one periodic offset per leaf, groups
+with more candidates or longer lists than a tile holds (the large form, and
+beyond it the list kernels), and active fractions on both sides of one half.
+Neighbour and iteration counts are exact; h and each force component agree to
+1e-12 of the rms (the parity tests' FP64 tolerance: sums of a few hundred FP64
+terms in another order, a few 1e-16 each)."""
+import numpy as np
+import pytest
+
+from phantom_amd import abi, setups
+from tests import parity
+
+pytestmark = pytest.mark.gpu
+
+
+def _noisy_star():
+    return setups.relaxation_target(n=9000, seed=7)
+
+
+def _active(frac):
+    s = setups.uniform_box(nx=18, ny=16, nz=20, seed=3, isothermal=False,
+                           box=(-0.45, 0.45, -0.4, 0.4, -0.5, 0.5))
+    return setups.with_levels(s, [(0, 1.0 - frac), (2, frac)], nbinmax=2, istepfrac=1)
+
+
+CASES = {
+    "box_67_per_node_cubic": lambda: setups.uniform_box(nx=17, ny=18, nz=14, seed=3, isothermal=False,
+                                                         box=(-0.425, 0.425, -0.45, 0.45, -0.35, 0.35)),
+    "box_quintic": lambda: setups.uniform_box(nx=20, ny=19, nz=21, seed=4, kernel=abi.KERNEL_QUINTIC,
+                                               box=(-0.5, 0.5, -0.475, 0.475, -0.525, 0.525)),
+    "small_box_quintic": lambda: setups.uniform_box(nx=12, seed=5, kernel=abi.KERNEL_QUINTIC),
+    "random_box_h_times_4": lambda: setups.random_box(n=7000, seed=12),
+    "random_box_quintic": lambda: setups.random_box(n=5000, seed=13, kernel=abi.KERNEL_QUINTIC),
+    "tube_interface": lambda: setups.shock_tube(ny=16),
+    "noisy_star": _noisy_star,
+    "mhd_dust_odd": lambda: setups.mhd_dust_box(nx=15, jitter=0.05, kernel=abi.KERNEL_CUBIC),
+    "active_0.45": lambda: _active(0.45),
+    "active_0.55": lambda: _active(0.55),
+}
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_tiles_match_oracle(name, gpu):
+    setup = CASES[name]()
+    print(f"\n[case {name}] n={setup['xyzh'].shape[0]}", flush=True)
+    g = parity.run_gpu(setup)
+    o = parity.run_oracle(setup)
+    act = setup["iphase"] > 0 if setup.get("iphase") is not None else np.ones(len(setup["xyzh"]), bool)
+    np.testing.assert_array_equal(g["nneigh"][act], o["dens"]["nneigh"][act])
+    np.testing.assert_array_equal(g["nits"][act], o["dens"]["nits"][act])
+    assert parity.rel_rms(g["xyzh"][:, 3], o["xyzh"][:, 3]) <= 1e-12
+    for k in ("gradh", "dvdx"):
+        # FP32 outputs: one unit in the last place of values up to the rms,
+        # relative above it
+        assert parity.rel_err(np.asarray(g["dens"][k])[act], np.asarray(o["dens"][k])[act]) <= 2.4e-7, k
+    ncomp = 4 if setup["params"].maxvxyzu >= 4 else 3
+    f, fo = g["force"]["fxyzu"][act], o["force"]["fxyzu"][act]
+    rms = np.sqrt(np.mean((fo[:, :3] ** 2).sum(axis=1)))
+    assert np.max(np.abs(f[:, :3] - fo[:, :3])) <= 1e-12 * rms
+    if ncomp == 4:
+        assert parity.rel_rms(f[:, 3], fo[:, 3]) <= 1e-12
+    if setup["params"].mhd:
+        for c in range(4):
+            assert parity.rel_rms(g["force"]["dBevol"][:, c], o["force"]["dBevol"][:, c]) <= 1e-12, c
+        assert parity.rel_rms(g["force"]["ddustevol"], o["force"]["ddustevol"]) <= 1e-12
+    if setup.get("bins") is not None:
+        np.testing.assert_array_equal(g["force"]["ibin"], o["force"]["ibin"])
+    g["ctx"].close()
