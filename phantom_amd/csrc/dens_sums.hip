@@ -6,29 +6,34 @@
 
 // FP64 records of a candidate in LDS, 16 bytes at a time: position with the
 // offset, velocity, f + fext, and with MHD B = Bevol rho(h at entry)
-template <bool MHD>
+template <int W, bool MHD>
 struct SumCap {
-  static constexpr int ND = MHD ? 12 : 10;   // doubles per record
-  static constexpr int NC = MHD ? 800 : 672;  // candidates staged at a time
-  static constexpr int WPE = MHD ? 2 : 3;     // wavefronts per SIMD that LDS and registers hold
+  static constexpr int ND = MHD ? 12 : 10;  // doubles per record
+  // candidates staged at a time, and wavefronts per SIMD that LDS and registers hold
+  static constexpr int NC = MHD ? 544 : W == 4 ? 480 : 672;
+  static constexpr int WPE = MHD ? 3 : 4;
 };
 
 // One workgroup per group as in k_dens_tile, four lanes per particle.  The
-// candidates' records are staged in LDS in chunks of equal length (one chunk
-// holds a node of 64 particles of a uniform set) and
+// candidates' records are staged in LDS in chunks of equal length (one
+// chunk holds a node of 64 particles of a uniform set with the cubic kernel) and
 // each lane sums every fourth entry of its particle's list, which is in
 // candidate order, so that a chunk's entries are consecutive.
 //
 // A pair reads 72 bytes (MHD 96) from LDS instead of six 16-byte loads whose
 // 64 lanes go to 64 cache lines each.  rho and its h derivative are the sums
 // the last iteration ended with.  Bound by vector instructions and LDS reads.
+// On the 8M-particle box 3.1 ms (6.7 ms as a list kernel; 3.8 ms with the ends
+// in one lane of four and three wavefronts per SIMD), MHD 2M particles 2.1 ms
+// (3.9), quintic 1M particles 1.9 ms (2.7; 2.9 where 135 registers let a SIMD
+// hold three wavefronts of the 80-particle groups' five).
 template <int K, int W, bool MHD, bool MIXED>
-__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(SumCap<MHD>::WPE)))
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu((SumCap<W, MHD>::WPE))))
 k_dens_sums(DevConst dc, int ngroups, const int32_t *__restrict__ act, TileLists tl, const int32_t *__restrict__ t_nl,
             const double *__restrict__ t_hsum, const double *__restrict__ t_hfin, const double2 *__restrict__ t_sums,
             const int32_t *__restrict__ retry, const int32_t *__restrict__ iparts, DensIn in,
             double *__restrict__ th_out, DensOut out, int32_t *__restrict__ p_nneigh, int32_t *__restrict__ flags) {
-  constexpr int ND = SumCap<MHD>::ND, NC = SumCap<MHD>::NC;
+  constexpr int ND = SumCap<W, MHD>::ND, NC = SumCap<W, MHD>::NC;
   __shared__ double2 rec[NC * ND / 2];
   TileGroup G;
   if (!G.find(tl, ngroups)) return;
@@ -176,10 +181,51 @@ k_dens_sums(DevConst dc, int ngroups, const int32_t *__restrict__ act, TileLists
   if (MIXED) rs_divv = quad_sum(rs_divv);
   else rs_divv = dv[0] + dv[4] + dv[8];
   nneigh = quad_sum_i(nneigh) + 1;
-  if (!live || sl != 0) return;
-  const double2 s = t_sums[t];
-  dens_store<MHD>(dc, p, t_hfin[t], s.x, s.y, rs_gs, rs_divv, MHD ? dB[0] + dB[4] + dB[8] : 0., dv, da, rr, dB, iparts,
-                  th_out, out, p_nneigh, nneigh, flags);
+  // the ends of all particles by the first lanes of the workgroup, so that
+  // they fill wavefronts (the ends are a fifth of the kernel in one lane of
+  // four): sums through LDS, one row per sum
+  constexpr int GP = W * TILE_P, NS = 27 + (MHD ? 4 : 0);
+  static_assert(GP * NS <= NC * ND, "the sums of the workgroup fit the record buffer");
+  double *R = reinterpret_cast<double *>(rec);
+  __syncthreads();
+  if (live && sl == 0) {
+    double *o = R + w * TILE_P + pi;
+#pragma unroll
+    for (int q = 0; q < 9; q++) {
+      o[q * GP] = dv[q];
+      o[(9 + q) * GP] = da[q];
+    }
+#pragma unroll
+    for (int q = 0; q < 6; q++) o[(18 + q) * GP] = rr[q];
+    o[24 * GP] = rs_gs;
+    o[25 * GP] = rs_divv;
+    o[26 * GP] = (double)nneigh;
+    if (MHD) {
+      o[27 * GP] = dB[0] + dB[4] + dB[8];
+      o[28 * GP] = dB[7] - dB[5];
+      o[29 * GP] = dB[2] - dB[6];
+      o[30 * GP] = dB[3] - dB[1];
+    }
+  }
+  __syncthreads();
+  const int te = G.t0 + tid;
+  if (tid >= GP || te >= G.t1) return;
+  const int pe = act[te];
+  if (retry[pe]) return;
+  const double *o = R + tid;
+#pragma unroll
+  for (int q = 0; q < 9; q++) {
+    dv[q] = o[q * GP];
+    da[q] = o[(9 + q) * GP];
+  }
+#pragma unroll
+  for (int q = 0; q < 6; q++) rr[q] = o[(18 + q) * GP];
+  double curl[3] = {0., 0., 0.};
+  if (MHD)
+    for (int q = 0; q < 3; q++) curl[q] = o[(28 + q) * GP];
+  const double2 s = t_sums[te];
+  dens_store<MHD>(dc, pe, t_hfin[te], s.x, s.y, o[24 * GP], o[25 * GP], MHD ? o[27 * GP] : 0., dv, da, rr, curl,
+                  iparts, th_out, out, p_nneigh, (int)o[26 * GP], flags);
 }
 
 void launch_dens_sums(phsph_ctx *c, const TileLists &tl, bool mhd, bool mixed, const DensIn &in, const DensOut &out) {

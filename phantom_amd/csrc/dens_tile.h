@@ -4,8 +4,7 @@
 #include "tile.h"
 
 enum { DFL_CAND = 1, DFL_LIST = 2, DFL_REWALK = 4, DFL_NOCONV = 8, DFL_NEGH = 16, DFL_STACK = 32, DFL_TILE = 64 };
-// c->counters: particles that outgrew their lists, groups for the large tile
-constexpr int CNT_REWALK = 8, CNT_BIG = 9;
+constexpr int CNT_REWALK = 8;  // c->counters: particles that outgrew their lists (tiles)
 
 struct DensIn {
   const double4 *tp;  // x, y, z (treecache) and h at entry
@@ -27,7 +26,7 @@ struct DensOut {
 template <bool MHD>
 __device__ __forceinline__ void dens_store(const DevConst &dc, int p, double hfin, double rs_rho, double rs_gh,
                                            double rs_gs, double rs_divv, double rs_divB, const double *dv,
-                                           const double *da, const double *rr, const double *dB,
+                                           const double *da, const double *rr, const double *curlB,
                                            const int32_t *__restrict__ iparts, double *__restrict__ th_out,
                                            const DensOut &out, int32_t *__restrict__ p_nneigh, int nneigh,
                                            int32_t *__restrict__ flags) {
@@ -79,9 +78,9 @@ __device__ __forceinline__ void dens_store(const DevConst &dc, int p, double hfi
     for (int k = 0; k < 9; k++) out.dvdx[(size_t)o * 9 + k] = (float)gv[k];
   if (MHD && out.divcurlB) {
     out.divcurlB[(size_t)o * 4 + 0] = (float)(-rs_divB * term);
-    out.divcurlB[(size_t)o * 4 + 1] = (float)(-(dB[7] - dB[5]) * term);
-    out.divcurlB[(size_t)o * 4 + 2] = (float)(-(dB[2] - dB[6]) * term);
-    out.divcurlB[(size_t)o * 4 + 3] = (float)(-(dB[3] - dB[1]) * term);
+    out.divcurlB[(size_t)o * 4 + 1] = (float)(-curlB[0] * term);
+    out.divcurlB[(size_t)o * 4 + 2] = (float)(-curlB[1] * term);
+    out.divcurlB[(size_t)o * 4 + 3] = (float)(-curlB[2] * term);
   }
   p_nneigh[p] = nneigh;
 }
@@ -89,9 +88,7 @@ __device__ __forceinline__ void dens_store(const DevConst &dc, int p, double hfi
 // outputs of the search and h iteration, by active slot (t_), tree position
 // (p_, retry, htraj, hconv) and leaf
 struct DensIterOut {
-  uint32_t *nlist;  // list_at layout, capl entries per slot
-  int capl;
-  int32_t *t_nl, *t_nlj;
+  int32_t *t_nl;
   double *t_hsum, *t_hfin;
   int32_t *p_nits, *leaf_nits, *retry, *nrewalk;
   double *htraj;
@@ -154,6 +151,4 @@ struct IterSums {
 void launch_dens_tile(phsph_ctx *c, int icall, double rfac, double lmargin, const double *hmax0,
                       const DensIterOut &out, const TileLists &tl);
 void launch_dens_sums(phsph_ctx *c, const TileLists &tl, bool mhd, bool mixed, const DensIn &in, const DensOut &out);
-// the list buffers for the context's tile groups
-int tile_lists(phsph_ctx *c, TileLists &tl);
 int dens_tile_list_cap(const phsph_ctx *c);

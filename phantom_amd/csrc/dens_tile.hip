@@ -26,7 +26,8 @@
 //
 // Bound by vector instructions: 83 % of the issue slots at 4600 per wavefront
 // of 16 particles on the 8M-particle box (5.4 ms) with an FP64 test and the
-// kernel evaluated per neighbour.
+// kernel evaluated per neighbour; 3.9 ms now (10.6 ms as a search and iteration
+// over per-lane lists).
 //
 // Offsets.  get_sep (kdtree.F90:1468-1501) takes a leaf's offset from the two
 // leaf centres.  Here it is taken from the group's box centre, which gives the
@@ -38,7 +39,7 @@
 // small for that go to the list kernels.
 template <int K, int V>
 __global__ void __launch_bounds__((64 * TileCap<K, V>::W)) __attribute__((amdgpu_waves_per_eu(TileCap<K, V>::WPE)))
-k_dens_tile(DevConst dc, int icall, double rfac, double lmargin, const int32_t *__restrict__ act, int nact, int ngroups,
+k_dens_tile(DevConst dc, int icall, double rfac, double lmargin, const int32_t *__restrict__ act, int ngroups,
             const int32_t *__restrict__ gt,
             const double *__restrict__ gbox, const int32_t *__restrict__ pleaf, const uint32_t *__restrict__ gcand,
             const int32_t *__restrict__ gncand, const int64_t *goff, int capg, const int32_t *__restrict__ nd_lo,
@@ -157,7 +158,6 @@ k_dens_tile(DevConst dc, int icall, double rfac, double lmargin, const int32_t *
     for (int k = tid; k < nc; k += 64 * W) gcl[k] = cj[k];
   if (tid == 0) (BIG ? tl.bnc[b] : tl.nc[g]) = bad ? -1 : nc;
   const int pi = lane / TILE_L, sl = lane % TILE_L;
-  const int lcap = min(LC, out.capl);
   bool redo = false;  // a list of this group did not fit
   auto wave16 = [&](const int wt) {  // 16 particles of the wavefront
     const int t = wt + pi;
@@ -241,9 +241,9 @@ k_dens_tile(DevConst dc, int icall, double rfac, double lmargin, const int32_t *
       }
       wave_lds_sync();
     }
-    const bool full = n > lcap;
-    redo = redo || __ballot(full && !BIG && n > LC) != 0ull;
-    if (full && sl == 0 && (BIG || n <= LC)) {
+    const bool full = n > LC;
+    redo = redo || __ballot(full && !BIG) != 0ull;
+    if (full && sl == 0 && BIG) {
       out.retry[p] = 1;
       atomicOr(flags, DFL_TILE);
     }
@@ -261,10 +261,7 @@ k_dens_tile(DevConst dc, int icall, double rfac, double lmargin, const int32_t *
     double r[NE];
     if constexpr (BIG) {
       uint16_t *ll = gll + (size_t)((wt - t0) / TILE_P) * tl.blc * TILE_P;
-      for (int k = sl; k < nl; k += TILE_L) {
-        out.nlist[list_at(nact, t, k)] = cj[L[k][pi]];
-        ll[k * TILE_P + pi] = L[k][pi];
-      }
+      for (int k = sl; k < nl; k += TILE_L) ll[k * TILE_P + pi] = L[k][pi];
     } else {
       uint16_t *ll = gll + (size_t)w * LC * TILE_P;
 #pragma unroll
@@ -276,7 +273,6 @@ k_dens_tile(DevConst dc, int icall, double rfac, double lmargin, const int32_t *
             const int s = L[k][pi];
             r[e] = dist(s);
             ll[k * TILE_P + pi] = (uint16_t)s;
-            out.nlist[((size_t)(TILE_L * e / LSEG) * nact + t) * LSEG + TILE_L * e % LSEG + sl] = cj[s];
           }
         }
       }
@@ -346,7 +342,6 @@ k_dens_tile(DevConst dc, int icall, double rfac, double lmargin, const int32_t *
           const int nit = (icall == 0) ? 1 : it;
           if (out.hconv) out.hconv[p] = hi;  // the h of the last summation (cell%h once converged)
           out.t_nl[t] = n;
-          if (out.t_nlj) out.t_nlj[t] = 0;
           out.t_sums[t] = make_double2(srho, sgh);
           out.t_hsum[t] = hi;
           out.t_hfin[t] = hfin;
@@ -392,7 +387,7 @@ void launch_dens_tile(phsph_ctx *c, int icall, double rfac, double lmargin, cons
   const dim3 gr(xcd_grid(ng)), gb((unsigned)(c->ncu > 0 ? c->ncu : 256));
 #define DT(KK, VV, GG)                                                                                             \
   hipLaunchKernelGGL((k_dens_tile<KK, VV>), GG, dim3(64 * TileCap<KK, VV>::W), 0, c->stream, c->dc, icall, rfac,   \
-                     lmargin, c->act.p, c->nact, ng, c->tg_t.p, c->gbox.p, c->pleaf.p, c->gcand.p, c->gncand.p,     \
+                     lmargin, c->act.p, ng, c->tg_t.p, c->gbox.p, c->pleaf.p, c->gcand.p, c->gncand.p,     \
                      c->goff_p, c->caps.gcand, c->nd_lo.p, c->nd_hi.p, c->nd.p, c->tp4.p, hmax0, out, tl,        \
                      c->counters.p)
   const bool w4 = c->tg_max <= 4 * TILE_P;
@@ -434,7 +429,7 @@ int tile_lists(phsph_ctx *c, TileLists &tl) {
   tl.list = c->tl_list.p;
   tl.nc = c->tl_nc.p;
   tl.big = c->tg_big.p;
-  tl.nbig = c->counters.p + CNT_BIG;
+  tl.nbig = c->tg_big.p + ng;
   tl.bcand = c->tl_bcand.p;
   tl.blist = c->tl_blist.p;
   tl.bnc = c->tl_bnc.p;

@@ -647,7 +647,8 @@ k_dens_final(DevConst dc, const int32_t *__restrict__ act, int nact, const uint3
       e = en; r = rn; vj = vn; fj = fn;
     }
   }
-  dens_store<MHD>(dc, p, hfin, rs_rho, rs_gh, rs_gs, rs_divv, rs_divB, dv, da, rr, dB, iparts, th_out, out,
+  const double curlB[3] = {dB[7] - dB[5], dB[2] - dB[6], dB[3] - dB[1]};
+  dens_store<MHD>(dc, p, hfin, rs_rho, rs_gh, rs_gs, rs_divv, rs_divB, dv, da, rr, curlB, iparts, th_out, out,
                   p_nneigh, nneigh, flags);
 }
 
@@ -728,8 +729,8 @@ k_dens_final_mixed(DevConst dc, const int32_t *__restrict__ act, int nact, const
     rr[0] -= (double)(dxf * runix); rr[1] -= (double)(dxf * runiy); rr[2] -= (double)(dxf * runiz);
     rr[3] -= (double)(dyf * runiy); rr[4] -= (double)(dyf * runiz); rr[5] -= (double)(dzf * runiz);
   }
-  const double dB[9] = {0., 0., 0., 0., 0., 0., 0., 0., 0.};
-  dens_store<false>(dc, p, hfin, rs_rho, rs_gh, rs_gs, rs_divv, 0., dv, da, rr, dB, iparts, th_out, out, p_nneigh,
+  const double curlB[3] = {0., 0., 0.};
+  dens_store<false>(dc, p, hfin, rs_rho, rs_gh, rs_gs, rs_divv, 0., dv, da, rr, curlB, iparts, th_out, out, p_nneigh,
                     nneigh, flags);
 }
 
@@ -1332,11 +1333,11 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
     // only the first attempt's lists serve the force pass
     const bool widen = attempt == 0 && reusable;
     const bool by_tile = tile && attempt == 0;
-    PH_HIPCHECK(c, LB.ensure((size_t)list_cap(dlist) * na + 1));
-    DBuf<double> &R2B = attempt == 0 ? c->nr2 : c->nr2_r;
-    if (c->tune.r2 || c->tune_mode == TUNE_PENDING) PH_HIPCHECK(c, R2B.ensure((size_t)list_cap(dlist) * na + 2));
     int32_t zero = 0, tfl = 0;  // tfl: list overflow seen by the autotuner
     if (!by_tile || (tile_tune && attempt == 0)) {
+      PH_HIPCHECK(c, LB.ensure((size_t)list_cap(dlist) * na + 1));
+      DBuf<double> &R2B = attempt == 0 ? c->nr2 : c->nr2_r;
+      if (c->tune.r2 || c->tune_mode == TUNE_PENDING) PH_HIPCHECK(c, R2B.ensure((size_t)list_cap(dlist) * na + 2));
       rc = walk_groups(c, 0, rfac * lmargin, c->th_in.p, widen ? c->hmax0.p : nullptr);
       if (rc) return rc;
       hipLaunchKernelGGL(k_zero_i32, dim3(nblocks(n, 256)), dim3(256), 0, s, c->tmpi.p, n, 0);
@@ -1366,11 +1367,11 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
       hipLaunchKernelGGL(k_zero_i32, dim3(nblocks(n, 256)), dim3(256), 0, s, c->tmpi.p, n, 0);
       PH_HIPCHECK(c, dev_set(c, c->counters.p, &zero, sizeof(int32_t)));
       PH_HIPCHECK(c, dev_set(c, c->counters.p + CNT_REWALK, &zero, sizeof(int32_t)));
-      PH_HIPCHECK(c, dev_set(c, c->counters.p + CNT_BIG, &zero, sizeof(int32_t)));
       rc = tile_lists(c, tl);
       if (rc) return rc;
+      PH_HIPCHECK(c, dev_set(c, tl.nbig, &zero, sizeof(int32_t)));
       PH_HIPCHECK(c, c->t_sums.ensure((size_t)na + 1));
-      const DensIterOut o{LB.p, list_cap(dlist), TNL.p, widen ? c->t_nlj.p : nullptr, THS.p, THF.p, c->p_nits.p, c->leaf_nits.p,
+      const DensIterOut o{TNL.p, THS.p, THF.p, c->p_nits.p, c->leaf_nits.p,
                           c->tmpi.p, c->counters.p + CNT_REWALK, c->htraj.p, (size_t)c->htraj_stride, c->hconv.p, c->t_sums.p};
       LaunchTimer lt(c, "density_iter");
       launch_dens_tile(c, icall, rfac, lmargin, widen ? c->hmax0.p : nullptr, o, tl);

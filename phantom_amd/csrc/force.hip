@@ -17,9 +17,7 @@
 // speed, MHD stress, stopping time) are evaluated once per particle by
 // k_force_prep with the same arithmetic and packed into one 128-byte record
 // per particle, so a pair reads one cache line of j data.
-#include "records.h"
-
-enum { FFL_LIST = 2, FFL_DTC = 32 };
+#include "force_tile.h"
 
 // per-particle j terms (force.F90:1455-1509 with get_stress)
 __global__ void k_force_prep(DevConst dc, int nlive, const int32_t *__restrict__ iparts,
@@ -449,85 +447,13 @@ k_force(DevConst dc, const int32_t *__restrict__ act, int nact, const int32_t *_
       }
     }
   }
-  // --- finish_cell_and_store_results ---
   double dtc_o = PH_HUGE64, dtf_o = PH_HUGE64;
   int bmax = -1;
   if (live) {
-      const int o = abs(iparts[p]) - 1;
-      if (MHD) {
-        const double B2i = Bxi * Bxi + Byi * Byi + Bzi * Bzi;
-        double frac = 0.;
-        if (B2i > 0.) {
-          const double betai = 2. * pri / B2i;
-          frac = (betai < 2.) ? 1. : (betai < 10.) ? (10. - betai) * 0.125 : 0.;
-        }
-        fx = fx - Bxi * divBsym * frac;
-        fy = fy - Byi * divBsym * frac;
-        fz = fz - Bzi * divBsym * frac;
-        if (out.divBsymm) out.divBsymm[o] = (float)(rhoi * divBsym);
-      }
-      const double f2i = fx * fx + fy * fy + fz * fz;
-      double *fo = out.fxyzu + (size_t)o * out.ldf;
-      fo[0] = fx; fo[1] = fy; fo[2] = fz;
-      const double drhodti = pm * drhodt;
-      const double divvi = -drhodti * rho1i;
-      out.divcurlv[(size_t)o * out.lddcv] = (float)divvi;
-      double dtc = dc.dtmax, dtf = PH_BIGNUMBER, dtclean = PH_BIGNUMBER, dtdusti = PH_BIGNUMBER;
-      double fxyz4 = 0.;
-      if (THERMAL) {
-        const double rhogasi = DUST ? rhoi * (1. - epsi) : rhoi;
-        const double fac = (rhogasi > PH_TINY64) ? rhoi / rhogasi : 0.;
-        const double pdv_work = fac * pri * rho1i * rho1i * drhodti;
-        if (dc.ipdv_heating > 0) fxyz4 += pdv_work;
-        if (dc.ishock_heating > 0) fxyz4 += fac * dudtdiss;
-        fxyz4 += fac * dendtdiss;
-        if (DUST) fxyz4 += 0.5 * fac * rho1i * dudtdust;
-      }
-      if (MHD) {
-        double *dB = out.dBevol + (size_t)o * 4;
-        dB[0] = dBx_s; dB[1] = dBy_s; dB[2] = dBz_s;
-        if (dc.psidecayfac > 0.) {
-          const double vclean = dc.overcleanfac * vwavei;
-          const double dtau = dc.psidecayfac * vclean * hi1;
-          dB[3] = -vclean * divBdiff * rho1i - psii * dtau - 0.5 * psii * divvi;
-          dtclean = dc.C_cour * hi / (vclean + PH_TINY64);
-        }
-      }
-      if (DUST) {
-        const double om = 1. - epsi;
-        out.ddustevol[o] = 0.5 * (ddust * rho1i / (om * om));
-        out.deltav[(size_t)o * 3 + 0] = dvx_s;
-        out.deltav[(size_t)o * 3 + 1] = dvy_s;
-        out.deltav[(size_t)o * 3 + 2] = dvz_s;
-        if (out.tstop) out.tstop[o] = tsi;
-        if (epsi > 0. && csi > 0. && epsi > PH_EPS64) {
-          const double tseff = (1. - epsi) / epsi * (epsi * tsi);
-          const double den = epsi * tseff * csi * csi;
-          if (den > PH_TINY64) dtdusti = dc.C_force * hi * hi / den;
-        }
-      }
-      const double vsigdtc = fmax(vsigmax, vwavei);
-      if (vsigdtc > PH_TINY64) dtc = dc.C_cour * hi / (vsigdtc * fmax(dc.alpha, 1.0));
-      if (THERMAL) {
-        if (eni + dtc * fxyz4 < PH_EPS64 && eni > PH_EPS64) fxyz4 = fxyz4 / (1. - dtc * fxyz4 / eni);
-        fo[3] = fxyz4;
-      }
-      if (fabs(f2i) > PH_EPS64) dtf = dc.C_force * sqrt(hi / sqrt(f2i));
-      if (!(dtc > PH_TINY64) || !(dtc < PH_HUGE64)) atomicOr(flags, FFL_DTC);
-      dtc_o = dtc;
-      dtf_o = fmin(fmin(dtf, dtdusti), dtclean);
-      if (ind) {
-        // force.F90:3272-3310: the particle's own timestep and its new bin
-        double dti = dtc;
-        const double dtitmp = fmin(fmin(dtf, dtclean), dtdusti);
-        if (dtitmp < dti + PH_TINY64 && dtitmp < dc.dtmax) dti = dtitmp;
-        int b = get_newbin_d(dti, dc.dtmax, (int)out.ibin[o], icall < 2, out.nbinmax, out.istepfrac);
-        b = max(b, ibin_neighi - 1);  // Saitoh-Makino limiter
-        out.ibin[o] = (int8_t)b;
-        bmax = b;
-        dtc_o = PH_HUGE64;
-        dtf_o = PH_HUGE64;
-      }
+    const ForceI I{hi, hi1, rhoi, rho1i, pri, csi, vwavei, eni, Bxi, Byi, Bzi, psii, epsi, tsi};
+    const ForceSums S{fx, fy, fz, drhodt, dudtdiss, dendtdiss, vsigmax, divBsym, dBx_s, dBy_s, dBz_s, divBdiff,
+                      ddust, dudtdust, dvx_s, dvy_s, dvz_s, ibin_neighi};
+    force_store<MHD, DUST, THERMAL>(dc, out, abs(iparts[p]) - 1, I, S, icall, dtc_o, dtf_o, bmax, flags);
   }
   // global minima (force.F90:3312-3327), pair count, highest bin
   reduce_force_block(dtc_o, dtf_o, npair, bmax, dtred, flags);
@@ -721,45 +647,13 @@ k_force_mixed(DevConst dc, const int32_t *__restrict__ act, int nact, const int3
       dendtdiss += (double)(vsigu * denij * (autermf * (float)grkerni + 0.5f * pmf * (float)rho1j * alphauf * (float)grkernj));
     }
   }
-  // --- finish_cell_and_store_results (hydro) ---
   double dtc_o = PH_HUGE64, dtf_o = PH_HUGE64;
   int bmax = -1;
   if (live) {
-    const int o = abs(iparts[p]) - 1;
-    const double f2i = fx * fx + fy * fy + fz * fz;
-    double *fo = out.fxyzu + (size_t)o * out.ldf;
-    fo[0] = fx; fo[1] = fy; fo[2] = fz;
-    const double drhodti = pm * drhodt;
-    const double divvi = -drhodti * rho1i;
-    out.divcurlv[(size_t)o * out.lddcv] = (float)divvi;
-    double dtc = dc.dtmax, dtf = PH_BIGNUMBER;
-    double fxyz4 = 0.;
-    if (THERMAL) {
-      const double pdv_work = pri * rho1i * rho1i * drhodti;
-      if (dc.ipdv_heating > 0) fxyz4 += pdv_work;
-      if (dc.ishock_heating > 0) fxyz4 += dudtdiss;
-      fxyz4 += dendtdiss;
-    }
-    const double vsigdtc = fmax(vsigmax, vwavei);
-    if (vsigdtc > PH_TINY64) dtc = dc.C_cour * hi / (vsigdtc * fmax(dc.alpha, 1.0));
-    if (THERMAL) {
-      if (eni + dtc * fxyz4 < PH_EPS64 && eni > PH_EPS64) fxyz4 = fxyz4 / (1. - dtc * fxyz4 / eni);
-      fo[3] = fxyz4;
-    }
-    if (fabs(f2i) > PH_EPS64) dtf = dc.C_force * sqrt(hi / sqrt(f2i));
-    if (!(dtc > PH_TINY64) || !(dtc < PH_HUGE64)) atomicOr(flags, FFL_DTC);
-    dtc_o = dtc;
-    dtf_o = dtf;
-    if (ind) {  // force.F90:3272-3310
-      double dti = dtc;
-      if (dtf < dti + PH_TINY64 && dtf < dc.dtmax) dti = dtf;
-      int b = get_newbin_d(dti, dc.dtmax, (int)out.ibin[o], icall < 2, out.nbinmax, out.istepfrac);
-      b = max(b, ibin_neighi - 1);
-      out.ibin[o] = (int8_t)b;
-      bmax = b;
-      dtc_o = PH_HUGE64;
-      dtf_o = PH_HUGE64;
-    }
+    const ForceI I{hi, hi1, rhoi, rho1i, pri, Ri.cs, vwavei, eni, 0., 0., 0., 0., 0., 0.};
+    const ForceSums S{fx, fy, fz, drhodt, dudtdiss, dendtdiss, vsigmax, 0., 0., 0., 0., 0., 0., 0., 0., 0., 0.,
+                      ibin_neighi};
+    force_store<false, false, THERMAL>(dc, out, abs(iparts[p]) - 1, I, S, icall, dtc_o, dtf_o, bmax, flags);
   }
   reduce_force_block(dtc_o, dtf_o, npair, bmax, dtred, flags);
 }
@@ -1080,9 +974,19 @@ int force_run(phsph_ctx *c, int icall, const ForceIOArgs &a, double *dtc_out, do
   ForcePass fp{rec, recB, recD, rec32, mixed, mhd, dust};
   if (reuse) {
     // the density lists, without the particles the density pass ran again
-    rc = force_pass(c, icall, a, fp, c->nlist.p, nullptr, c->t_nl.p, c->t_nlj.p, c->dlist_cap,
-                    c->dlist_nretry > 0 ? c->dretry0.p : nullptr);
-    if (rc) return rc;
+    const int32_t *skip = c->dlist_nretry > 0 ? c->dretry0.p : nullptr;
+    if (c->dlist_tile) {
+      TileLists tl;
+      rc = tile_lists(c, tl);
+      if (rc) return rc;
+      LaunchTimer lt(c, "force");
+      launch_force_tile(c, icall, a, tl, ForceTileIn{rec, recB, recD, rec32, c->fpos.p, c->fvel.p}, mixed, mhd, dust,
+                        skip);
+      PH_HIPCHECK(c, hipGetLastError());
+    } else {
+      rc = force_pass(c, icall, a, fp, c->nlist.p, nullptr, c->t_nl.p, c->t_nlj.p, c->dlist_cap, skip);
+      if (rc) return rc;
+    }
     if (c->dlist_nretry > 0) {  // those particles get lists of their own
       // the walk and the compaction below use the flag counters: keep this
       // pass's flags and bin maximum

@@ -101,6 +101,8 @@ struct TileGroup {
     return nc >= 0 && t0 < t1;
   }
 };
+// the list buffers for the context's tile groups (dens_tile.hip)
+int tile_lists(phsph_ctx *c, TileLists &tl);
 static inline unsigned tile_grid(int ngroups, const TileLists &tl) { return xcd_grid(ngroups) + (unsigned)tl.bcap; }
 
 // r and 1/(r + eps) of a squared separation, from a reciprocal square root
@@ -120,6 +122,20 @@ __device__ __forceinline__ void sqrt_rsqrt_sep(double r2, double eps, double &r,
   h = h + h;
   const double e1 = fma(-(r + eps), h, 1.);
   r1 = fma(h, e1, h);
+}
+
+// 1/sqrt(x) for x >= 0 (below 1e-290: about 1e145), to about one unit in the
+// last place
+__device__ __forceinline__ double rsqrt_pos(double x) {
+  const double a = fmax(x, 1e-290);
+  const double y = __builtin_amdgcn_rsq(a);
+  double g = a * y, h = 0.5 * y;
+  const double e = fma(-h, g, 0.5);
+  g = fma(g, e, g);
+  h = fma(h, e, h);
+  h = h + h;
+  const double e1 = fma(-g, h, 1.);
+  return fma(h, 0.5 * e1, h);
 }
 
 // dw/dq without branches: sums of max(k - q, 0)^n (kernel_cubic.f90:34-60,
