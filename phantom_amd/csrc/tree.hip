@@ -854,27 +854,39 @@ __global__ void k_bn_finish(const BigNode *bn, int maxch, int32_t *counters, con
 
 // ------------------------------------------------------------------------
 // small nodes: one workgroup builds the whole subtree in LDS, level by
-// level, with the reference's sequential arithmetic.  A node of more than
-// SUB_WAVE_MIN particles is built by one wavefront: its maxima, minima and
-// the partition run across the lanes (the partition as the permutation of
-// sort_particles_in_cell, see k_bn_pcount), and its four running sums are
-// four dependent chains in lanes 0-3.  Smaller nodes take one thread each.
+// level, with the reference's sequential arithmetic.  A node takes L lanes of
+// one wavefront, L the power of two that spreads the level's nodes over the
+// workgroup (64 lanes for the first four nodes, one for more than 128): maxima,
+// minima and the partition run across the lanes (the partition as the
+// permutation of sort_particles_in_cell, see k_bn_pcount), and the four running
+// sums are four dependent chains in the lanes, one each where there are four.
+// Latency-bound by the chains: 1.98 ms on 8.4M particles, 0.70 ms on the 1M
+// polytrope; one thread per node of up to 64 particles took 2.82 and 0.87 (16 to
+// 64 lanes of 256 busy, reads of nodes of equal size in one LDS bank).  The rows carry one word of padding per 32 particles and start 16 banks
+// apart, so that equal nodes and the four chains read distinct banks.
 // ------------------------------------------------------------------------
-#define SUB_WAVE_MIN 64
+__device__ __forceinline__ int sub_at(int k) { return k + (k >> 5); }
+#define SUB_ROW (SUB_MAX + SUB_MAX / 32 + 8)
 
-// the running sum of one node's row in position order: lanes 0-2 add
-// fac*x, fac*y, fac*z, lane 3 adds the particle mass (kdtree.F90:655-665)
+// the running sum of one node's row in position order: fac*x for the
+// coordinates, the particle mass for the mass (kdtree.F90:655-665)
 __device__ __forceinline__ double sub_chain(const double *row, int a0, int a1, bool ism, double pm, double fac) {
   double acc = 0.;
-  int k = a0;
-  for (; k + 16 <= a1 + 1; k += 16) {
+  for (int k = a0; k <= a1; k += 16) {
     double v[16];
 #pragma unroll
-    for (int u = 0; u < 16; u++) v[u] = row[k + u];
+    for (int u = 0; u < 16; u++) v[u] = ism ? pm : row[sub_at(min(k + u, a1))];
+    if (k + 15 <= a1) {
 #pragma unroll
-    for (int u = 0; u < 16; u++) acc = xadd(acc, ism ? pm : xmul(fac, v[u]));
+      for (int u = 0; u < 16; u++) acc = xadd(acc, ism ? v[u] : xmul(fac, v[u]));
+    } else {
+#pragma unroll
+      for (int u = 0; u < 16; u++) {
+        const double b = xadd(acc, ism ? v[u] : xmul(fac, v[u]));
+        acc = (k + u <= a1) ? b : acc;
+      }
+    }
   }
-  for (; k <= a1; k++) acc = xadd(acc, ism ? pm : xmul(fac, row[k]));
   return acc;
 }
 
@@ -883,24 +895,27 @@ __global__ void __launch_bounds__(SUB_BS) k_subtrees(DevConst dc, const int32_t 
                                                      int32_t *iparts, int32_t *nd_lo, int32_t *nd_hi,
                                                      phsph_kdnode *nd, int32_t *leaf_flag, int level0,
                                                      int maxlevel_indexed, int64_t nslots, int32_t *counters) {
-  __shared__ double sx[SUB_MAX], sy[SUB_MAX], sz[SUB_MAX], shh[SUB_MAX];
+  __shared__ double srow[4][SUB_ROW];  // x, y, z, h
   __shared__ int32_t sip[SUB_MAX];
-  __shared__ int32_t sidx[SUB_MAX];  // partition pairs of the wavefront-built nodes
-  __shared__ int32_t qn[2][SUB_QMAX], ql[2][SUB_QMAX], qh[2][SUB_QMAX];
-  __shared__ double qb[2][SUB_QMAX][6];
+  __shared__ int32_t sidx[SUB_MAX];  // partition pairs
+  // nodes of a level: id, range, axis of the longest side of the bounding box
+  __shared__ int32_t qn[2][SUB_QMAX], ql[2][SUB_QMAX], qh[2][SUB_QMAX], qx[2][SUB_QMAX];
   __shared__ int qcount[2];
   const int f = blockIdx.x;
   const int root = frontier[f];
   const int lo = nd_lo[root], hi = nd_hi[root];
   const int n = hi - lo + 1;
   if (n > SUB_MAX) return;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  double *sx = srow[0], *sy = srow[1], *sz = srow[2], *shh = srow[3];
   for (int k = tid; k < n; k += SUB_BS) {
-    sx[k] = tx[lo + k]; sy[k] = ty[lo + k]; sz[k] = tz[lo + k]; shh[k] = th[lo + k]; sip[k] = iparts[lo + k];
+    const int s = sub_at(k);
+    sx[s] = tx[lo + k]; sy[s] = ty[lo + k]; sz[s] = tz[lo + k]; shh[s] = th[lo + k];
+    sip[k] = iparts[lo + k];
   }
   if (tid == 0) {
     qn[0][0] = root; ql[0][0] = 0; qh[0][0] = n - 1;
-    for (int c = 0; c < 6; c++) qb[0][0][c] = fbox[(size_t)f * 6 + c];
+    qx[0][0] = pick_axis(fbox + (size_t)f * 6);
     qcount[0] = 1;
     qcount[1] = 0;
   }
@@ -914,218 +929,146 @@ __global__ void __launch_bounds__(SUB_BS) k_subtrees(DevConst dc, const int32_t 
   while (qcount[cur] > 0) {
     const int nq = min(qcount[cur], SUB_QMAX);
     const int nxt = cur ^ 1;
-    // nodes of more than SUB_WAVE_MIN particles: one wavefront each
-    for (int t = wv; t < nq; t += SUB_BS / 64) {
-      const int a0 = ql[cur][t], a1 = qh[cur][t];
+    int L = 64;
+    while (L > 1 && nq * L > SUB_BS) L >>= 1;
+    const int sub = lane & (L - 1), l0 = lane & ~(L - 1);  // lane within the node's lanes, their first lane
+    // this node's lanes of a ballot, and those below this lane
+    const unsigned long long lm = (L == 64) ? ~0ull : (((1ull << L) - 1ull) << l0);
+    const unsigned long long lt = lm & lanemask_lt();
+    for (int t = tid / L; t < nq; t += SUB_BS / L) {
+      const int a0 = ql[cur][t], a1 = qh[cur][t], nnode = qn[cur][t];
       const int npn = a1 - a0 + 1;
-      if (npn <= SUB_WAVE_MIN) continue;
-      const int nnode = qn[cur][t];
-      double hmax = 0.;
-      for (int k = a0 + lane; k <= a1; k += 64) hmax = (shh[k] > hmax) ? shh[k] : hmax;
-      hmax = wave_max(hmax);
-      double acc = 0.;
-      if (lane < 4) acc = sub_chain(lane == 0 ? sx : (lane == 1 ? sy : sz), a0, a1, lane == 3, pm, fac);
-      const double xc = __shfl(acc, 0, 64), yc = __shfl(acc, 1, 64), zc = __shfl(acc, 2, 64);
-      const double tot = __shfl(acc, 3, 64);
-      const double D = xmul(tot, dfac);
-      const double com0 = xc / D, com1 = yc / D, com2 = zc / D;
-      double r2max = 0.;
-      for (int k = a0 + lane; k <= a1; k += 64) {
-        const double r2 = r2_exact(xsub(sx[k], com0), xsub(sy[k], com1), xsub(sz[k], com2));
-        r2max = (r2 > r2max) ? r2 : r2max;
+      double s[4];
+      if (L >= 4) {
+        double acc = 0.;
+        if (sub < 4) acc = sub_chain(srow[sub & 3], a0, a1, sub == 3, pm, fac);
+#pragma unroll
+        for (int c = 0; c < 4; c++) s[c] = __shfl(acc, l0 + c, 64);
+      } else {
+#pragma unroll
+        for (int c = 0; c < 4; c++) s[c] = sub_chain(srow[c], a0, a1, c == 3, pm, fac);
       }
-      r2max = wave_max(r2max);
+      const double tot = s[3], D = xmul(tot, dfac);
+      const double com0 = s[0] / D, com1 = s[1] / D, com2 = s[2] / D;
+      const int iaxis = qx[cur][t];
+      const double pivot = (iaxis == 0) ? com0 : (iaxis == 1) ? com1 : com2;
+      const double *sa = srow[iaxis];
+      double hmax = 0., r2max = 0.;
+      int act = 0, cl = 0;
+#pragma unroll 4
+      for (int k = a0 + sub; k <= a1; k += L) {
+        const int q = sub_at(k);
+        const double r2 = r2_exact(xsub(sx[q], com0), xsub(sy[q], com1), xsub(sz[q], com2));
+        r2max = (r2 > r2max) ? r2 : r2max;
+        hmax = (shh[q] > hmax) ? shh[q] : hmax;
+        act |= sip[k] > 0;
+        cl += sa[q] <= pivot;
+      }
+      for (int o = L >> 1; o > 0; o >>= 1) {
+        r2max = fmax(r2max, __shfl_xor(r2max, o, 64));
+        hmax = fmax(hmax, __shfl_xor(hmax, o, 64));
+        act |= __shfl_xor(act, o, 64);
+        cl += __shfl_xor(cl, o, 64);
+      }
+      const bool isleaf = npn <= PH_MINPART;
       const int il = 2 * nnode, ir = il + 1;
-      const bool bad_id = (level >= maxlevel_indexed || (int64_t)ir >= nslots);
-      if (lane == 0) {
+      const bool bad_id = !isleaf && (level >= maxlevel_indexed || (int64_t)ir >= nslots);
+      if (sub == 0) {
         phsph_kdnode e;
         e.xcen[0] = com0; e.xcen[1] = com1; e.xcen[2] = com2;
         e.size = xadd(sqrt(r2max), PH_EPS64);
         e.hmax = hmax;
         e.mass = tot;
-        e.leftchild = il;
-        e.rightchild = ir;
+        e.leftchild = isleaf ? 0 : il;
+        e.rightchild = isleaf ? 0 : ir;
         e.parent = nnode / 2;
         e.idum = 0;
         nd[nnode] = e;
         nd_lo[nnode] = lo + a0;
         nd_hi[nnode] = lo + a1;
-        leaf_flag[nnode] = 0;
+        leaf_flag[nnode] = isleaf ? ((dc.ind_timesteps && !act) ? -1 : 1) : 0;
         if (bad_id) atomicOr(&counters[CNT_ERR], TERR_NODEID);
+        if (isleaf) {
+          maxlev = max(maxlev, level);
+          minlev = min(minlev, level);
+        }
       }
-      if (bad_id) continue;
-      const double *box = qb[cur][t];
-      const int iaxis = pick_axis(box);
-      const double pivot = (iaxis == 0) ? com0 : (iaxis == 1) ? com1 : com2;
-      const double *sa = (iaxis == 0) ? sx : (iaxis == 1) ? sy : sz;
-      int cl = 0;
-      for (int base = a0; base <= a1; base += 64) {
-        const int k = base + lane;
-        cl += __popcll(__ballot(k <= a1 && sa[k] <= pivot));
-      }
+      if (isleaf || bad_id) continue;
       int nl = npn / 2;  // everything on one side: halves in place (kdtree.F90:856-865)
       if (cl > 0 && cl < npn) {
         // the k-th element > pivot of the left part [a0, a0+cl-1] swaps
         // with the k-th element <= pivot counted from the right end
         const int lend = a0 + cl - 1;
-        const unsigned long long lt = lanemask_lt();
         int nbad = 0;
-        for (int base = a0; base <= lend; base += 64) {
-          const int k = base + lane;
-          const bool b = k <= lend && !(sa[k] <= pivot);
-          const unsigned long long m = __ballot(b);
+        for (int base = a0; base <= lend; base += L) {
+          const int k = base + sub;
+          const bool b = k <= lend && !(sa[sub_at(min(k, lend))] <= pivot);
+          const unsigned long long m = __ballot(b) & lm;
           if (b) sidx[a0 + nbad + __popcll(m & lt)] = k;
           nbad += __popcll(m);
         }
         int nr = 0;
-        for (int base = lend + 1; base <= a1; base += 64) {
-          const int k = base + lane;
-          const bool b = k <= a1 && sa[k] <= pivot;
-          const unsigned long long m = __ballot(b);
+        for (int base = lend + 1; base <= a1; base += L) {
+          const int k = base + sub;
+          const bool b = k <= a1 && sa[sub_at(min(k, a1))] <= pivot;
+          const unsigned long long m = __ballot(b) & lm;
           const int j = nbad - 1 - (nr + __popcll(m & lt));
           if (b && j >= 0) sidx[a0 + nbad + j] = k;
           nr += __popcll(m);
         }
-        if (nr != nbad && lane == 0) atomicOr(&counters[CNT_ERR], TERR_COUNT);
+        if (nr != nbad && sub == 0) atomicOr(&counters[CNT_ERR], TERR_COUNT);
         const int npair = min(nbad, nr);
         wave_lds_sync();
-        for (int j = lane; j < npair; j += 64) {
-          const int pa = sidx[a0 + j], pb = sidx[a0 + nbad + j];
+        for (int j = sub; j < npair; j += L) {
+          const int ia = sidx[a0 + j], ib = sidx[a0 + nbad + j];
+          const int pa = sub_at(ia), pb = sub_at(ib);
           const double t0 = sx[pa], t1 = sy[pa], t2 = sz[pa], t3 = shh[pa];
-          const int32_t ti = sip[pa];
-          sx[pa] = sx[pb]; sy[pa] = sy[pb]; sz[pa] = sz[pb]; shh[pa] = shh[pb]; sip[pa] = sip[pb];
-          sx[pb] = t0; sy[pb] = t1; sz[pb] = t2; shh[pb] = t3; sip[pb] = ti;
+          const int32_t ti = sip[ia];
+          sx[pa] = sx[pb]; sy[pa] = sy[pb]; sz[pa] = sz[pb]; shh[pa] = shh[pb]; sip[ia] = sip[ib];
+          sx[pb] = t0; sy[pb] = t1; sz[pb] = t2; shh[pb] = t3; sip[ib] = ti;
         }
         wave_lds_sync();
         nl = cl;
       }
-      const int lA = a0, hA = a0 + nl - 1, lB = a0 + nl, hB = a1;
+      const int hA = a0 + nl - 1;
       double bA[6], bB[6];
+#pragma unroll
       for (int c = 0; c < 3; c++) {
         bA[c] = PH_HUGE64; bA[3 + c] = -PH_HUGE64;
         bB[c] = PH_HUGE64; bB[3 + c] = -PH_HUGE64;
       }
-      for (int k = lA + lane; k <= hA; k += 64) {
-        bA[0] = fmin(bA[0], sx[k]); bA[1] = fmin(bA[1], sy[k]); bA[2] = fmin(bA[2], sz[k]);
-        bA[3] = fmax(bA[3], sx[k]); bA[4] = fmax(bA[4], sy[k]); bA[5] = fmax(bA[5], sz[k]);
+#pragma unroll 4
+      for (int k = a0 + sub; k <= a1; k += L) {
+        const bool left = k <= hA;
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+          const double v = srow[c][sub_at(k)];
+          bA[c] = left ? fmin(bA[c], v) : bA[c];
+          bA[3 + c] = left ? fmax(bA[3 + c], v) : bA[3 + c];
+          bB[c] = left ? bB[c] : fmin(bB[c], v);
+          bB[3 + c] = left ? bB[3 + c] : fmax(bB[3 + c], v);
+        }
       }
-      for (int k = lB + lane; k <= hB; k += 64) {
-        bB[0] = fmin(bB[0], sx[k]); bB[1] = fmin(bB[1], sy[k]); bB[2] = fmin(bB[2], sz[k]);
-        bB[3] = fmax(bB[3], sx[k]); bB[4] = fmax(bB[4], sy[k]); bB[5] = fmax(bB[5], sz[k]);
+      for (int o = L >> 1; o > 0; o >>= 1) {
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+          bA[c] = fmin(bA[c], __shfl_xor(bA[c], o, 64));
+          bA[3 + c] = fmax(bA[3 + c], __shfl_xor(bA[3 + c], o, 64));
+          bB[c] = fmin(bB[c], __shfl_xor(bB[c], o, 64));
+          bB[3 + c] = fmax(bB[3 + c], __shfl_xor(bB[3 + c], o, 64));
+        }
       }
-      for (int c = 0; c < 3; c++) {
-        bA[c] = wave_min(bA[c]); bA[3 + c] = wave_max(bA[3 + c]);
-        bB[c] = wave_min(bB[c]); bB[3 + c] = wave_max(bB[3 + c]);
-      }
-      if (lane == 0) {
+      if (sub == 0) {
         const int slot = atomicAdd(&qcount[nxt], 2);
         if (slot + 1 >= SUB_QMAX) {
           atomicOr(&counters[CNT_ERR], TERR_QUEUE);
         } else {
-          qn[nxt][slot] = il; ql[nxt][slot] = lA; qh[nxt][slot] = hA;
-          qn[nxt][slot + 1] = ir; ql[nxt][slot + 1] = lB; qh[nxt][slot + 1] = hB;
-          for (int c = 0; c < 6; c++) { qb[nxt][slot][c] = bA[c]; qb[nxt][slot + 1][c] = bB[c]; }
+          qn[nxt][slot] = il; ql[nxt][slot] = a0; qh[nxt][slot] = hA;
+          qn[nxt][slot + 1] = ir; ql[nxt][slot + 1] = hA + 1; qh[nxt][slot + 1] = a1;
+          qx[nxt][slot] = pick_axis(bA);
+          qx[nxt][slot + 1] = pick_axis(bB);
         }
       }
-    }
-    // nodes of at most SUB_WAVE_MIN particles: one thread each
-    for (int t = tid; t < nq; t += SUB_BS) {
-      const int nnode = qn[cur][t];
-      const int a0 = ql[cur][t], a1 = qh[cur][t];
-      const int npn = a1 - a0 + 1;
-      if (npn > SUB_WAVE_MIN) continue;
-      // construct_node: sequential sums in node order
-      int nodeisactive = 0;
-      for (int k = a0; k <= a1; k++)
-        if (sip[k] > 0) { nodeisactive = 1; break; }
-      double hmax = 0., xc = 0., yc = 0., zc = 0., tot = 0.;
-      for (int k = a0; k <= a1; k++) {
-        hmax = (shh[k] > hmax) ? shh[k] : hmax;
-        tot = xadd(tot, pm);
-        xc = xadd(xc, xmul(fac, sx[k]));
-        yc = xadd(yc, xmul(fac, sy[k]));
-        zc = xadd(zc, xmul(fac, sz[k]));
-      }
-      double D = xmul(tot, dfac);
-      double com0 = xc / D, com1 = yc / D, com2 = zc / D;
-      double r2max = 0.;
-      for (int k = a0; k <= a1; k++) {
-        double r2 = r2_exact(xsub(sx[k], com0), xsub(sy[k], com1), xsub(sz[k], com2));
-        r2max = (r2 > r2max) ? r2 : r2max;
-      }
-      phsph_kdnode e;
-      e.xcen[0] = com0; e.xcen[1] = com1; e.xcen[2] = com2;
-      e.size = xadd(sqrt(r2max), PH_EPS64);
-      e.hmax = hmax;
-      e.mass = tot;
-      e.parent = nnode / 2;
-      e.idum = 0;
-      nd_lo[nnode] = lo + a0;
-      nd_hi[nnode] = lo + a1;
-      if (npn <= PH_MINPART) {
-        e.leftchild = 0; e.rightchild = 0;
-        nd[nnode] = e;
-        leaf_flag[nnode] = dc.ind_timesteps ? (nodeisactive ? 1 : -1) : 1;
-        maxlev = max(maxlev, level);
-        minlev = min(minlev, level);
-        continue;
-      }
-      const int il = 2 * nnode, ir = il + 1;
-      e.leftchild = il; e.rightchild = ir;
-      nd[nnode] = e;
-      leaf_flag[nnode] = 0;
-      if (level >= maxlevel_indexed || (int64_t)ir >= nslots) {
-        atomicOr(&counters[CNT_ERR], TERR_NODEID);
-        continue;
-      }
-      const double *box = qb[cur][t];
-      const int iaxis = pick_axis(box);
-      const double pivot = (iaxis == 0) ? com0 : (iaxis == 1) ? com1 : com2;
-      double *sa = (iaxis == 0) ? sx : (iaxis == 1) ? sy : sz;
-      // sort_particles_in_cell (kdtree.F90:937-1001), verbatim two-pointer
-      int i = a0, j = a1;
-      bool ilt = sa[i] <= pivot, jlt = sa[j] <= pivot;
-      while (i < j) {
-        if (ilt) {
-          i = i + 1;
-          ilt = sa[i] <= pivot;
-        } else if (!jlt) {
-          j = j - 1;
-          jlt = sa[j] <= pivot;
-        } else {
-          double t0 = sx[i], t1 = sy[i], t2 = sz[i], t3 = shh[i];
-          int32_t ti = sip[i];
-          sx[i] = sx[j]; sy[i] = sy[j]; sz[i] = sz[j]; shh[i] = shh[j]; sip[i] = sip[j];
-          sx[j] = t0; sy[j] = t1; sz[j] = t2; shh[j] = t3; sip[j] = ti;
-          i = i + 1;
-          j = j - 1;
-          ilt = sa[i] <= pivot;
-          jlt = sa[j] <= pivot;
-        }
-      }
-      if (!ilt) i = i - 1;
-      int nl = i - a0 + 1;
-      int nr = a1 - (jlt ? j + 1 : j) + 1;
-      if (nl == npn || nr == npn) nl = npn / 2;
-      const int lA = a0, hA = a0 + nl - 1, lB = a0 + nl, hB = a1;
-      double bA[6] = {sx[lA], sy[lA], sz[lA], sx[lA], sy[lA], sz[lA]};
-      for (int k = lA + 1; k <= hA; k++) {
-        bA[0] = fmin(bA[0], sx[k]); bA[1] = fmin(bA[1], sy[k]); bA[2] = fmin(bA[2], sz[k]);
-        bA[3] = fmax(bA[3], sx[k]); bA[4] = fmax(bA[4], sy[k]); bA[5] = fmax(bA[5], sz[k]);
-      }
-      double bB[6] = {sx[lB], sy[lB], sz[lB], sx[lB], sy[lB], sz[lB]};
-      for (int k = lB + 1; k <= hB; k++) {
-        bB[0] = fmin(bB[0], sx[k]); bB[1] = fmin(bB[1], sy[k]); bB[2] = fmin(bB[2], sz[k]);
-        bB[3] = fmax(bB[3], sx[k]); bB[4] = fmax(bB[4], sy[k]); bB[5] = fmax(bB[5], sz[k]);
-      }
-      int slot = atomicAdd(&qcount[nxt], 2);
-      if (slot + 1 >= SUB_QMAX) {
-        atomicOr(&counters[CNT_ERR], TERR_QUEUE);
-        continue;
-      }
-      qn[nxt][slot] = il; ql[nxt][slot] = lA; qh[nxt][slot] = hA;
-      qn[nxt][slot + 1] = ir; ql[nxt][slot + 1] = lB; qh[nxt][slot + 1] = hB;
-      for (int c = 0; c < 6; c++) { qb[nxt][slot][c] = bA[c]; qb[nxt][slot + 1][c] = bB[c]; }
     }
     __syncthreads();
     if (tid == 0) qcount[cur] = 0;
@@ -1134,7 +1077,9 @@ __global__ void __launch_bounds__(SUB_BS) k_subtrees(DevConst dc, const int32_t 
     __syncthreads();
   }
   for (int k = tid; k < n; k += SUB_BS) {
-    tx[lo + k] = sx[k]; ty[lo + k] = sy[k]; tz[lo + k] = sz[k]; th[lo + k] = shh[k]; iparts[lo + k] = sip[k];
+    const int s = sub_at(k);
+    tx[lo + k] = sx[s]; ty[lo + k] = sy[s]; tz[lo + k] = sz[s]; th[lo + k] = shh[s];
+    iparts[lo + k] = sip[k];
   }
   // block max/min of levels
   if (maxlev > 0 || minlev < (1 << 30)) {
