@@ -108,6 +108,12 @@ __global__ void k_walk(DevConst dc, double rfac, const phsph_kdnode *__restrict_
 // mode 0 with hmaxn: rcut = rfac*radkern*max(h of the group, hmax of the node)
 //   (density lists that also hold every j whose own radius reaches i)
 // ------------------------------------------------------------------------
+// STACK: nodes of the LDS stack.  A walk that needs more than WALK_STACK_LO
+// leaves its group to a second launch with WALK_STACK (gncand = -1).  The walk
+// is a chain of dependent node loads, about twenty per group, so what counts is
+// how many groups a CU has in flight: 4 kB of stack allow 32, the 16 kB that
+// the widest groups need allowed 10.  8M-particle box 0.67 ms (1.53 with 16 kB).
+template <int STACK>
 __global__ void __launch_bounds__(64)
 k_group_walk(DevConst dc, int mode, double rfac, const phsph_kdnode *__restrict__ nd,
              const double *__restrict__ hmaxn, const int32_t *__restrict__ leaf_flag,
@@ -116,9 +122,10 @@ k_group_walk(DevConst dc, int mode, double rfac, const phsph_kdnode *__restrict_
              const double *__restrict__ ty, const double *__restrict__ tz, const double *__restrict__ hsrc,
              int ngroups, uint32_t *__restrict__ gcand, int32_t *__restrict__ gncand, const int64_t *goff,
              int capg, double *__restrict__ gbox, int32_t *__restrict__ flags) {
-  __shared__ int stk[WALK_STACK];
+  __shared__ int stk[STACK];
   const int g = xcd_block(blockIdx.x, gridDim.x);
   if (g >= ngroups) return;
+  if (STACK == WALK_STACK && gncand[g] >= 0) return;
   const size_t gbase = cand_base(goff, g, capg);
   const int gcap = cand_cap(goff, g, capg);
   const int lane = threadIdx.x;
@@ -187,7 +194,7 @@ k_group_walk(DevConst dc, int mode, double rfac, const phsph_kdnode *__restrict_
     const bool push = open && !isleaf;
     const unsigned long long mi = __ballot(push);
     const int npush = 2 * __popcll(mi);
-    if (top + npush > WALK_STACK) {
+    if (top + npush > STACK) {
       ovf = true;
       break;
     }
@@ -200,9 +207,9 @@ k_group_walk(DevConst dc, int mode, double rfac, const phsph_kdnode *__restrict_
     __syncthreads();
   }
   if (lane == 0) {
-    gncand[g] = nc;
-    if (nc > gcap) atomicOr(flags, DFL_CAND);
-    if (ovf) atomicOr(flags, DFL_STACK);
+    gncand[g] = ovf ? -1 : nc;
+    if (ovf) atomicOr(flags, STACK == WALK_STACK ? DFL_STACK : DFL_STACK_LO);
+    else if (nc > gcap) atomicOr(flags, DFL_CAND);
   }
 }
 
@@ -984,17 +991,26 @@ int walk_groups(phsph_ctx *c, int mode, double rfac, const double *d_hsrc, const
     PH_HIPCHECK(c, c->gbox.ensure((size_t)(ng + 1) * GBOX));
     int32_t zero = 0;
     PH_HIPCHECK(c, dev_set(c, c->counters.p, &zero, sizeof(int32_t)));
+#define WALK(SS)                                                                                                \
+  hipLaunchKernelGGL((k_group_walk<SS>), dim3(xcd_grid(ng)), dim3(64), 0, s, c->dc, mode, rfac, c->nd.p, d_hmaxn, \
+                     c->leaf_flag.p, c->act.p, c->nact, tiles ? c->tg_t.p : nullptr, c->tx.p, c->ty.p, c->tz.p,   \
+                     d_hsrc, ng, c->gcand.p, c->gncand.p, goff, c->caps.gcand, c->gbox.p, c->counters.p)
     if (ng > 0) {
       LaunchTimer lt(c, mode == 0 ? "walk_density" : "walk_force");
-      hipLaunchKernelGGL(k_group_walk, dim3(xcd_grid(ng)), dim3(64), 0, s, c->dc, mode, rfac, c->nd.p, d_hmaxn,
-                         c->leaf_flag.p, c->act.p, c->nact, tiles ? c->tg_t.p : nullptr, c->tx.p, c->ty.p, c->tz.p,
-                         d_hsrc, ng, c->gcand.p,
-                         c->gncand.p, goff, c->caps.gcand, c->gbox.p, c->counters.p);
+      WALK(WALK_STACK_LO);
     }
     PH_HIPCHECK(c, hipGetLastError());
     int32_t fl = 0;
     PH_HIPCHECK(c, hipMemcpyAsync(&fl, c->counters.p, sizeof(int32_t), hipMemcpyDeviceToHost, s));
     PH_HIPCHECK(c, hipStreamSynchronize(s));
+    if (fl & DFL_STACK_LO) {
+      LaunchTimer lt(c, mode == 0 ? "walk_density" : "walk_force");
+      WALK(WALK_STACK);
+      PH_HIPCHECK(c, hipGetLastError());
+      PH_HIPCHECK(c, hipMemcpyAsync(&fl, c->counters.p, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+      PH_HIPCHECK(c, hipStreamSynchronize(s));
+    }
+#undef WALK
     if (getenv("PHSPH_DEBUG")) {
       size_t fr = 0, tot = 0;
       (void)hipMemGetInfo(&fr, &tot);

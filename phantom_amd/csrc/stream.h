@@ -26,7 +26,8 @@
 #include "ctx.h"
 
 constexpr int GROUP = 64;                         // particles per group = wavefront size
-constexpr int WALK_STACK = 4096;                  // node stack of the group walk (LDS)
+constexpr int WALK_STACK_LO = 1024;               // node stack of the group walk (LDS), and of the groups
+constexpr int WALK_STACK = 4096;                  // that need more
 constexpr int HTRAJ = 16;                         // h after each density iteration kept per particle (self-gravity)
 
 // separation code of a candidate leaf for a lane: 0..26 periodic offset
