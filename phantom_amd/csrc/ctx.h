@@ -44,7 +44,7 @@ struct DBuf {
 constexpr int TREE_SUB_MAX = 1024;
 
 // One node of the tree build's large-node phase (more particles than one
-// workgroup builds in LDS): its range, split decision and chunk span.
+// workgroup splits): its range, split decision and chunk span.
 struct BigNode {
   double com[3];   // centre of mass (parallel sums, or sequential after amb)
   double tot;      // node mass
@@ -54,7 +54,7 @@ struct BigNode {
   int lo, hi;      // particle range (tree positions, inclusive)
   int nnode;       // node id
   int iaxis;       // split axis
-  int chunk0, nchunk;  // chunks of this node (0 for a small node)
+  int chunk0, nchunk;  // chunks of this node
   int nl;          // particles in the left child (0: no children)
   int part;        // the two-pointer partition moves particles
   int nbad;        // swaps of the partition
@@ -129,10 +129,11 @@ struct phsph_ctx {
   DBuf<double> th_in;        // h at densityiterate entry (tree order)
   DBuf<double> tmpd;         // scratch (tree build)
   DBuf<int32_t> tmpi, tmpi2;  // scratch (tree build)
-  DBuf<int32_t> frontier_a, frontier_b;  // node ids of a tree level
-  DBuf<double> fbox_a, fbox_b;           // their bounding boxes (6 each)
-  DBuf<BigNode> bnode;       // large nodes of a level (one per frontier entry)
-  DBuf<int32_t> ch_node;     // chunk -> frontier entry
+  DBuf<int32_t> small_n, small_x;  // nodes built in LDS, and their split axes
+  DBuf<int32_t> mid_n;       // nodes split by one workgroup, then their split axes
+  DBuf<int32_t> lev_cnt;     // large nodes and chunks of each level
+  DBuf<BigNode> bnode;       // large nodes of two levels in turn
+  DBuf<int32_t> ch_node;     // chunk -> large node, of two levels in turn
   DBuf<int32_t> ch_i;        // per-chunk counts (4 each)
   DBuf<int32_t> ch_off;      // per-chunk partition offsets (2 each)
   DBuf<double> ch_red;       // per-chunk partial sums and bounds (12 each)

@@ -9,8 +9,8 @@
 //  * Every node's centre of mass is the sequential FP64 sum over the node's
 //    particles in their current order, divided by (total mass * 1/m_gas)
 //    (:612-675).  Nodes with at most SUB_MAX particles are built inside one
-//    workgroup, one node per thread, with exactly that sequential
-//    arithmetic on LDS-resident particles.  Larger nodes (the top levels)
+//    workgroup with exactly that sequential arithmetic on LDS-resident
+//    particles.  Larger nodes (up to MID_MAX by one workgroup, above by all)
 //    sum in parallel and bound the difference to the sequential sum
 //    (|S_seq - S| <= 2 gamma_{n-1} sum|a_i|); if any particle lies within
 //    that bound of the split plane the node is re-summed sequentially, so
@@ -20,17 +20,21 @@
 //    > pivot in the left part swaps with the k-th element <= pivot counted
 //    from the right end of the right part, everything else stays.
 //  * Children are numbered 2n, 2n+1 (Gafton & Rosswog indexing, :820-823).
-#include "stream.h"
+#include "tile.h"
 
 #include <algorithm>
 
 #define SUB_MAX TREE_SUB_MAX  // particles per LDS subtree
 #define SUB_BS 256
 #define SUB_QMAX 192  // >= 2*floor(SUB_MAX/(MINPART+1)) nodes per level
+#define MID_MAX 16384  // particles per node that one workgroup splits (k_mid)
+#define MID_BS 1024
+#define MAXLEVELS 64
 
-enum { CNT_NEXT = 0, CNT_ERR = 1, CNT_FALLBACK = 2, CNT_MAXLEVEL = 3, CNT_MINLEVEL = 4, CNT_NAN = 5,
-       CNT_NLEAF = 6, CNT_LIVE = 7, CNT_NCHUNK = 8, CNT_NBIG = 9, CNT_SEQMAX = 10, CNT_TGMAX = 11, CNT_NTG = 12,
-       CNT_N = 13 };
+enum { CNT_ERR = 0, CNT_FALLBACK = 1, CNT_MAXLEVEL = 2, CNT_MINLEVEL = 3, CNT_NAN = 4, CNT_NLEAF = 5, CNT_LIVE = 6,
+       CNT_SEQMAX = 7, CNT_TGMAX = 8, CNT_NTG = 9, CNT_NSMALL = 10, CNT_NMID = 11, CNT_N = 12 };
+// per level of the large nodes: their number and that of their chunks
+enum { LEV_NBIG = 0, LEV_NCHUNK = 1, LEV_N = 2 };
 enum { TERR_NODEID = 1, TERR_QUEUE = 2, TERR_COUNT = 4 };
 
 // ------------------------------------------------------------------------
@@ -229,14 +233,14 @@ __device__ __forceinline__ int pick_axis(const double *box) {
 }
 
 // ------------------------------------------------------------------------
-// large nodes (more than SUB_MAX particles).  Every large node of a level is
+// large nodes (more than MID_MAX particles).  Every large node of a level is
 // cut into chunks of BN_CH consecutive tree positions, and each pass of
 // construct_node runs over all chunks of all large nodes of the level at
 // once, one workgroup per chunk.  One wavefront per node combines its chunk
-// results in a fixed order.  Per level: plan -> sums -> centre -> ambiguity
+// results in a fixed order.  Per level: sums -> centre -> ambiguity
 // test -> sequential sums (ambiguous nodes only) -> size and left count ->
-// node record -> partition (count, scan, scatter, swap) -> child boxes ->
-// children.
+// node record -> partition (count, scan, scatter, swap) -> children, which
+// go to the next level's large nodes or to the list of their size.
 // ------------------------------------------------------------------------
 #define BN_CH 2048
 #define BN_BS 256
@@ -301,69 +305,97 @@ __device__ __forceinline__ const double *axis_arr(int a, const double *tx, const
   return (a == 0) ? tx : (a == 1) ? ty : tz;
 }
 
-// chunk c of the level: its node (frontier entry) and positions [p0, p1];
+// The lists that split nodes add their children to: nodes of at most SUB_MAX
+// particles (k_subtrees) and of at most MID_MAX (k_mid), each with its split
+// axis, and the large nodes of the next level with their chunks.
+struct NodeLists {
+  int32_t *small, *smallx, *mid, *midx;
+  BigNode *bn;       // next level's
+  int32_t *ch_node;  // chunk -> entry of bn
+  int32_t *lev;      // next level's LEV_ counts
+  int bncap, maxch;
+  int32_t *counters;
+};
+
+// one node to its list, by a whole wavefront
+__device__ __forceinline__ void list_node(const NodeLists &L, int nnode, int lo, int hi, int axis) {
+  const int lane = threadIdx.x & 63, n = hi - lo + 1;
+  if (n <= MID_MAX) {
+    if (lane == 0) {
+      const bool sm = n <= SUB_MAX;
+      const int idx = atomicAdd(&L.counters[sm ? CNT_NSMALL : CNT_NMID], 1);
+      (sm ? L.small : L.mid)[idx] = nnode;
+      (sm ? L.smallx : L.midx)[idx] = axis;
+    }
+    return;
+  }
+  const int nch = (n + BN_CH - 1) / BN_CH;
+  int idx = 0, off = 0;
+  if (lane == 0) {
+    idx = atomicAdd(&L.lev[LEV_NBIG], 1);
+    off = atomicAdd(&L.lev[LEV_NCHUNK], nch);
+  }
+  idx = __shfl(idx, 0, 64);
+  off = __shfl(off, 0, 64);
+  if (idx >= L.bncap || off + nch > L.maxch) {
+    if (lane == 0) atomicOr(&L.counters[CNT_ERR], TERR_QUEUE);
+    return;
+  }
+  if (lane == 0) {
+    BigNode b;
+    for (int k = 0; k < 3; k++) b.com[k] = 0.;
+    b.tot = 0.; b.hmax = 0.; b.delta = 0.; b.pivot = 0.;
+    b.lo = lo; b.hi = hi; b.nnode = nnode;
+    b.iaxis = axis;
+    b.chunk0 = off; b.nchunk = nch;
+    b.nl = 0; b.part = 0; b.nbad = 0; b.pad_ = 0;
+    L.bn[idx] = b;
+  }
+  for (int k = lane; k < nch; k += 64) L.ch_node[off + k] = idx;
+}
+
+// the root: its range, and its list
+__global__ void k_tree_seed(const double *rootbox, int nlive, int32_t *nd_lo, int32_t *nd_hi, NodeLists L) {
+  if (threadIdx.x == 0) {
+    nd_lo[1] = 0;
+    nd_hi[1] = nlive - 1;
+  }
+  list_node(L, 1, 0, nlive - 1, pick_axis(rootbox));
+}
+
+// node f of the level; false past the level's count.  A level whose nodes or
+// chunks passed their capacity has raised an error and is not built.
+__device__ __forceinline__ bool bn_node(const int32_t *lev, int bncap, int maxch, int f) {
+  return f < lev[LEV_NBIG] && lev[LEV_NBIG] <= bncap && lev[LEV_NCHUNK] <= maxch;
+}
+// chunk c of the level: its node (entry of bn) and positions [p0, p1];
 // false for a block past the level's chunk count
-__device__ __forceinline__ bool bn_chunk(const BigNode *bn, const int32_t *ch_node, const int32_t *counters,
+__device__ __forceinline__ bool bn_chunk(const BigNode *bn, const int32_t *ch_node, const int32_t *lev, int bncap,
                                          int maxch, int c, int &f, int &p0, int &p1) {
-  const int nch = counters[CNT_NCHUNK];
-  if (nch > maxch || c >= nch) return false;
+  if (c >= lev[LEV_NCHUNK] || lev[LEV_NBIG] > bncap || lev[LEV_NCHUNK] > maxch) return false;
   f = ch_node[c];
   p0 = bn[f].lo + (c - bn[f].chunk0) * BN_CH;
   p1 = min(bn[f].hi, p0 + BN_CH - 1);
   return true;
 }
 
-// the level's large nodes, their chunks and split axes
-__global__ void __launch_bounds__(1024) k_bn_plan(const int32_t *frontier, const double *fbox, int nfront,
-                                                  const int32_t *nd_lo, const int32_t *nd_hi, BigNode *bn,
-                                                  int32_t *ch_node, int maxch, int32_t *counters) {
-  __shared__ int shi[16];
-  __shared__ int carry;
-  if (threadIdx.x == 0) carry = 0;
-  __syncthreads();
-  for (int base = 0; base < nfront; base += 1024) {
-    const int f = base + threadIdx.x;
-    int nch = 0, lo = 0, hi = -1, nnode = 0;
-    if (f < nfront) {
-      nnode = frontier[f];
-      lo = nd_lo[nnode];
-      hi = nd_hi[nnode];
-      const int n = hi - lo + 1;
-      nch = (n > SUB_MAX) ? (n + BN_CH - 1) / BN_CH : 0;
-    }
-    int tot;
-    const int off = carry + block_excl_scan_int<1024>(nch, shi, &tot);
-    if (f < nfront) {
-      BigNode b;
-      for (int k = 0; k < 3; k++) b.com[k] = 0.;
-      b.tot = 0.; b.hmax = 0.; b.delta = 0.; b.pivot = 0.;
-      b.lo = lo; b.hi = hi; b.nnode = nnode;
-      b.iaxis = pick_axis(fbox + (size_t)f * 6);
-      b.chunk0 = off; b.nchunk = nch;
-      b.nl = 0; b.part = 0; b.nbad = 0; b.pad_ = 0;
-      bn[f] = b;
-      for (int k = 0; k < nch; k++)
-        if (off + k < maxch) ch_node[off + k] = f;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) carry += tot;
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    counters[CNT_NCHUNK] = carry;
-    if (carry > maxch) atomicOr(&counters[CNT_ERR], TERR_QUEUE);
-  }
+// the bound on the distance of the parallel centre of a node from the
+// sequential one on the split axis (|S_seq - S| <= 2 gamma_{n-1} sum|a_i|)
+__device__ __forceinline__ double centre_bound(int n, double sum_abs, double D, double centre) {
+  const double uu = 1.1102230246251565e-16;
+  const double nu = (double)(n - 1) * uu;
+  const double gam = nu / (1. - nu);
+  return 2. * (2. * gam * sum_abs / D + (2. * gam + 4. * uu) * fabs(centre)) + 1e-300;
 }
 
 // parallel sums of m*x over a chunk, their absolute values, and hmax
-__global__ void __launch_bounds__(BN_BS) k_bn_sums(DevConst dc, const BigNode *bn, const int32_t *ch_node,
-                                                   int maxch, const int32_t *counters, const double *tx,
-                                                   const double *ty, const double *tz, const double *th,
-                                                   double *ch_red) {
+__global__ void __launch_bounds__(BN_BS) k_bn_sums(DevConst dc, const BigNode *bn, const int32_t *ch_node, int bncap,
+                                                   int maxch, const int32_t *lev, const double *tx, const double *ty,
+                                                   const double *tz, const double *th, double *ch_red) {
   __shared__ double sh[BN_BS / 64 * 7];
   const int c = blockIdx.x;
   int f, p0, p1;
-  if (!bn_chunk(bn, ch_node, counters, maxch, c, f, p0, p1)) return;
+  if (!bn_chunk(bn, ch_node, lev, bncap, maxch, c, f, p0, p1)) return;
   const double pm = dc.pmass;
   const double dfac = (pm > 0.) ? 1. / pm : 1.;
   const double fac = xmul(pm, dfac);
@@ -386,12 +418,12 @@ __global__ void __launch_bounds__(BN_BS) k_bn_sums(DevConst dc, const BigNode *b
 
 // centre of mass from the parallel sums, and the bound on its distance from
 // the sequential one on the split axis (|S_seq - S| <= 2 gamma_{n-1} sum|a_i|)
-__global__ void k_bn_centre(DevConst dc, BigNode *bn, int maxch, const int32_t *counters, const double *ch_red) {
+__global__ void k_bn_centre(DevConst dc, BigNode *bn, int bncap, int maxch, const int32_t *lev,
+                            const double *ch_red) {
   const int f = blockIdx.x, lane = threadIdx.x;
-  if (counters[CNT_NCHUNK] > maxch) return;
+  if (!bn_node(lev, bncap, maxch, f)) return;
   BigNode *b = bn + f;
   const int nchunk = b->nchunk, chunk0 = b->chunk0;
-  if (nchunk == 0) return;
   double s[3] = {0., 0., 0.}, a[3] = {0., 0., 0.}, hm = 0.;
   for (int k = lane; k < nchunk; k += 64) {
     const double *r = ch_red + (size_t)(chunk0 + k) * BN_RED;
@@ -412,26 +444,23 @@ __global__ void k_bn_centre(DevConst dc, BigNode *bn, int maxch, const int32_t *
     const double D = xmul(tot, dfac);
     double com[3];
     for (int k = 0; k < 3; k++) com[k] = s[k] / D;
-    const double uu = 1.1102230246251565e-16;
-    const double nu = (double)(n - 1) * uu;
-    const double gam = nu / (1. - nu);
     const int ia = b->iaxis;
     const double a_ax = a[ia], c_ax = com[ia];
     for (int k = 0; k < 3; k++) b->com[k] = com[k];
     b->tot = tot;
     b->hmax = hm;
-    b->delta = 2. * (2. * gam * a_ax / D + (2. * gam + 4. * uu) * fabs(c_ax)) + 1e-300;
+    b->delta = centre_bound(n, a_ax, D, c_ax);
     b->pivot = c_ax;
   }
 }
 
 // does any particle of the chunk lie within delta of the split plane?
-__global__ void __launch_bounds__(BN_BS) k_bn_amb(const BigNode *bn, const int32_t *ch_node, int maxch,
-                                                  const int32_t *counters, const double *tx, const double *ty,
+__global__ void __launch_bounds__(BN_BS) k_bn_amb(const BigNode *bn, const int32_t *ch_node, int bncap, int maxch,
+                                                  const int32_t *lev, const double *tx, const double *ty,
                                                   const double *tz, int32_t *ch_i) {
   const int c = blockIdx.x;
   int f, p0, p1;
-  if (!bn_chunk(bn, ch_node, counters, maxch, c, f, p0, p1)) return;
+  if (!bn_chunk(bn, ch_node, lev, bncap, maxch, c, f, p0, p1)) return;
   const double *tax = axis_arr(bn[f].iaxis, tx, ty, tz);
   const double c_ax = bn[f].pivot, delta = bn[f].delta;
   int amb = 0;
@@ -472,43 +501,31 @@ __device__ __forceinline__ double seq_chain(double acc, const double *src, int c
   return acc;
 }
 
-// exact sequential sums (kdtree.F90:655-665) of the nodes with a particle
-// within delta of the plane.  The four running sums (x, y, z, mass) are four
+// Exact sequential sums (kdtree.F90:655-665) of the particles [lo, hi], by a
+// whole workgroup: x, y, z and mass to seq.  The four running sums are four
 // dependent chains in lanes 0-3 of wavefront 0; the other wavefronts stage
 // the products fac*x of the next BN_SEQ positions into LDS meanwhile.  The
 // rows are padded so that the four lanes read distinct LDS banks.
 #define BN_SEQ_LD (BN_SEQ + 20)
-__global__ void __launch_bounds__(BN_SEQ_BS) k_bn_seq(DevConst dc, BigNode *bn, int maxch, int32_t *counters,
-                                                      const int32_t *ch_i, const double *tx, const double *ty,
-                                                      const double *tz) {
-  __shared__ double buf[2][3][BN_SEQ_LD];
-  __shared__ double mrow[BN_SEQ_LD];
-  __shared__ double seq[4];
-  const int f = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
-  if (counters[CNT_NCHUNK] > maxch) return;
-  const int nchunk = bn[f].nchunk, chunk0 = bn[f].chunk0;
-  if (nchunk == 0) return;
-  int amb = 0;
-  for (int k = tid; k < nchunk; k += BN_SEQ_BS) amb |= ch_i[(size_t)(chunk0 + k) * 4 + 0];
-  amb = __syncthreads_or(amb);
-  if (!amb) return;
-  const int lo = bn[f].lo, hi = bn[f].hi, iaxis = bn[f].iaxis;
-  const double pm = dc.pmass;
-  const double dfac = (pm > 0.) ? 1. / pm : 1.;
-  const double fac = xmul(pm, dfac);
+constexpr int BN_SEQ_BUF = 7 * BN_SEQ_LD;  // doubles of LDS: two stages of three rows, and a row of masses
+template <int BS>
+__device__ void seq_sums(double *buf, double *seq, int lo, int hi, double pm, double fac, const double *tx,
+                         const double *ty, const double *tz) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  double *mrow = buf + 6 * BN_SEQ_LD;
   const int n = hi - lo + 1;
   const int nst = (n + BN_SEQ - 1) / BN_SEQ;
   auto fill = [&](int st) {
     const int base = lo + st * BN_SEQ;
     const int cnt = min(BN_SEQ, hi - base + 1);
-    double(*dst)[BN_SEQ_LD] = buf[st & 1];
-    for (int k = tid - 64; k < cnt; k += BN_SEQ_BS - 64) {
-      dst[0][k] = xmul(fac, tx[base + k]);
-      dst[1][k] = xmul(fac, ty[base + k]);
-      dst[2][k] = xmul(fac, tz[base + k]);
+    double *dst = buf + (st & 1) * 3 * BN_SEQ_LD;
+    for (int k = tid - 64; k < cnt; k += BS - 64) {
+      dst[k] = xmul(fac, tx[base + k]);
+      dst[BN_SEQ_LD + k] = xmul(fac, ty[base + k]);
+      dst[2 * BN_SEQ_LD + k] = xmul(fac, tz[base + k]);
     }
   };
-  for (int k = tid; k < BN_SEQ_LD; k += BN_SEQ_BS) mrow[k] = pm;
+  for (int k = tid; k < BN_SEQ_LD; k += BS) mrow[k] = pm;
   if (tid >= 64) fill(0);
   __syncthreads();
   double acc = 0.;
@@ -517,12 +534,31 @@ __global__ void __launch_bounds__(BN_SEQ_BS) k_bn_seq(DevConst dc, BigNode *bn, 
       if (st + 1 < nst) fill(st + 1);
     } else if (lane < 4) {
       const int cnt = min(BN_SEQ, hi - (lo + st * BN_SEQ) + 1);
-      acc = seq_chain(acc, lane < 3 ? buf[st & 1][lane] : mrow, cnt);
+      acc = seq_chain(acc, lane < 3 ? buf + ((st & 1) * 3 + lane) * BN_SEQ_LD : mrow, cnt);
     }
     __syncthreads();
   }
   if (tid < 4) seq[tid] = acc;
   __syncthreads();
+}
+
+// the sequential sums of the nodes with a particle within delta of the plane
+__global__ void __launch_bounds__(BN_SEQ_BS) k_bn_seq(DevConst dc, BigNode *bn, int bncap, int maxch,
+                                                      const int32_t *lev, int32_t *counters, const int32_t *ch_i,
+                                                      const double *tx, const double *ty, const double *tz) {
+  __shared__ double buf[BN_SEQ_BUF];
+  __shared__ double seq[4];
+  const int f = blockIdx.x, tid = threadIdx.x;
+  if (!bn_node(lev, bncap, maxch, f)) return;
+  const int nchunk = bn[f].nchunk, chunk0 = bn[f].chunk0;
+  int amb = 0;
+  for (int k = tid; k < nchunk; k += BN_SEQ_BS) amb |= ch_i[(size_t)(chunk0 + k) * 4 + 0];
+  amb = __syncthreads_or(amb);
+  if (!amb) return;
+  const int lo = bn[f].lo, hi = bn[f].hi, iaxis = bn[f].iaxis;
+  const double pm = dc.pmass;
+  const double dfac = (pm > 0.) ? 1. / pm : 1.;
+  seq_sums<BN_SEQ_BS>(buf, seq, lo, hi, pm, xmul(pm, dfac), tx, ty, tz);
   if (tid == 0) {
     const double tot = seq[3];
     const double D = xmul(tot, dfac);
@@ -531,7 +567,7 @@ __global__ void __launch_bounds__(BN_SEQ_BS) k_bn_seq(DevConst dc, BigNode *bn, 
     b->tot = tot;
     b->pivot = b->com[iaxis];
     atomicAdd(&counters[CNT_FALLBACK], 1);
-    atomicMax(&counters[CNT_SEQMAX], n);
+    atomicMax(&counters[CNT_SEQMAX], hi - lo + 1);
   }
 }
 
@@ -539,13 +575,13 @@ __global__ void __launch_bounds__(BN_SEQ_BS) k_bn_seq(DevConst dc, BigNode *bn, 
 // pivot, per chunk; under self-gravity also the chunk's share of the second
 // moments about the centre of mass (kdtree.F90:724-750)
 __global__ void __launch_bounds__(BN_BS) k_bn_size(DevConst dc, const BigNode *bn, const int32_t *ch_node,
-                                                   int maxch, const int32_t *counters, const double *tx,
+                                                   int bncap, int maxch, const int32_t *lev, const double *tx,
                                                    const double *ty, const double *tz, double *ch_red,
                                                    int32_t *ch_i, int quads) {
   __shared__ double sh[BN_BS / 64 * 20];
   const int c = blockIdx.x;
   int f, p0, p1;
-  if (!bn_chunk(bn, ch_node, counters, maxch, c, f, p0, p1)) return;
+  if (!bn_chunk(bn, ch_node, lev, bncap, maxch, c, f, p0, p1)) return;
   const double c0 = bn[f].com[0], c1 = bn[f].com[1], c2 = bn[f].com[2], pivot = bn[f].pivot;
   const double *tax = axis_arr(bn[f].iaxis, tx, ty, tz);
   const double pm = dc.pmass;
@@ -589,14 +625,13 @@ __global__ void __launch_bounds__(BN_BS) k_bn_size(DevConst dc, const BigNode *b
 
 // the node record, and the split: left count or, with everything on one
 // side, half and half in place (kdtree.F90:856-865)
-__global__ void k_bn_node(BigNode *bn, int maxch, int32_t *counters, const double *ch_red, const int32_t *ch_i,
-                          phsph_kdnode *nd, int32_t *leaf_flag, int level, int maxlevel_indexed, int64_t nslots,
-                          double *quads) {
+__global__ void k_bn_node(BigNode *bn, int bncap, int maxch, const int32_t *lev, int32_t *counters,
+                          const double *ch_red, const int32_t *ch_i, phsph_kdnode *nd, int32_t *leaf_flag, int level,
+                          int maxlevel_indexed, int64_t nslots, double *quads) {
   const int f = blockIdx.x, lane = threadIdx.x;
-  if (counters[CNT_NCHUNK] > maxch) return;
+  if (!bn_node(lev, bncap, maxch, f)) return;
   BigNode *b = bn + f;
   const int nchunk = b->nchunk, chunk0 = b->chunk0;
-  if (nchunk == 0) return;
   double r2 = 0.;
   int cl = 0;
   for (int k = lane; k < nchunk; k += 64) {
@@ -645,13 +680,13 @@ __global__ void k_bn_node(BigNode *bn, int maxch, int32_t *counters, const doubl
 // sort_particles_in_cell as a permutation: the k-th element > pivot in the
 // left part [lo, lo+nl-1] swaps with the k-th element <= pivot counted from
 // the right end of the right part.  Per chunk, the counts of both kinds.
-__global__ void __launch_bounds__(BN_BS) k_bn_pcount(const BigNode *bn, const int32_t *ch_node, int maxch,
-                                                     const int32_t *counters, const double *tx, const double *ty,
+__global__ void __launch_bounds__(BN_BS) k_bn_pcount(const BigNode *bn, const int32_t *ch_node, int bncap, int maxch,
+                                                     const int32_t *lev, const double *tx, const double *ty,
                                                      const double *tz, int32_t *ch_i) {
   __shared__ double sh[BN_BS / 64 * 2];
   const int c = blockIdx.x;
   int f, p0, p1;
-  if (!bn_chunk(bn, ch_node, counters, maxch, c, f, p0, p1)) return;
+  if (!bn_chunk(bn, ch_node, lev, bncap, maxch, c, f, p0, p1)) return;
   if (!bn[f].part) return;
   const int lend = bn[f].lo + bn[f].nl - 1;
   const double pivot = bn[f].pivot;
@@ -675,11 +710,12 @@ __global__ void __launch_bounds__(BN_BS) k_bn_pcount(const BigNode *bn, const in
 }
 
 // per node: chunk offsets of both kinds in position order
-__global__ void k_bn_pscan(BigNode *bn, int maxch, int32_t *counters, const int32_t *ch_i, int32_t *ch_off) {
+__global__ void k_bn_pscan(BigNode *bn, int bncap, int maxch, const int32_t *lev, int32_t *counters,
+                           const int32_t *ch_i, int32_t *ch_off) {
   const int f = blockIdx.x, lane = threadIdx.x;
-  if (counters[CNT_NCHUNK] > maxch) return;
+  if (!bn_node(lev, bncap, maxch, f)) return;
   BigNode *b = bn + f;
-  if (b->nchunk == 0 || !b->part) return;
+  if (!b->part) return;
   const int nchunk = b->nchunk, chunk0 = b->chunk0;
   int carry_l = 0, carry_r = 0;
   for (int base = 0; base < nchunk; base += 64) {
@@ -709,14 +745,14 @@ __global__ void k_bn_pscan(BigNode *bn, int maxch, int32_t *counters, const int3
 
 // ranks of the misplaced elements: the k-th left one goes to tmpA[lo+k],
 // the k-th right one counted from the right end to tmpB[lo+k]
-__global__ void __launch_bounds__(BN_BS) k_bn_pscatter(const BigNode *bn, const int32_t *ch_node, int maxch,
-                                                       const int32_t *counters, const double *tx,
+__global__ void __launch_bounds__(BN_BS) k_bn_pscatter(const BigNode *bn, const int32_t *ch_node, int bncap, int maxch,
+                                                       const int32_t *lev, const double *tx,
                                                        const double *ty, const double *tz, const int32_t *ch_off,
                                                        int32_t *tmpA, int32_t *tmpB) {
   __shared__ int shi[BN_BS / 64];
   const int c = blockIdx.x;
   int f, p0, p1;
-  if (!bn_chunk(bn, ch_node, counters, maxch, c, f, p0, p1)) return;
+  if (!bn_chunk(bn, ch_node, lev, bncap, maxch, c, f, p0, p1)) return;
   if (!bn[f].part) return;
   const int lo = bn[f].lo, lend = lo + bn[f].nl - 1, nbad = bn[f].nbad;
   const double pivot = bn[f].pivot;
@@ -752,43 +788,37 @@ __global__ void __launch_bounds__(BN_BS) k_bn_pscatter(const BigNode *bn, const 
   }
 }
 
-// the swaps: chunk c of a node takes pairs k0 .. k0+BN_CH-1
-__global__ void __launch_bounds__(BN_BS) k_bn_swap(const BigNode *bn, const int32_t *ch_node, int maxch,
-                                                   const int32_t *counters, const int32_t *tmpA,
-                                                   const int32_t *tmpB, double *tx, double *ty, double *tz,
-                                                   double *th, int32_t *iparts) {
-  const int c = blockIdx.x;
-  int f, p0, p1;
-  if (!bn_chunk(bn, ch_node, counters, maxch, c, f, p0, p1)) return;
-  if (!bn[f].part) return;
-  const int lo = bn[f].lo, hi = bn[f].hi, nbad = bn[f].nbad;
-  const int k0 = p0 - lo;
-#pragma unroll
-  for (int u = 0; u < BN_U; u++) {
-    const int k = k0 + u * BN_BS + threadIdx.x;
-    if (k < nbad) {
-      const int pa = tmpA[lo + k], pb = tmpB[lo + k];
-      if (pa >= lo && pa <= hi && pb >= lo && pb <= hi) {
-        const double t0 = tx[pa], t1 = ty[pa], t2 = tz[pa], t3 = th[pa];
-        const int32_t ti = iparts[pa];
-        tx[pa] = tx[pb]; ty[pa] = ty[pb]; tz[pa] = tz[pb]; th[pa] = th[pb]; iparts[pa] = iparts[pb];
-        tx[pb] = t0; ty[pb] = t1; tz[pb] = t2; th[pb] = t3; iparts[pb] = ti;
-      }
-    }
-  }
-}
-
-// bounding boxes of both children, per chunk
-__global__ void __launch_bounds__(BN_BS) k_bn_box(const BigNode *bn, const int32_t *ch_node, int maxch,
-                                                  const int32_t *counters, const double *tx, const double *ty,
-                                                  const double *tz, double *ch_red) {
+// The swaps: chunk c of a node takes pairs k0 .. k0+BN_CH-1.  A node that is
+// halved in place gets the bounding boxes of both halves here instead, per
+// chunk (one split at the pivot has its children's boxes from k_bn_size).
+__global__ void __launch_bounds__(BN_BS) k_bn_swap(const BigNode *bn, const int32_t *ch_node, int bncap, int maxch,
+                                                   const int32_t *lev, const int32_t *tmpA, const int32_t *tmpB,
+                                                   double *tx, double *ty, double *tz, double *th, int32_t *iparts,
+                                                   double *ch_red) {
   __shared__ double sh[BN_BS / 64 * 12];
   const int c = blockIdx.x;
   int f, p0, p1;
-  if (!bn_chunk(bn, ch_node, counters, maxch, c, f, p0, p1)) return;
-  // a node split at the pivot has its children's boxes from k_bn_size
-  if (bn[f].nl == 0 || bn[f].part) return;
-  const int hA = bn[f].lo + bn[f].nl - 1;
+  if (!bn_chunk(bn, ch_node, lev, bncap, maxch, c, f, p0, p1)) return;
+  const int lo = bn[f].lo, hi = bn[f].hi, nbad = bn[f].nbad, nl = bn[f].nl;
+  if (bn[f].part) {
+    const int k0 = p0 - lo;
+#pragma unroll
+    for (int u = 0; u < BN_U; u++) {
+      const int k = k0 + u * BN_BS + threadIdx.x;
+      if (k < nbad) {
+        const int pa = tmpA[lo + k], pb = tmpB[lo + k];
+        if (pa >= lo && pa <= hi && pb >= lo && pb <= hi) {
+          const double t0 = tx[pa], t1 = ty[pa], t2 = tz[pa], t3 = th[pa];
+          const int32_t ti = iparts[pa];
+          tx[pa] = tx[pb]; ty[pa] = ty[pb]; tz[pa] = tz[pb]; th[pa] = th[pb]; iparts[pa] = iparts[pb];
+          tx[pb] = t0; ty[pb] = t1; tz[pb] = t2; th[pb] = t3; iparts[pb] = ti;
+        }
+      }
+    }
+    return;
+  }
+  if (nl == 0) return;
+  const int hA = lo + nl - 1;
   double v[12];
   for (int k = 0; k < 3; k++) {
     v[k] = PH_HUGE64; v[3 + k] = -PH_HUGE64;
@@ -812,14 +842,14 @@ __global__ void __launch_bounds__(BN_BS) k_bn_box(const BigNode *bn, const int32
     for (int k = 0; k < 12; k++) ch_red[(size_t)c * BN_RED + BN_BOX + k] = v[k];
 }
 
-// children: ranges, boxes, next frontier
-__global__ void k_bn_finish(const BigNode *bn, int maxch, int32_t *counters, const double *ch_red,
-                            int32_t *nd_lo, int32_t *nd_hi, int32_t *next_front, double *next_box) {
+// children: ranges, split axes, lists
+__global__ void k_bn_finish(const BigNode *bn, int bncap, int maxch, const int32_t *lev, const double *ch_red,
+                            int32_t *nd_lo, int32_t *nd_hi, NodeLists L) {
   const int f = blockIdx.x, lane = threadIdx.x;
-  if (counters[CNT_NCHUNK] > maxch) return;
+  if (!bn_node(lev, bncap, maxch, f)) return;
   const BigNode *b = bn + f;
   const int nchunk = b->nchunk, chunk0 = b->chunk0, nl = b->nl;
-  if (nchunk == 0 || nl == 0) return;
+  if (nl == 0) return;
   double v[12];
   for (int k = 0; k < 3; k++) {
     v[k] = PH_HUGE64; v[3 + k] = -PH_HUGE64;
@@ -836,19 +866,361 @@ __global__ void k_bn_finish(const BigNode *bn, int maxch, int32_t *counters, con
     v[k] = wave_min(v[k]); v[3 + k] = wave_max(v[3 + k]);
     v[6 + k] = wave_min(v[6 + k]); v[9 + k] = wave_max(v[9 + k]);
   }
+  const int il = 2 * b->nnode, ir = il + 1;
+  const int lA = b->lo, hA = b->lo + nl - 1, lB = b->lo + nl, hB = b->hi;
   if (lane == 0) {
-    const int il = 2 * b->nnode, ir = il + 1;
-    const int lA = b->lo, hA = b->lo + nl - 1, lB = b->lo + nl, hB = b->hi;
     nd_lo[il] = lA; nd_hi[il] = hA; nd_lo[ir] = lB; nd_hi[ir] = hB;
-    const int idx = atomicAdd(&counters[CNT_NEXT], 2);
-    next_front[idx] = il;
-    next_front[idx + 1] = ir;
-    for (int k = 0; k < 6; k++) {
-      next_box[(size_t)idx * 6 + k] = v[k];
-      next_box[(size_t)(idx + 1) * 6 + k] = v[6 + k];
+  }
+  list_node(L, il, lA, hA, pick_axis(v));
+  list_node(L, ir, lB, hB, pick_axis(v + 6));
+}
+
+// ------------------------------------------------------------------------
+// middle nodes (more than SUB_MAX and at most MID_MAX particles): one
+// workgroup splits a node and its descendants down to SUB_MAX, level by
+// level, with the passes of the large nodes.  The wavefronts are shared out
+// over the nodes of a level, 16 for one, 8 each for two, down to one each for
+// the 9 to 15 there can be.  Which particles lie on the left of the pivot is
+// kept as one word per 64 particles, so the partition's counts and ranks need
+// no pass over memory, and its pairs go through LDS.
+//
+// As launches over all chunks the levels of these nodes cost 13 launches each,
+// 5 us a launch on sets that do not fill the chip: the call on 262144 particles
+// 2.32 -> 1.84 ms, on 4096 1.11 -> 0.95 ms.  0.57 ms on 8.4M particles (the last
+// four levels of large nodes took 1.6 ms).  Bound by latency on small sets, by
+// memory where the workgroups' particles pass the L2.  MID_MAX: the range of a
+// 16-bit position in the pairs is 65536; 16384 leaves a set of 262144 16
+// workgroups, and above it a workgroup is no faster than the launches.
+// ------------------------------------------------------------------------
+#define MID_W (MID_BS / 64)
+#define MID_Q 16      // nodes of a level: floor(MID_MAX / (SUB_MAX + 1)) = 15 at most
+#define MID_RED 20    // doubles per wavefront: sums, or size, child boxes and second moments
+#define MID_WORDS (MID_MAX / 64 + 2 * MID_Q)
+
+template <int CTRL, class OP>
+__device__ __forceinline__ double dpp_op(double v, OP op) { return op(v, dpp_quad<CTRL>(v)); }
+// a reduction over the wavefront, the result in every lane
+template <class OP>
+__device__ __forceinline__ double wave_all(double v, OP op) {
+  v = dpp_op<DPP_XOR1>(v, op);
+  v = dpp_op<DPP_XOR2>(v, op);
+  v = dpp_op<0x141>(v, op);  // row_half_mirror
+  v = dpp_op<0x140>(v, op);  // row_mirror
+  v = op(v, __shfl_xor(v, 16, 64));
+  return op(v, __shfl_xor(v, 32, 64));
+}
+struct OpAdd { __device__ __forceinline__ double operator()(double a, double b) const { return a + b; } };
+struct OpMin { __device__ __forceinline__ double operator()(double a, double b) const { return fmin(a, b); } };
+struct OpMax { __device__ __forceinline__ double operator()(double a, double b) const { return fmax(a, b); } };
+
+__global__ void __launch_bounds__(MID_BS) k_mid(DevConst dc, double *tx, double *ty, double *tz, double *th,
+                                                int32_t *iparts, int32_t *nd_lo, int32_t *nd_hi, phsph_kdnode *nd,
+                                                int32_t *leaf_flag, int maxlevel_indexed, int64_t nslots,
+                                                double *quads, NodeLists L) {
+  // the stages of the sequential sums, then the pairs of the partition
+  static_assert(BN_SEQ_BUF * 8 >= MID_MAX * 2, "the pairs fit the stages");
+  __shared__ double buf[BN_SEQ_BUF];
+  uint16_t *pairs = reinterpret_cast<uint16_t *>(buf);
+  __shared__ double seq[4];
+  __shared__ double red[MID_W][MID_RED];
+  __shared__ int redn[MID_W];                       // particles on the left of the pivot
+  __shared__ unsigned long long lew[MID_WORDS];     // bit of each particle: on the left
+  __shared__ uint16_t rkl[MID_WORDS], rkr[MID_WORDS];  // misplaced ones before the word, left and right part
+  // nodes of a level: id, range, split axis; then centre, pivot, mass, split
+  __shared__ int qn[2][MID_Q], ql[2][MID_Q], qh[2][MID_Q], qx[2][MID_Q];
+  __shared__ int qcount[2];
+  __shared__ double qcom[MID_Q][3], qtot[MID_Q];
+  __shared__ int qamb[MID_Q], qnl[MID_Q], qnbad[MID_Q], qcx[MID_Q][2];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  if ((int)blockIdx.x >= L.counters[CNT_NMID]) return;
+  const int root = L.mid[blockIdx.x];
+  const int lo0 = nd_lo[root], n0 = nd_hi[root] - lo0 + 1;
+  if (n0 <= SUB_MAX || n0 > MID_MAX) return;
+  const double pm = dc.pmass;
+  const double dfac = (pm > 0.) ? 1. / pm : 1.;
+  const double fac = xmul(pm, dfac);
+  if (tid == 0) {
+    qn[0][0] = root; ql[0][0] = 0; qh[0][0] = n0 - 1; qx[0][0] = L.midx[blockIdx.x];
+    qcount[0] = 1;
+    qcount[1] = 0;
+  }
+  __syncthreads();
+  int cur = 0, level = 31 - __clz(root);
+  while (true) {
+    const int nq = min(qcount[cur], MID_Q);
+    if (nq == 0) break;
+    const int nxt = cur ^ 1;
+    int Lw = MID_W;  // wavefronts per node
+    while (Lw > 1 && nq * Lw > MID_W) Lw >>= 1;
+    const int t = w / Lw, wi = w % Lw, w0 = t * Lw;  // node, wavefront of the node, its first wavefront
+    const bool on = t < nq;
+    const int tq = on ? t : 0;
+    const int a0 = ql[cur][tq], n = on ? qh[cur][tq] - a0 + 1 : 0, axis = qx[cur][tq], nnode = qn[cur][tq];
+    const int nw = (n + 63) / 64;               // words of 64 particles
+    const int wo = a0 / 64 + a0 / SUB_MAX;      // first word: nodes of more than SUB_MAX share none
+    const int base = lo0 + a0;
+    if (tid < MID_Q) qamb[tid] = 0;
+    {  // sums
+      double v0 = 0., v1 = 0., v2 = 0., va = 0., vh = 0.;
+#pragma unroll 4
+      for (int j = wi; j < nw; j += Lw) {
+        const int k = 64 * j + lane;
+        if (k < n) {
+          const double x = xmul(fac, tx[base + k]), y = xmul(fac, ty[base + k]), z = xmul(fac, tz[base + k]);
+          v0 += x; v1 += y; v2 += z;
+          va += fabs(axis == 0 ? x : axis == 1 ? y : z);
+          vh = fmax(vh, th[base + k]);
+        }
+      }
+      v0 = wave_all(v0, OpAdd()); v1 = wave_all(v1, OpAdd()); v2 = wave_all(v2, OpAdd());
+      va = wave_all(va, OpAdd()); vh = wave_all(vh, OpMax());
+      if (lane == 0) {
+        red[w][0] = v0; red[w][1] = v1; red[w][2] = v2; red[w][3] = va; red[w][4] = vh;
+      }
     }
-    const int nbig = (hA - lA + 1 > SUB_MAX ? 1 : 0) + (hB - lB + 1 > SUB_MAX ? 1 : 0);
-    if (nbig) atomicAdd(&counters[CNT_NBIG], nbig);
+    __syncthreads();
+    double c0 = 0., c1 = 0., c2 = 0., tot = 0., hmax = 0., delta = 0.;
+    if (on) {
+      double s0 = 0., s1 = 0., s2 = 0., sa = 0.;
+      for (int i = w0; i < w0 + Lw; i++) {
+        s0 += red[i][0]; s1 += red[i][1]; s2 += red[i][2]; sa += red[i][3];
+        hmax = fmax(hmax, red[i][4]);
+      }
+      tot = xmul((double)n, pm);
+      const double D = xmul(tot, dfac);
+      c0 = s0 / D; c1 = s1 / D; c2 = s2 / D;
+      delta = centre_bound(n, sa, D, axis == 0 ? c0 : axis == 1 ? c1 : c2);
+    }
+    __syncthreads();  // red is written again
+    // size, left count and the children's boxes; with a particle within delta
+    // of the plane once more about the sequential centre
+    bool todo = on, exact = false;
+    while (true) {
+      const double piv = (axis == 0) ? c0 : (axis == 1) ? c1 : c2;
+      if (todo) {
+        double r2 = 0., bx[12], q[6] = {0., 0., 0., 0., 0., 0.};
+        for (int k = 0; k < 3; k++) {
+          bx[k] = bx[6 + k] = PH_HUGE64;
+          bx[3 + k] = bx[9 + k] = -PH_HUGE64;
+        }
+        int amb = 0, cl = 0;
+#pragma unroll 2
+        for (int j = wi; j < nw; j += Lw) {
+          const int k = 64 * j + lane;
+          const bool in = k < n;
+          const int p = base + min(k, n - 1);
+          const double x = tx[p], y = ty[p], z = tz[p];
+          const double ax = (axis == 0) ? x : (axis == 1) ? y : z;
+          const bool left = in && ax <= piv;
+          amb |= in && fabs(ax - piv) <= delta;
+          const unsigned long long m = __ballot(left);
+          if (lane == 0) lew[wo + j] = m;
+          cl += __popcll(m);
+          if (in) {
+            r2 = fmax(r2, r2_exact(xsub(x, c0), xsub(y, c1), xsub(z, c2)));
+            bx[0] = left ? fmin(bx[0], x) : bx[0];    bx[6] = left ? bx[6] : fmin(bx[6], x);
+            bx[1] = left ? fmin(bx[1], y) : bx[1];    bx[7] = left ? bx[7] : fmin(bx[7], y);
+            bx[2] = left ? fmin(bx[2], z) : bx[2];    bx[8] = left ? bx[8] : fmin(bx[8], z);
+            bx[3] = left ? fmax(bx[3], x) : bx[3];    bx[9] = left ? bx[9] : fmax(bx[9], x);
+            bx[4] = left ? fmax(bx[4], y) : bx[4];    bx[10] = left ? bx[10] : fmax(bx[10], y);
+            bx[5] = left ? fmax(bx[5], z) : bx[5];    bx[11] = left ? bx[11] : fmax(bx[11], z);
+            if (quads) {
+              const double dx = x - c0, dy = y - c1, dz = z - c2;
+              q[0] += pm * (dx * dx); q[1] += pm * (dx * dy); q[2] += pm * (dx * dz);
+              q[3] += pm * (dy * dy); q[4] += pm * (dy * dz); q[5] += pm * (dz * dz);
+            }
+          }
+        }
+        r2 = wave_all(r2, OpMax());
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+          bx[k] = wave_all(bx[k], OpMin()); bx[6 + k] = wave_all(bx[6 + k], OpMin());
+          bx[3 + k] = wave_all(bx[3 + k], OpMax()); bx[9 + k] = wave_all(bx[9 + k], OpMax());
+        }
+        if (quads)
+          for (int k = 0; k < 6; k++) q[k] = wave_all(q[k], OpAdd());
+        const bool anyamb = __ballot(amb) != 0ull;
+        if (lane == 0) {
+          red[w][0] = r2;
+          for (int k = 0; k < 12; k++) red[w][1 + k] = bx[k];
+          if (quads)
+            for (int k = 0; k < 6; k++) red[w][13 + k] = q[k];
+          redn[w] = cl;
+          if (!exact && anyamb) qamb[t] = 1;
+        }
+      }
+      __syncthreads();
+      // nodes that are ambiguous and not yet exact
+      bool any = false;
+      for (int i = 0; i < nq; i++) {
+        if (qamb[i] != 1) continue;
+        any = true;
+        seq_sums<MID_BS>(buf, seq, lo0 + ql[cur][i], lo0 + qh[cur][i], pm, fac, tx, ty, tz);
+        if (tid == 0) {
+          const double D = xmul(seq[3], dfac);
+          for (int k = 0; k < 3; k++) qcom[i][k] = seq[k] / D;
+          qtot[i] = seq[3];
+          atomicAdd(&L.counters[CNT_FALLBACK], 1);
+          atomicMax(&L.counters[CNT_SEQMAX], qh[cur][i] - ql[cur][i] + 1);
+        }
+        __syncthreads();
+      }
+      if (!any) break;
+      todo = on && qamb[t] == 1;
+      if (todo) {
+        c0 = qcom[t][0]; c1 = qcom[t][1]; c2 = qcom[t][2];
+        tot = qtot[t];
+        exact = true;
+      }
+      __syncthreads();
+      if (tid < MID_Q && qamb[tid] == 1) qamb[tid] = 2;
+      __syncthreads();
+    }
+    if (on && wi == 0) {  // the node's record and the split, by its first wavefront
+      double r2 = 0., bx[12];
+      int cl = 0;
+      for (int k = 0; k < 3; k++) {
+        bx[k] = bx[6 + k] = PH_HUGE64;
+        bx[3 + k] = bx[9 + k] = -PH_HUGE64;
+      }
+      for (int i = w0; i < w0 + Lw; i++) {
+        r2 = fmax(r2, red[i][0]);
+        cl += redn[i];
+        for (int k = 0; k < 3; k++) {
+          bx[k] = fmin(bx[k], red[i][1 + k]); bx[6 + k] = fmin(bx[6 + k], red[i][7 + k]);
+          bx[3 + k] = fmax(bx[3 + k], red[i][4 + k]); bx[9 + k] = fmax(bx[9 + k], red[i][10 + k]);
+        }
+      }
+      if (quads && lane < 6) {
+        double q = 0.;
+        for (int i = w0; i < w0 + Lw; i++) q += red[i][13 + lane];
+        quads[6 * (size_t)nnode + lane] = q;
+      }
+      const int il = 2 * nnode, ir = il + 1;
+      const bool bad_id = level >= maxlevel_indexed || (int64_t)ir >= nslots;
+      if (lane == 0) {
+        phsph_kdnode e;
+        e.xcen[0] = c0; e.xcen[1] = c1; e.xcen[2] = c2;
+        e.size = xadd(sqrt(r2), PH_EPS64);
+        e.hmax = hmax;
+        e.mass = tot;
+        e.leftchild = il;
+        e.rightchild = ir;
+        e.parent = nnode / 2;
+        e.idum = 0;
+        nd[nnode] = e;
+        leaf_flag[nnode] = 0;
+        if (bad_id) atomicOr(&L.counters[CNT_ERR], TERR_NODEID);
+      }
+      int nl = 0, nbad = 0;
+      if (!bad_id && cl > 0 && cl < n) {
+        nl = cl;
+        int nr = 0;
+        for (int b = 0; b < nw; b += 64) {
+          const int j = b + lane;
+          int vl = 0, vr = 0;
+          if (j < nw) {
+            const unsigned long long m = lew[wo + j];
+            const int r = cl - 64 * j;  // particles of the word in the left part
+            const unsigned long long lp = (r >= 64) ? ~0ull : (r <= 0) ? 0ull : ((1ull << r) - 1ull);
+            vl = __popcll(~m & lp);
+            vr = __popcll(m & ~lp);
+          }
+          int sl = vl, sr = vr;
+          for (int o = 1; o < 64; o <<= 1) {
+            const int ul = __shfl_up(sl, o, 64), ur = __shfl_up(sr, o, 64);
+            if (lane >= o) { sl += ul; sr += ur; }
+          }
+          if (j < nw) {
+            rkl[wo + j] = (uint16_t)(nbad + sl - vl);
+            rkr[wo + j] = (uint16_t)(nr + sr - vr);
+          }
+          nbad += __shfl(sl, 63, 64);
+          nr += __shfl(sr, 63, 64);
+        }
+        if (nbad != nr) {
+          if (lane == 0) atomicOr(&L.counters[CNT_ERR], TERR_COUNT);
+          nbad = 0;
+        }
+      } else if (!bad_id) {  // everything on one side: halves in place (kdtree.F90:856-865)
+        nl = n / 2;
+        for (int k = 0; k < 3; k++) {
+          bx[k] = bx[6 + k] = PH_HUGE64;
+          bx[3 + k] = bx[9 + k] = -PH_HUGE64;
+        }
+        for (int k = lane; k < n; k += 64) {
+          const double r[3] = {tx[base + k], ty[base + k], tz[base + k]};
+          const bool left = k < nl;
+          for (int i = 0; i < 3; i++) {
+            bx[i] = left ? fmin(bx[i], r[i]) : bx[i];
+            bx[3 + i] = left ? fmax(bx[3 + i], r[i]) : bx[3 + i];
+            bx[6 + i] = left ? bx[6 + i] : fmin(bx[6 + i], r[i]);
+            bx[9 + i] = left ? bx[9 + i] : fmax(bx[9 + i], r[i]);
+          }
+        }
+        for (int i = 0; i < 3; i++) {
+          bx[i] = wave_min(bx[i]); bx[6 + i] = wave_min(bx[6 + i]);
+          bx[3 + i] = wave_max(bx[3 + i]); bx[9 + i] = wave_max(bx[9 + i]);
+        }
+      }
+      if (lane == 0) {
+        qnl[t] = nl;
+        qnbad[t] = nbad;
+        qcx[t][0] = pick_axis(bx);
+        qcx[t][1] = pick_axis(bx + 6);
+      }
+    }
+    __syncthreads();
+    const int nl = on ? qnl[t] : 0, nbad = on ? qnbad[t] : 0;
+    // ranks of the misplaced ones (k_bn_pscatter): pair j is pairs[a0 + j] and
+    // pairs[a0 + nbad + j], positions of this workgroup's particles
+    if (nbad > 0) {
+      const unsigned long long lt = lanemask_lt();
+      for (int j = wi; j < nw; j += Lw) {
+        const unsigned long long m = lew[wo + j];
+        const int r = nl - 64 * j;
+        const unsigned long long lp = (r >= 64) ? ~0ull : (r <= 0) ? 0ull : ((1ull << r) - 1ull);
+        const unsigned long long ml = ~m & lp, mr = m & ~lp;
+        const uint16_t pos = (uint16_t)(a0 + 64 * j + lane);
+        if ((ml >> lane) & 1ull) pairs[a0 + rkl[wo + j] + __popcll(ml & lt)] = pos;
+        if ((mr >> lane) & 1ull) pairs[a0 + 2 * nbad - 1 - (rkr[wo + j] + __popcll(mr & lt))] = pos;
+      }
+    }
+    __syncthreads();
+#pragma unroll 2
+    for (int k = wi * 64 + lane; k < nbad; k += 64 * Lw) {
+      const int pa = lo0 + pairs[a0 + k], pb = lo0 + pairs[a0 + nbad + k];
+      const double t0 = tx[pa], t1 = ty[pa], t2 = tz[pa], t3 = th[pa];
+      const double u0 = tx[pb], u1 = ty[pb], u2 = tz[pb], u3 = th[pb];
+      const int32_t ti = iparts[pa], ui = iparts[pb];
+      tx[pa] = u0; ty[pa] = u1; tz[pa] = u2; th[pa] = u3; iparts[pa] = ui;
+      tx[pb] = t0; ty[pb] = t1; tz[pb] = t2; th[pb] = t3; iparts[pb] = ti;
+    }
+    if (nl > 0 && wi == 0) {
+      const int il = 2 * nnode;
+      if (lane < 2) {
+        const int a = lane ? a0 + nl : a0, e = lane ? a0 + n - 1 : a0 + nl - 1, x = qcx[t][lane];
+        nd_lo[il + lane] = lo0 + a;
+        nd_hi[il + lane] = lo0 + e;
+        if (e - a + 1 > SUB_MAX) {
+          const int slot = atomicAdd(&qcount[nxt], 1);
+          if (slot < MID_Q) {
+            qn[nxt][slot] = il + lane; ql[nxt][slot] = a; qh[nxt][slot] = e; qx[nxt][slot] = x;
+          } else {
+            atomicOr(&L.counters[CNT_ERR], TERR_QUEUE);
+          }
+        } else {
+          const int idx = atomicAdd(&L.counters[CNT_NSMALL], 1);
+          L.small[idx] = il + lane;
+          L.smallx[idx] = x;
+        }
+      }
+    }
+    __syncthreads();
+    if (tid == 0) qcount[cur] = 0;
+    cur = nxt;
+    level++;
+    __syncthreads();
   }
 }
 
@@ -860,10 +1232,12 @@ __global__ void k_bn_finish(const BigNode *bn, int maxch, int32_t *counters, con
 // minima and the partition run across the lanes (the partition as the
 // permutation of sort_particles_in_cell, see k_bn_pcount), and the four running
 // sums are four dependent chains in the lanes, one each where there are four.
-// Latency-bound by the chains: 1.98 ms on 8.4M particles, 0.70 ms on the 1M
+// Latency-bound by the chains: 1.94 ms on 8.4M particles, 0.36 ms on the 1M
 // polytrope; one thread per node of up to 64 particles took 2.82 and 0.87 (16 to
-// 64 lanes of 256 busy, reads of nodes of equal size in one LDS bank).  The rows carry one word of padding per 32 particles and start 16 banks
-// apart, so that equal nodes and the four chains read distinct banks.
+// 64 lanes of 256 busy, reads of nodes of equal size in one LDS bank), and one
+// launch per level 0.70 on the polytrope, whose nodes get small at three levels.
+// The rows carry one word of padding per 32 particles and start 16 banks apart,
+// so that equal nodes and the four chains read distinct banks.
 // ------------------------------------------------------------------------
 __device__ __forceinline__ int sub_at(int k) { return k + (k >> 5); }
 #define SUB_ROW (SUB_MAX + SUB_MAX / 32 + 8)
@@ -890,196 +1264,200 @@ __device__ __forceinline__ double sub_chain(const double *row, int a0, int a1, b
   return acc;
 }
 
-__global__ void __launch_bounds__(SUB_BS) k_subtrees(DevConst dc, const int32_t *frontier, const double *fbox,
-                                                     int nfront, double *tx, double *ty, double *tz, double *th,
+__global__ void __launch_bounds__(SUB_BS) k_subtrees(DevConst dc, const int32_t *small, const int32_t *smallx,
+                                                     double *tx, double *ty, double *tz, double *th,
                                                      int32_t *iparts, int32_t *nd_lo, int32_t *nd_hi,
-                                                     phsph_kdnode *nd, int32_t *leaf_flag, int level0,
-                                                     int maxlevel_indexed, int64_t nslots, int32_t *counters) {
+                                                     phsph_kdnode *nd, int32_t *leaf_flag, int maxlevel_indexed,
+                                                     int64_t nslots, int32_t *counters) {
   __shared__ double srow[4][SUB_ROW];  // x, y, z, h
   __shared__ int32_t sip[SUB_MAX];
   __shared__ int32_t sidx[SUB_MAX];  // partition pairs
   // nodes of a level: id, range, axis of the longest side of the bounding box
   __shared__ int32_t qn[2][SUB_QMAX], ql[2][SUB_QMAX], qh[2][SUB_QMAX], qx[2][SUB_QMAX];
   __shared__ int qcount[2];
-  const int f = blockIdx.x;
-  const int root = frontier[f];
-  const int lo = nd_lo[root], hi = nd_hi[root];
-  const int n = hi - lo + 1;
-  if (n > SUB_MAX) return;
   const int tid = threadIdx.x, lane = tid & 63;
   double *sx = srow[0], *sy = srow[1], *sz = srow[2], *shh = srow[3];
-  for (int k = tid; k < n; k += SUB_BS) {
-    const int s = sub_at(k);
-    sx[s] = tx[lo + k]; sy[s] = ty[lo + k]; sz[s] = tz[lo + k]; shh[s] = th[lo + k];
-    sip[k] = iparts[lo + k];
-  }
-  if (tid == 0) {
-    qn[0][0] = root; ql[0][0] = 0; qh[0][0] = n - 1;
-    qx[0][0] = pick_axis(fbox + (size_t)f * 6);
-    qcount[0] = 1;
-    qcount[1] = 0;
-  }
-  __syncthreads();
-  const double pm = dc.pmass;
-  const double dfac = (pm > 0.) ? 1. / pm : 1.;
-  const double fac = xmul(pm, dfac);
-  int cur = 0;
-  int level = level0;
+  const int nsmall = counters[CNT_NSMALL];
   int maxlev = 0, minlev = 1 << 30;
-  while (qcount[cur] > 0) {
-    const int nq = min(qcount[cur], SUB_QMAX);
-    const int nxt = cur ^ 1;
-    int L = 64;
-    while (L > 1 && nq * L > SUB_BS) L >>= 1;
-    const int sub = lane & (L - 1), l0 = lane & ~(L - 1);  // lane within the node's lanes, their first lane
-    // this node's lanes of a ballot, and those below this lane
-    const unsigned long long lm = (L == 64) ? ~0ull : (((1ull << L) - 1ull) << l0);
-    const unsigned long long lt = lm & lanemask_lt();
-    for (int t = tid / L; t < nq; t += SUB_BS / L) {
-      const int a0 = ql[cur][t], a1 = qh[cur][t], nnode = qn[cur][t];
-      const int npn = a1 - a0 + 1;
-      double s[4];
-      if (L >= 4) {
-        double acc = 0.;
-        if (sub < 4) acc = sub_chain(srow[sub & 3], a0, a1, sub == 3, pm, fac);
-#pragma unroll
-        for (int c = 0; c < 4; c++) s[c] = __shfl(acc, l0 + c, 64);
-      } else {
-#pragma unroll
-        for (int c = 0; c < 4; c++) s[c] = sub_chain(srow[c], a0, a1, c == 3, pm, fac);
-      }
-      const double tot = s[3], D = xmul(tot, dfac);
-      const double com0 = s[0] / D, com1 = s[1] / D, com2 = s[2] / D;
-      const int iaxis = qx[cur][t];
-      const double pivot = (iaxis == 0) ? com0 : (iaxis == 1) ? com1 : com2;
-      const double *sa = srow[iaxis];
-      double hmax = 0., r2max = 0.;
-      int act = 0, cl = 0;
-#pragma unroll 4
-      for (int k = a0 + sub; k <= a1; k += L) {
-        const int q = sub_at(k);
-        const double r2 = r2_exact(xsub(sx[q], com0), xsub(sy[q], com1), xsub(sz[q], com2));
-        r2max = (r2 > r2max) ? r2 : r2max;
-        hmax = (shh[q] > hmax) ? shh[q] : hmax;
-        act |= sip[k] > 0;
-        cl += sa[q] <= pivot;
-      }
-      for (int o = L >> 1; o > 0; o >>= 1) {
-        r2max = fmax(r2max, __shfl_xor(r2max, o, 64));
-        hmax = fmax(hmax, __shfl_xor(hmax, o, 64));
-        act |= __shfl_xor(act, o, 64);
-        cl += __shfl_xor(cl, o, 64);
-      }
-      const bool isleaf = npn <= PH_MINPART;
-      const int il = 2 * nnode, ir = il + 1;
-      const bool bad_id = !isleaf && (level >= maxlevel_indexed || (int64_t)ir >= nslots);
-      if (sub == 0) {
-        phsph_kdnode e;
-        e.xcen[0] = com0; e.xcen[1] = com1; e.xcen[2] = com2;
-        e.size = xadd(sqrt(r2max), PH_EPS64);
-        e.hmax = hmax;
-        e.mass = tot;
-        e.leftchild = isleaf ? 0 : il;
-        e.rightchild = isleaf ? 0 : ir;
-        e.parent = nnode / 2;
-        e.idum = 0;
-        nd[nnode] = e;
-        nd_lo[nnode] = lo + a0;
-        nd_hi[nnode] = lo + a1;
-        leaf_flag[nnode] = isleaf ? ((dc.ind_timesteps && !act) ? -1 : 1) : 0;
-        if (bad_id) atomicOr(&counters[CNT_ERR], TERR_NODEID);
-        if (isleaf) {
-          maxlev = max(maxlev, level);
-          minlev = min(minlev, level);
-        }
-      }
-      if (isleaf || bad_id) continue;
-      int nl = npn / 2;  // everything on one side: halves in place (kdtree.F90:856-865)
-      if (cl > 0 && cl < npn) {
-        // the k-th element > pivot of the left part [a0, a0+cl-1] swaps
-        // with the k-th element <= pivot counted from the right end
-        const int lend = a0 + cl - 1;
-        int nbad = 0;
-        for (int base = a0; base <= lend; base += L) {
-          const int k = base + sub;
-          const bool b = k <= lend && !(sa[sub_at(min(k, lend))] <= pivot);
-          const unsigned long long m = __ballot(b) & lm;
-          if (b) sidx[a0 + nbad + __popcll(m & lt)] = k;
-          nbad += __popcll(m);
-        }
-        int nr = 0;
-        for (int base = lend + 1; base <= a1; base += L) {
-          const int k = base + sub;
-          const bool b = k <= a1 && sa[sub_at(min(k, a1))] <= pivot;
-          const unsigned long long m = __ballot(b) & lm;
-          const int j = nbad - 1 - (nr + __popcll(m & lt));
-          if (b && j >= 0) sidx[a0 + nbad + j] = k;
-          nr += __popcll(m);
-        }
-        if (nr != nbad && sub == 0) atomicOr(&counters[CNT_ERR], TERR_COUNT);
-        const int npair = min(nbad, nr);
-        wave_lds_sync();
-        for (int j = sub; j < npair; j += L) {
-          const int ia = sidx[a0 + j], ib = sidx[a0 + nbad + j];
-          const int pa = sub_at(ia), pb = sub_at(ib);
-          const double t0 = sx[pa], t1 = sy[pa], t2 = sz[pa], t3 = shh[pa];
-          const int32_t ti = sip[ia];
-          sx[pa] = sx[pb]; sy[pa] = sy[pb]; sz[pa] = sz[pb]; shh[pa] = shh[pb]; sip[ia] = sip[ib];
-          sx[pb] = t0; sy[pb] = t1; sz[pb] = t2; shh[pb] = t3; sip[ib] = ti;
-        }
-        wave_lds_sync();
-        nl = cl;
-      }
-      const int hA = a0 + nl - 1;
-      double bA[6], bB[6];
-#pragma unroll
-      for (int c = 0; c < 3; c++) {
-        bA[c] = PH_HUGE64; bA[3 + c] = -PH_HUGE64;
-        bB[c] = PH_HUGE64; bB[3 + c] = -PH_HUGE64;
-      }
-#pragma unroll 4
-      for (int k = a0 + sub; k <= a1; k += L) {
-        const bool left = k <= hA;
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-          const double v = srow[c][sub_at(k)];
-          bA[c] = left ? fmin(bA[c], v) : bA[c];
-          bA[3 + c] = left ? fmax(bA[3 + c], v) : bA[3 + c];
-          bB[c] = left ? bB[c] : fmin(bB[c], v);
-          bB[3 + c] = left ? bB[3 + c] : fmax(bB[3 + c], v);
-        }
-      }
-      for (int o = L >> 1; o > 0; o >>= 1) {
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-          bA[c] = fmin(bA[c], __shfl_xor(bA[c], o, 64));
-          bA[3 + c] = fmax(bA[3 + c], __shfl_xor(bA[3 + c], o, 64));
-          bB[c] = fmin(bB[c], __shfl_xor(bB[c], o, 64));
-          bB[3 + c] = fmax(bB[3 + c], __shfl_xor(bB[3 + c], o, 64));
-        }
-      }
-      if (sub == 0) {
-        const int slot = atomicAdd(&qcount[nxt], 2);
-        if (slot + 1 >= SUB_QMAX) {
-          atomicOr(&counters[CNT_ERR], TERR_QUEUE);
-        } else {
-          qn[nxt][slot] = il; ql[nxt][slot] = a0; qh[nxt][slot] = hA;
-          qn[nxt][slot + 1] = ir; ql[nxt][slot + 1] = hA + 1; qh[nxt][slot + 1] = a1;
-          qx[nxt][slot] = pick_axis(bA);
-          qx[nxt][slot + 1] = pick_axis(bB);
-        }
-      }
+  // the launch has about as many workgroups as there are nodes
+  for (int f = blockIdx.x; f < nsmall; f += gridDim.x) {
+    const int root = small[f];
+    const int lo = nd_lo[root], hi = nd_hi[root];
+    const int n = hi - lo + 1;
+    if (n > SUB_MAX) continue;
+    for (int k = tid; k < n; k += SUB_BS) {
+      const int s = sub_at(k);
+      sx[s] = tx[lo + k]; sy[s] = ty[lo + k]; sz[s] = tz[lo + k]; shh[s] = th[lo + k];
+      sip[k] = iparts[lo + k];
+    }
+    if (tid == 0) {
+      qn[0][0] = root; ql[0][0] = 0; qh[0][0] = n - 1;
+      qx[0][0] = smallx[f];
+      qcount[0] = 1;
+      qcount[1] = 0;
     }
     __syncthreads();
-    if (tid == 0) qcount[cur] = 0;
-    cur ^= 1;
-    level++;
+    const double pm = dc.pmass;
+    const double dfac = (pm > 0.) ? 1. / pm : 1.;
+    const double fac = xmul(pm, dfac);
+    int cur = 0;
+    int level = 31 - __clz(root);
+    while (qcount[cur] > 0) {
+      const int nq = min(qcount[cur], SUB_QMAX);
+      const int nxt = cur ^ 1;
+      int L = 64;
+      while (L > 1 && nq * L > SUB_BS) L >>= 1;
+      const int sub = lane & (L - 1), l0 = lane & ~(L - 1);  // lane within the node's lanes, their first lane
+      // this node's lanes of a ballot, and those below this lane
+      const unsigned long long lm = (L == 64) ? ~0ull : (((1ull << L) - 1ull) << l0);
+      const unsigned long long lt = lm & lanemask_lt();
+      for (int t = tid / L; t < nq; t += SUB_BS / L) {
+        const int a0 = ql[cur][t], a1 = qh[cur][t], nnode = qn[cur][t];
+        const int npn = a1 - a0 + 1;
+        double s[4];
+        if (L >= 4) {
+          double acc = 0.;
+          if (sub < 4) acc = sub_chain(srow[sub & 3], a0, a1, sub == 3, pm, fac);
+  #pragma unroll
+          for (int c = 0; c < 4; c++) s[c] = __shfl(acc, l0 + c, 64);
+        } else {
+  #pragma unroll
+          for (int c = 0; c < 4; c++) s[c] = sub_chain(srow[c], a0, a1, c == 3, pm, fac);
+        }
+        const double tot = s[3], D = xmul(tot, dfac);
+        const double com0 = s[0] / D, com1 = s[1] / D, com2 = s[2] / D;
+        const int iaxis = qx[cur][t];
+        const double pivot = (iaxis == 0) ? com0 : (iaxis == 1) ? com1 : com2;
+        const double *sa = srow[iaxis];
+        double hmax = 0., r2max = 0.;
+        int act = 0, cl = 0;
+  #pragma unroll 4
+        for (int k = a0 + sub; k <= a1; k += L) {
+          const int q = sub_at(k);
+          const double r2 = r2_exact(xsub(sx[q], com0), xsub(sy[q], com1), xsub(sz[q], com2));
+          r2max = (r2 > r2max) ? r2 : r2max;
+          hmax = (shh[q] > hmax) ? shh[q] : hmax;
+          act |= sip[k] > 0;
+          cl += sa[q] <= pivot;
+        }
+        for (int o = L >> 1; o > 0; o >>= 1) {
+          r2max = fmax(r2max, __shfl_xor(r2max, o, 64));
+          hmax = fmax(hmax, __shfl_xor(hmax, o, 64));
+          act |= __shfl_xor(act, o, 64);
+          cl += __shfl_xor(cl, o, 64);
+        }
+        const bool isleaf = npn <= PH_MINPART;
+        const int il = 2 * nnode, ir = il + 1;
+        const bool bad_id = !isleaf && (level >= maxlevel_indexed || (int64_t)ir >= nslots);
+        if (sub == 0) {
+          phsph_kdnode e;
+          e.xcen[0] = com0; e.xcen[1] = com1; e.xcen[2] = com2;
+          e.size = xadd(sqrt(r2max), PH_EPS64);
+          e.hmax = hmax;
+          e.mass = tot;
+          e.leftchild = isleaf ? 0 : il;
+          e.rightchild = isleaf ? 0 : ir;
+          e.parent = nnode / 2;
+          e.idum = 0;
+          nd[nnode] = e;
+          nd_lo[nnode] = lo + a0;
+          nd_hi[nnode] = lo + a1;
+          leaf_flag[nnode] = isleaf ? ((dc.ind_timesteps && !act) ? -1 : 1) : 0;
+          if (bad_id) atomicOr(&counters[CNT_ERR], TERR_NODEID);
+          if (isleaf) {
+            maxlev = max(maxlev, level);
+            minlev = min(minlev, level);
+          }
+        }
+        if (isleaf || bad_id) continue;
+        int nl = npn / 2;  // everything on one side: halves in place (kdtree.F90:856-865)
+        if (cl > 0 && cl < npn) {
+          // the k-th element > pivot of the left part [a0, a0+cl-1] swaps
+          // with the k-th element <= pivot counted from the right end
+          const int lend = a0 + cl - 1;
+          int nbad = 0;
+          for (int base = a0; base <= lend; base += L) {
+            const int k = base + sub;
+            const bool b = k <= lend && !(sa[sub_at(min(k, lend))] <= pivot);
+            const unsigned long long m = __ballot(b) & lm;
+            if (b) sidx[a0 + nbad + __popcll(m & lt)] = k;
+            nbad += __popcll(m);
+          }
+          int nr = 0;
+          for (int base = lend + 1; base <= a1; base += L) {
+            const int k = base + sub;
+            const bool b = k <= a1 && sa[sub_at(min(k, a1))] <= pivot;
+            const unsigned long long m = __ballot(b) & lm;
+            const int j = nbad - 1 - (nr + __popcll(m & lt));
+            if (b && j >= 0) sidx[a0 + nbad + j] = k;
+            nr += __popcll(m);
+          }
+          if (nr != nbad && sub == 0) atomicOr(&counters[CNT_ERR], TERR_COUNT);
+          const int npair = min(nbad, nr);
+          wave_lds_sync();
+          for (int j = sub; j < npair; j += L) {
+            const int ia = sidx[a0 + j], ib = sidx[a0 + nbad + j];
+            const int pa = sub_at(ia), pb = sub_at(ib);
+            const double t0 = sx[pa], t1 = sy[pa], t2 = sz[pa], t3 = shh[pa];
+            const int32_t ti = sip[ia];
+            sx[pa] = sx[pb]; sy[pa] = sy[pb]; sz[pa] = sz[pb]; shh[pa] = shh[pb]; sip[ia] = sip[ib];
+            sx[pb] = t0; sy[pb] = t1; sz[pb] = t2; shh[pb] = t3; sip[ib] = ti;
+          }
+          wave_lds_sync();
+          nl = cl;
+        }
+        const int hA = a0 + nl - 1;
+        double bA[6], bB[6];
+  #pragma unroll
+        for (int c = 0; c < 3; c++) {
+          bA[c] = PH_HUGE64; bA[3 + c] = -PH_HUGE64;
+          bB[c] = PH_HUGE64; bB[3 + c] = -PH_HUGE64;
+        }
+  #pragma unroll 4
+        for (int k = a0 + sub; k <= a1; k += L) {
+          const bool left = k <= hA;
+  #pragma unroll
+          for (int c = 0; c < 3; c++) {
+            const double v = srow[c][sub_at(k)];
+            bA[c] = left ? fmin(bA[c], v) : bA[c];
+            bA[3 + c] = left ? fmax(bA[3 + c], v) : bA[3 + c];
+            bB[c] = left ? bB[c] : fmin(bB[c], v);
+            bB[3 + c] = left ? bB[3 + c] : fmax(bB[3 + c], v);
+          }
+        }
+        for (int o = L >> 1; o > 0; o >>= 1) {
+  #pragma unroll
+          for (int c = 0; c < 3; c++) {
+            bA[c] = fmin(bA[c], __shfl_xor(bA[c], o, 64));
+            bA[3 + c] = fmax(bA[3 + c], __shfl_xor(bA[3 + c], o, 64));
+            bB[c] = fmin(bB[c], __shfl_xor(bB[c], o, 64));
+            bB[3 + c] = fmax(bB[3 + c], __shfl_xor(bB[3 + c], o, 64));
+          }
+        }
+        if (sub == 0) {
+          const int slot = atomicAdd(&qcount[nxt], 2);
+          if (slot + 1 >= SUB_QMAX) {
+            atomicOr(&counters[CNT_ERR], TERR_QUEUE);
+          } else {
+            qn[nxt][slot] = il; ql[nxt][slot] = a0; qh[nxt][slot] = hA;
+            qn[nxt][slot + 1] = ir; ql[nxt][slot + 1] = hA + 1; qh[nxt][slot + 1] = a1;
+            qx[nxt][slot] = pick_axis(bA);
+            qx[nxt][slot + 1] = pick_axis(bB);
+          }
+        }
+      }
+      __syncthreads();
+      if (tid == 0) qcount[cur] = 0;
+      cur ^= 1;
+      level++;
+      __syncthreads();
+    }
+    for (int k = tid; k < n; k += SUB_BS) {
+      const int s = sub_at(k);
+      tx[lo + k] = sx[s]; ty[lo + k] = sy[s]; tz[lo + k] = sz[s]; th[lo + k] = shh[s];
+      iparts[lo + k] = sip[k];
+    }
     __syncthreads();
-  }
-  for (int k = tid; k < n; k += SUB_BS) {
-    const int s = sub_at(k);
-    tx[lo + k] = sx[s]; ty[lo + k] = sy[s]; tz[lo + k] = sz[s]; th[lo + k] = shh[s];
-    iparts[lo + k] = sip[k];
   }
   // block max/min of levels
   if (maxlev > 0 || minlev < (1 << 30)) {
@@ -1158,17 +1536,18 @@ int tree_build(phsph_ctx *c, double *d_xyzh, int ld, int np, const int8_t *d_iph
   PH_HIPCHECK(c, c->iparts.ensure(np));
   PH_HIPCHECK(c, c->tmpi.ensure(np)); PH_HIPCHECK(c, c->tmpi2.ensure(np));
   PH_HIPCHECK(c, c->dred.ensure((size_t)nb * 6 + 16));
-  PH_HIPCHECK(c, c->frontier_a.ensure((size_t)np + nb + 2));
-  PH_HIPCHECK(c, c->frontier_b.ensure((size_t)np + nb + 2));
-  PH_HIPCHECK(c, c->fbox_a.ensure((size_t)(np + 2) * 6));
-  PH_HIPCHECK(c, c->fbox_b.ensure((size_t)(np + 2) * 6));
-  // large nodes are disjoint sets of more than SUB_MAX particles: at most
-  // np/(SUB_MAX+1) per level, twice that in a frontier, and their chunks at
-  // most np/BN_CH + one per node
-  const int bn_cap = 2 * (np / (SUB_MAX + 1)) + 4;
-  const int maxch = np / BN_CH + np / (SUB_MAX + 1) + 2;
-  PH_HIPCHECK(c, c->bnode.ensure(bn_cap));
-  PH_HIPCHECK(c, c->ch_node.ensure(maxch));
+  // Disjoint sets of particles: the nodes of at most SUB_MAX are at most np,
+  // those of at most MID_MAX np/(SUB_MAX+1), the large ones np/(MID_MAX+1)
+  // per level, and their chunks at most np/BN_CH + one per node.
+  const int mid_cap = np / (SUB_MAX + 1) + 1;
+  const int bn_cap = np / (MID_MAX + 1) + 1;
+  const int maxch = np / BN_CH + bn_cap + 1;
+  PH_HIPCHECK(c, c->small_n.ensure((size_t)np + nb + 2));
+  PH_HIPCHECK(c, c->small_x.ensure((size_t)np + 2));
+  PH_HIPCHECK(c, c->mid_n.ensure((size_t)mid_cap * 2));
+  PH_HIPCHECK(c, c->lev_cnt.ensure((size_t)(MAXLEVELS + 2) * LEV_N));
+  PH_HIPCHECK(c, c->bnode.ensure((size_t)bn_cap * 2));
+  PH_HIPCHECK(c, c->ch_node.ensure((size_t)maxch * 2));
   PH_HIPCHECK(c, c->ch_i.ensure((size_t)maxch * 4));
   PH_HIPCHECK(c, c->ch_off.ensure((size_t)maxch * 2));
   PH_HIPCHECK(c, c->ch_red.ensure((size_t)maxch * BN_RED));
@@ -1179,12 +1558,13 @@ int tree_build(phsph_ctx *c, double *d_xyzh, int ld, int np, const int8_t *d_iph
     quads = c->quads.p;
   }
   int32_t *live = c->tmpi.p;
-  int32_t *bcount = c->frontier_b.p;  // block counts of the compaction
+  int32_t *bcount = c->small_n.p;  // block counts of the compaction
 
   // the reference seeds the bounds with particle 1 before wrapping it
   double x0[3];
   PH_HIPCHECK(c, hipMemcpyAsync(x0, d_xyzh, 3 * sizeof(double), hipMemcpyDeviceToHost, s));
-  int32_t hc[CNT_N] = {0, 0, 0, 0, 1 << 30, 0, 0, 0, 0, 0, 0, 0, 0};
+  int32_t hc[CNT_N] = {};
+  hc[CNT_MINLEVEL] = 1 << 30;
   PH_HIPCHECK(c, dev_set(c, c->counters.p, hc, sizeof(hc)));
   PH_HIPCHECK(c, hipStreamSynchronize(s));
   {
@@ -1207,77 +1587,86 @@ int tree_build(phsph_ctx *c, double *d_xyzh, int ld, int np, const int8_t *d_iph
   double *rootbox = c->dred.p + (size_t)nb * 6;
   hipLaunchKernelGGL(k_root_bounds, dim3(1), dim3(256), 0, s, c->dred.p, (int)nb, x0[0], x0[1], x0[2], rootbox);
   hipLaunchKernelGGL(k_fill_i32, dim3(nblocks(c->nslots, 256)), dim3(256), 0, s, c->leaf_flag.p, c->nslots, 0);
-  int32_t root_init[2] = {0, c->nlive - 1};
-  PH_HIPCHECK(c, dev_set(c, c->nd_lo.p + 1, &root_init[0], sizeof(int32_t)));
-  PH_HIPCHECK(c, dev_set(c, c->nd_hi.p + 1, &root_init[1], sizeof(int32_t)));
-  int32_t one = 1;
-  PH_HIPCHECK(c, dev_set(c, c->frontier_a.p, &one, sizeof(int32_t)));
-  PH_HIPCHECK(c, hipMemcpyAsync(c->fbox_a.p, rootbox, 6 * sizeof(double), hipMemcpyDeviceToDevice, s));
-  const bool dbg = getenv("PHSPH_DEBUG") != nullptr;
-  int nfront = 1;
-  int nbig = (c->nlive > SUB_MAX) ? 1 : 0;  // large nodes in the frontier
+  hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(256), 0, s, c->lev_cnt.p, (int64_t)(MAXLEVELS + 2) * LEV_N, 0);
   int level = 0;
-  int32_t *fa = c->frontier_a.p, *fb = c->frontier_b.p;
-  double *ba = c->fbox_a.p, *bb = c->fbox_b.p;
-  while (nfront > 0) {
-    int32_t zero = 0;
-    PH_HIPCHECK(c, dev_set(c, c->counters.p + CNT_NEXT, &zero, sizeof(int32_t)));
-    static_assert(CNT_SEQMAX == CNT_NBIG + 1, "adjacent level counters");
-    const int32_t zero2[2] = {0, 0};
-    PH_HIPCHECK(c, dev_set(c, c->counters.p + CNT_NBIG, zero2, sizeof(zero2)));
-    if (nbig < nfront) {
-      LaunchTimer lt(c, "tree_subtrees");
-      hipLaunchKernelGGL(k_subtrees, dim3(nfront), dim3(SUB_BS), 0, s, c->dc, fa, ba, nfront, c->tx.p, c->ty.p,
-                         c->tz.p, c->th.p, c->iparts.p, c->nd_lo.p, c->nd_hi.p, c->nd.p, c->leaf_flag.p, level,
-                         c->maxlevel_indexed, c->nslots, c->counters.p);
-    }
-    if (nbig > 0) {
-      if (nfront > bn_cap) PH_RET(c, PHSPH_ERR_STATE, "maketree: large-node frontier beyond its capacity");
-      LaunchTimer lt(c, "tree_bignodes");
-      // chunks <= sum over large nodes of ceil(n/BN_CH) <= nlive/BN_CH + nbig
-      const int gch = std::min(maxch, (c->nlive + BN_CH - 1) / BN_CH + nbig);
-      BigNode *bn = c->bnode.p;
-      int32_t *cnt_d = c->counters.p;
-      const int32_t *chn = c->ch_node.p;
-      hipLaunchKernelGGL(k_bn_plan, dim3(1), dim3(1024), 0, s, fa, ba, nfront, c->nd_lo.p, c->nd_hi.p, bn,
-                         c->ch_node.p, maxch, cnt_d);
-      hipLaunchKernelGGL(k_bn_sums, dim3(gch), dim3(BN_BS), 0, s, c->dc, bn, chn, maxch, cnt_d, c->tx.p, c->ty.p,
+  auto lists = [&](int lv) {  // the lists of nodes whose large ones are of level lv
+    NodeLists L;
+    L.small = c->small_n.p; L.smallx = c->small_x.p;
+    L.mid = c->mid_n.p; L.midx = c->mid_n.p + mid_cap;
+    L.bn = c->bnode.p + (size_t)(lv & 1) * bn_cap;
+    L.ch_node = c->ch_node.p + (size_t)(lv & 1) * maxch;
+    L.lev = c->lev_cnt.p + (size_t)lv * LEV_N;
+    L.bncap = bn_cap; L.maxch = maxch;
+    L.counters = c->counters.p;
+    return L;
+  };
+  hipLaunchKernelGGL(k_tree_seed, dim3(1), dim3(64), 0, s, rootbox, c->nlive, c->nd_lo.p, c->nd_hi.p, lists(0));
+  const bool dbg = getenv("PHSPH_DEBUG") != nullptr;
+  int nmid = (c->nlive > SUB_MAX && c->nlive <= MID_MAX) ? 1 : 0;
+  if (c->nlive > MID_MAX) {
+    LaunchTimer lt(c, "tree_bignodes");
+    int32_t *cnt_d = c->counters.p;
+    while (true) {
+      const NodeLists L = lists(level), Ln = lists(level + 1);
+      BigNode *bn = L.bn;
+      const int32_t *chn = L.ch_node, *lev = L.lev;
+      // at most 2^level large nodes, and chunks of BN_CH with one part chunk a node
+      const int gn = (level < 20) ? std::min(bn_cap, 1 << level) : bn_cap;
+      const int gch = std::min(maxch, c->nlive / BN_CH + gn);
+      hipLaunchKernelGGL(k_bn_sums, dim3(gch), dim3(BN_BS), 0, s, c->dc, bn, chn, bn_cap, maxch, lev, c->tx.p, c->ty.p,
                          c->tz.p, c->th.p, c->ch_red.p);
-      hipLaunchKernelGGL(k_bn_centre, dim3(nfront), dim3(64), 0, s, c->dc, bn, maxch, cnt_d, c->ch_red.p);
-      hipLaunchKernelGGL(k_bn_amb, dim3(gch), dim3(BN_BS), 0, s, bn, chn, maxch, cnt_d, c->tx.p, c->ty.p, c->tz.p,
-                         c->ch_i.p);
-      hipLaunchKernelGGL(k_bn_seq, dim3(nfront), dim3(BN_SEQ_BS), 0, s, c->dc, bn, maxch, cnt_d, c->ch_i.p,
-                         c->tx.p, c->ty.p, c->tz.p);
-      hipLaunchKernelGGL(k_bn_size, dim3(gch), dim3(BN_BS), 0, s, c->dc, bn, chn, maxch, cnt_d, c->tx.p, c->ty.p,
-                         c->tz.p, c->ch_red.p, c->ch_i.p, quads ? 1 : 0);
-      hipLaunchKernelGGL(k_bn_node, dim3(nfront), dim3(64), 0, s, bn, maxch, cnt_d, c->ch_red.p, c->ch_i.p,
-                         c->nd.p, c->leaf_flag.p, level, c->maxlevel_indexed, c->nslots, quads);
-      hipLaunchKernelGGL(k_bn_pcount, dim3(gch), dim3(BN_BS), 0, s, bn, chn, maxch, cnt_d, c->tx.p, c->ty.p,
+      hipLaunchKernelGGL(k_bn_centre, dim3(gn), dim3(64), 0, s, c->dc, bn, bn_cap, maxch, lev, c->ch_red.p);
+      hipLaunchKernelGGL(k_bn_amb, dim3(gch), dim3(BN_BS), 0, s, bn, chn, bn_cap, maxch, lev, c->tx.p, c->ty.p,
                          c->tz.p, c->ch_i.p);
-      hipLaunchKernelGGL(k_bn_pscan, dim3(nfront), dim3(64), 0, s, bn, maxch, cnt_d, c->ch_i.p, c->ch_off.p);
-      hipLaunchKernelGGL(k_bn_pscatter, dim3(gch), dim3(BN_BS), 0, s, bn, chn, maxch, cnt_d, c->tx.p, c->ty.p,
+      hipLaunchKernelGGL(k_bn_seq, dim3(gn), dim3(BN_SEQ_BS), 0, s, c->dc, bn, bn_cap, maxch, lev, cnt_d, c->ch_i.p,
+                         c->tx.p, c->ty.p, c->tz.p);
+      hipLaunchKernelGGL(k_bn_size, dim3(gch), dim3(BN_BS), 0, s, c->dc, bn, chn, bn_cap, maxch, lev, c->tx.p, c->ty.p,
+                         c->tz.p, c->ch_red.p, c->ch_i.p, quads ? 1 : 0);
+      hipLaunchKernelGGL(k_bn_node, dim3(gn), dim3(64), 0, s, bn, bn_cap, maxch, lev, cnt_d, c->ch_red.p, c->ch_i.p,
+                         c->nd.p, c->leaf_flag.p, level, c->maxlevel_indexed, c->nslots, quads);
+      hipLaunchKernelGGL(k_bn_pcount, dim3(gch), dim3(BN_BS), 0, s, bn, chn, bn_cap, maxch, lev, c->tx.p, c->ty.p,
+                         c->tz.p, c->ch_i.p);
+      hipLaunchKernelGGL(k_bn_pscan, dim3(gn), dim3(64), 0, s, bn, bn_cap, maxch, lev, cnt_d, c->ch_i.p, c->ch_off.p);
+      hipLaunchKernelGGL(k_bn_pscatter, dim3(gch), dim3(BN_BS), 0, s, bn, chn, bn_cap, maxch, lev, c->tx.p, c->ty.p,
                          c->tz.p, c->ch_off.p, c->tmpi.p, c->tmpi2.p);
-      hipLaunchKernelGGL(k_bn_swap, dim3(gch), dim3(BN_BS), 0, s, bn, chn, maxch, cnt_d, c->tmpi.p, c->tmpi2.p,
-                         c->tx.p, c->ty.p, c->tz.p, c->th.p, c->iparts.p);
-      hipLaunchKernelGGL(k_bn_box, dim3(gch), dim3(BN_BS), 0, s, bn, chn, maxch, cnt_d, c->tx.p, c->ty.p, c->tz.p,
-                         c->ch_red.p);
-      hipLaunchKernelGGL(k_bn_finish, dim3(nfront), dim3(64), 0, s, bn, maxch, cnt_d, c->ch_red.p, c->nd_lo.p,
-                         c->nd_hi.p, fb, bb);
+      hipLaunchKernelGGL(k_bn_swap, dim3(gch), dim3(BN_BS), 0, s, bn, chn, bn_cap, maxch, lev, c->tmpi.p, c->tmpi2.p,
+                         c->tx.p, c->ty.p, c->tz.p, c->th.p, c->iparts.p, c->ch_red.p);
+      hipLaunchKernelGGL(k_bn_finish, dim3(gn), dim3(64), 0, s, bn, bn_cap, maxch, lev, c->ch_red.p, c->nd_lo.p,
+                         c->nd_hi.p, Ln);
+      PH_HIPCHECK(c, hipGetLastError());
+      level++;
+      // the largest node of a level holds at least nlive / 2^level particles:
+      // while that is a large one there is a next level without asking
+      if (level < 20 && ((int64_t)MID_MAX << level) < (int64_t)c->nlive) continue;
+      int32_t lc[LEV_N];
+      PH_HIPCHECK(c, hipMemcpyAsync(lc, Ln.lev, sizeof(lc), hipMemcpyDeviceToHost, s));
+      PH_HIPCHECK(c, hipMemcpyAsync(cnt, c->counters.p, sizeof(cnt), hipMemcpyDeviceToHost, s));
+      PH_HIPCHECK(c, hipStreamSynchronize(s));
+      nmid = cnt[CNT_NMID];
+      if (cnt[CNT_ERR] || lc[LEV_NBIG] == 0) break;
+      if (level > MAXLEVELS) PH_RET(c, PHSPH_ERR_CAPACITY, "maketree: more than 64 levels");
     }
-    PH_HIPCHECK(c, hipGetLastError());
-    PH_HIPCHECK(c, hipMemcpyAsync(cnt, c->counters.p, sizeof(cnt), hipMemcpyDeviceToHost, s));
-    PH_HIPCHECK(c, hipStreamSynchronize(s));
-    if (dbg)
-      fprintf(stderr, "maketree level %d: frontier %d, large %d, sequential sums so far %d, longest this level %d\n",
-              level, nfront, nbig, cnt[CNT_FALLBACK], cnt[CNT_SEQMAX]);
-    if (cnt[CNT_ERR]) break;
-    nfront = cnt[CNT_NEXT];
-    nbig = cnt[CNT_NBIG];
-    std::swap(fa, fb);
-    std::swap(ba, bb);
-    level++;
-    if (level > 64) PH_RET(c, PHSPH_ERR_CAPACITY, "maketree: more than 64 levels");
   }
+  if (!cnt[CNT_ERR] && nmid > 0) {
+    LaunchTimer lt(c, "tree_midnodes");
+    hipLaunchKernelGGL(k_mid, dim3(std::min(nmid, mid_cap)), dim3(MID_BS), 0, s, c->dc, c->tx.p, c->ty.p, c->tz.p,
+                       c->th.p, c->iparts.p, c->nd_lo.p, c->nd_hi.p, c->nd.p, c->leaf_flag.p, c->maxlevel_indexed,
+                       c->nslots, quads, lists(level + 1));
+  }
+  if (!cnt[CNT_ERR]) {
+    LaunchTimer lt(c, "tree_subtrees");
+    // nodes of at most SUB_MAX particles have 512 to 1024 in an even set
+    const unsigned g = (unsigned)std::min<int64_t>((int64_t)np, 64 + (int64_t)c->nlive / 384);
+    hipLaunchKernelGGL(k_subtrees, dim3(g), dim3(SUB_BS), 0, s, c->dc, c->small_n.p, c->small_x.p, c->tx.p, c->ty.p,
+                       c->tz.p, c->th.p, c->iparts.p, c->nd_lo.p, c->nd_hi.p, c->nd.p, c->leaf_flag.p,
+                       c->maxlevel_indexed, c->nslots, c->counters.p);
+  }
+  PH_HIPCHECK(c, hipGetLastError());
+  PH_HIPCHECK(c, hipMemcpyAsync(cnt, c->counters.p, sizeof(cnt), hipMemcpyDeviceToHost, s));
+  PH_HIPCHECK(c, hipStreamSynchronize(s));
+  if (dbg)
+    fprintf(stderr, "maketree: %d levels of large nodes, %d middle nodes, %d subtrees, %d sums in order, longest %d\n",
+            level, nmid, cnt[CNT_NSMALL], cnt[CNT_FALLBACK], cnt[CNT_SEQMAX]);
   if (cnt[CNT_ERR] & TERR_NODEID)
     PH_RET(c, PHSPH_ERR_CAPACITY,
            "maketree: tree deeper than maxlevel_indexed; pass a larger maxp (ncellsmax = 2*maxp)");
