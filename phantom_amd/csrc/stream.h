@@ -345,6 +345,61 @@ __device__ __forceinline__ void build_list(ListStage<CL> &S, const DevConst &dc,
   }
 }
 
+// The candidates of one particle searched by a whole wavefront: 64 leaves of
+// its group at a time are tested for reach, the particles of those in reach are
+// lined up in LDS and taken 64 at a time, visit(in, j, code, r2, w) in every
+// lane (in: the lane has a particle; w: the fourth word of its record).
+constexpr int SOLO_SLOTS = 64 * PH_MINPART + 64;
+template <class Rec, class Reach, class Visit>
+__device__ __forceinline__ void solo_search(uint32_t *__restrict__ slot, const DevConst &dc,
+                                            const uint32_t *__restrict__ gc, int nc,
+                                            const phsph_kdnode *__restrict__ nd, const int32_t *__restrict__ nd_lo,
+                                            const int32_t *__restrict__ nd_hi, const double *__restrict__ hmaxn,
+                                            const Rec *__restrict__ rec, double xi, double yi, double zi, double lcx,
+                                            double lcy, double lcz, double lsz, Reach reach, Visit visit) {
+  const int lane = threadIdx.x & 63;
+  int fill = 0;  // particles waiting in slot, fewer than 64 between the rounds
+  for (int k0 = 0; k0 < nc; k0 += 64) {
+    int cnt = 0, lo = 0, code = SEP_PLAIN;
+    if (k0 + lane < nc) {
+      const int n = (int)gc[k0 + lane];
+      const double cx = nd[n].xcen[0], cy = nd[n].xcen[1], cz = nd[n].xcen[2], sz = nd[n].size;
+      if (reach(cx, cy, cz, sz, hmaxn ? hmaxn[n] : 0.)) {
+        lo = nd_lo[n];
+        cnt = min(nd_hi[n] - lo + 1, PH_MINPART);
+        code = leaf_sep_code(dc, cx, cy, cz, sz, lcx, lcy, lcz, lsz);
+      }
+    }
+    int incl = cnt;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += v;
+    }
+    uint32_t *const d = slot + fill + incl - cnt;
+#pragma unroll
+    for (int u = 0; u < PH_MINPART; u++)
+      if (u < cnt) d[u] = cand_pack(lo + u, code);
+    const int total = fill + __shfl(incl, 63, 64);
+    const bool last = k0 + 64 >= nc;
+    wave_lds_sync();
+    int s0 = 0;
+    for (; s0 + 64 <= total || (last && s0 < total); s0 += 64) {
+      const bool in = s0 + lane < total;
+      const uint32_t e = slot[in ? s0 + lane : s0];
+      const int j = cand_node(e), cj = cand_code(e);
+      double xj, yj, zj, wj, dx, dy, dz;
+      rec_xyzi(rec, j, xj, yj, zj, wj);
+      sep_of(dc, cj, xi, yi, zi, xj, yj, zj, dx, dy, dz);
+      visit(in, j, cj, r2_exact(dx, dy, dz), wj);
+    }
+    fill = max(total - s0, 0);
+    const uint32_t e = (lane < fill) ? slot[s0 + lane] : 0u;
+    wave_lds_sync();
+    if (lane < fill) slot[lane] = e;
+    wave_lds_sync();
+  }
+}
+
 // the reach test of a lane: |x_i - xcen| (minimum image) against the leaf
 // size plus the lane's search radius, with a margin for rounding
 __device__ __forceinline__ bool leaf_in_reach(const DevConst &dc, double xi, double yi, double zi, double ccx,

@@ -184,3 +184,19 @@ __device__ __forceinline__ int quad_max_i(int v) {
   v = max(v, dpp_quad_i<DPP_XOR1>(v));
   return max(v, dpp_quad_i<DPP_XOR2>(v));
 }
+
+template <int CTRL, class OP>
+__device__ __forceinline__ double dpp_op(double v, OP op) { return op(v, dpp_quad<CTRL>(v)); }
+// a reduction over the wavefront, the result in every lane
+template <class OP>
+__device__ __forceinline__ double wave_all(double v, OP op) {
+  v = dpp_op<DPP_XOR1>(v, op);
+  v = dpp_op<DPP_XOR2>(v, op);
+  v = dpp_op<0x141>(v, op);  // row_half_mirror
+  v = dpp_op<0x140>(v, op);  // row_mirror
+  v = op(v, __shfl_xor(v, 16, 64));
+  return op(v, __shfl_xor(v, 32, 64));
+}
+struct OpAdd { __device__ __forceinline__ double operator()(double a, double b) const { return a + b; } };
+struct OpMin { __device__ __forceinline__ double operator()(double a, double b) const { return fmin(a, b); } };
+struct OpMax { __device__ __forceinline__ double operator()(double a, double b) const { return fmax(a, b); } };

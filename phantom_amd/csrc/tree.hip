@@ -897,22 +897,6 @@ __global__ void k_bn_finish(const BigNode *bn, int bncap, int maxch, const int32
 #define MID_RED 20    // doubles per wavefront: sums, or size, child boxes and second moments
 #define MID_WORDS (MID_MAX / 64 + 2 * MID_Q)
 
-template <int CTRL, class OP>
-__device__ __forceinline__ double dpp_op(double v, OP op) { return op(v, dpp_quad<CTRL>(v)); }
-// a reduction over the wavefront, the result in every lane
-template <class OP>
-__device__ __forceinline__ double wave_all(double v, OP op) {
-  v = dpp_op<DPP_XOR1>(v, op);
-  v = dpp_op<DPP_XOR2>(v, op);
-  v = dpp_op<0x141>(v, op);  // row_half_mirror
-  v = dpp_op<0x140>(v, op);  // row_mirror
-  v = op(v, __shfl_xor(v, 16, 64));
-  return op(v, __shfl_xor(v, 32, 64));
-}
-struct OpAdd { __device__ __forceinline__ double operator()(double a, double b) const { return a + b; } };
-struct OpMin { __device__ __forceinline__ double operator()(double a, double b) const { return fmin(a, b); } };
-struct OpMax { __device__ __forceinline__ double operator()(double a, double b) const { return fmax(a, b); } };
-
 __global__ void __launch_bounds__(MID_BS) k_mid(DevConst dc, double *tx, double *ty, double *tz, double *th,
                                                 int32_t *iparts, int32_t *nd_lo, int32_t *nd_hi, phsph_kdnode *nd,
                                                 int32_t *leaf_flag, int maxlevel_indexed, int64_t nslots,
