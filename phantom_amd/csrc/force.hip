@@ -160,6 +160,51 @@ k_flist(DevConst dc, const int32_t *__restrict__ act, int nact, int ngroups, con
   if (nl > capl) atomicOr(flags, FFL_LIST);
 }
 
+// The same for one particle per wavefront (solo_search): the slowest wavefront
+// is that of one particle, not of the 64 with the most leaves in their reach.
+constexpr int FSOLO_W = 4;  // wavefronts per workgroup
+__global__ void __launch_bounds__(64 * FSOLO_W)
+k_flist_solo(DevConst dc, const int32_t *__restrict__ act, int nact, const int32_t *__restrict__ pleaf,
+             const int32_t *__restrict__ leaves, const uint32_t *__restrict__ gcand,
+             const int32_t *__restrict__ gncand, const int64_t *goff, int capg, const int32_t *__restrict__ nd_lo,
+             const int32_t *__restrict__ nd_hi, const phsph_kdnode *__restrict__ nd, const double *__restrict__ hmaxn,
+             const double4 *__restrict__ fpos, uint32_t *__restrict__ nlist, const int64_t *loff, int ucap,
+             int32_t *__restrict__ t_nl, int32_t *__restrict__ flags) {
+  __shared__ uint32_t slots[FSOLO_W][SOLO_SLOTS];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int t = xcd_block(blockIdx.x, gridDim.x) * FSOLO_W + w;
+  if (t >= nact) return;
+  const int p = act[t];
+  if (p < 0) {  // padding of a partial group
+    if (lane == 0) t_nl[t] = 0;
+    return;
+  }
+  const int c = leaves[pleaf[p]], g = t / GROUP;
+  const double4 ri = fpos[p];
+  const double xi = ri.x, yi = ri.y, zi = ri.z, hi1 = ri.w, hi = 1. / hi1, hi21 = xmul(hi1, hi1);
+  const double R2 = dc.radkern2;
+  const int capl = list_cap_g(loff, g * GROUP, ucap);
+  const unsigned long long lt = lanemask_lt();
+  int nl = 0;
+  solo_search(
+      slots[w], dc, gcand + cand_base(goff, g, capg), gncand[g], nd, nd_lo, nd_hi, hmaxn, fpos, xi, yi, zi,
+      nd[c].xcen[0], nd[c].xcen[1], nd[c].xcen[2], nd[c].size,
+      [&](double ccx, double ccy, double ccz, double csz, double chm) {
+        return leaf_in_reach(dc, xi, yi, zi, ccx, ccy, ccz, csz, dc.radkern * fmax(hi, chm));
+      },
+      [&](bool in, int j, int code, double r2, double hj1) {
+        const bool hit = in && j != p && (xmul(r2, hi21) < R2 || xmul(r2, xmul(hj1, hj1)) < R2);
+        const unsigned long long m = __ballot(hit);
+        const int k = nl + __popcll(m & lt);
+        if (hit && k < capl) nlist[list_at_g(loff, nact, t, k)] = cand_pack(j, code);
+        nl += __popcll(m);
+      });
+  if (lane == 0) {
+    t_nl[t] = nl;
+    if (nl > capl) atomicOr(flags, FFL_LIST);
+  }
+}
+
 // Force, part 2: the pair terms (force.F90:1227-2056) over each particle's
 // list and finish_cell_and_store_results.  One thread per active particle.
 template <int K, bool MHD, bool DUST, bool THERMAL>
@@ -779,6 +824,13 @@ int cons2prim_run(phsph_ctx *c, int np, const double *xyzh, int ldx, const doubl
   return PHSPH_OK;
 }
 
+// Active slots below which the lists are searched by a wavefront per particle:
+// 0.18 ms on a box of 101520 particles (0.45 by groups of 64) and 0.92 ms on a
+// 500k polytrope (3.1, waiting for the groups of its outer layers).  In an even
+// set the groups take less from about half a million on (the density search
+// by groups costs 1.3 ns a particle in a box of 8.4M, by particles 1.8).
+constexpr int FLIST_SOLO_MAX = 1 << 20;
+
 // ------------------------------------------------------------------------
 // Force neighbour lists of the active slots c->act[0..c->nact) into L (list
 // lengths into TNL): a uniform capacity, doubled (and kept) while the lists of
@@ -807,8 +859,14 @@ static int force_lists(phsph_ctx *c, DBuf<uint32_t> &L, DBuf<int32_t> &TNL, cons
   hipLaunchKernelGGL((k_flist<CC, LL>), dim3(list_grid<LL>(ng)), dim3(64 * LL), 0, s, c->dc, c->act.p, nact, ng,   \
                      c->pleaf.p, c->leaves.p, c->gcand.p, c->gncand.p, c->goff_p, c->caps.gcand, c->nd_lo.p,       \
                      c->nd_hi.p, c->nd.p, c->hmaxf.p, c->fpos.p, L.p, loff, ucap, TNL.p, c->counters.p + 3)
+      if (nact < FLIST_SOLO_MAX) {
+        hipLaunchKernelGGL(k_flist_solo, dim3(xcd_grid(nblocks(nact, FSOLO_W))), dim3(64 * FSOLO_W), 0, s, c->dc,
+                           c->act.p, nact, c->pleaf.p, c->leaves.p, c->gcand.p, c->gncand.p, c->goff_p, c->caps.gcand,
+                           c->nd_lo.p, c->nd_hi.p, c->nd.p, c->hmaxf.p, c->fpos.p, L.p, loff, ucap, TNL.p,
+                           c->counters.p + 3);
+      }
       // the chunk length and wavefronts per block the density autotuner chose
-      if (c->tune.cl == 8) { if (c->tune.lw == 2) FLIST(8, 2); else FLIST(8, 4); }
+      else if (c->tune.cl == 8) { if (c->tune.lw == 2) FLIST(8, 2); else FLIST(8, 4); }
       else { if (c->tune.lw == 2) FLIST(16, 2); else FLIST(16, 4); }
 #undef FLIST
     }
