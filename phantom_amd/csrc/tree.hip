@@ -245,8 +245,6 @@ __device__ __forceinline__ int pick_axis(const double *box) {
 #define BN_CH 2048
 #define BN_BS 256
 #define BN_U (BN_CH / BN_BS)
-#define BN_SEQ 1024     // positions per LDS stage of the sequential sums
-#define BN_SEQ_BS 512   // wavefront 0 sums, the others stage
 #define BN_RED 24       // doubles per chunk in ch_red: sums/size/quads, then
 #define BN_BOX 12       // from BN_BOX the two children's bounding boxes
 
@@ -473,99 +471,204 @@ __global__ void __launch_bounds__(BN_BS) k_bn_amb(const BigNode *bn, const int32
   if (threadIdx.x == 0) ch_i[(size_t)c * 4 + 0] = amb;
 }
 
-// cnt additions of one running sum in order, from an LDS row, with the
-// next 16 values loaded while the current 16 are added (two register sets
-// in turn).  Reads up to 15 values past cnt: the rows are BN_SEQ_LD long.
-__device__ __forceinline__ double seq_chain(double acc, const double *src, int cnt) {
-  int k = 0;
-  if (cnt >= 16) {
-    double v[16], w[16];
-#pragma unroll
-    for (int u = 0; u < 16; u++) v[u] = src[u];
-    while (true) {
-#pragma unroll
-      for (int u = 0; u < 16; u++) w[u] = src[k + 16 + u];
-#pragma unroll
-      for (int u = 0; u < 16; u++) acc = xadd(acc, v[u]);
-      k += 16;
-      if (k + 16 > cnt) break;
-#pragma unroll
-      for (int u = 0; u < 16; u++) v[u] = src[k + 16 + u];
-#pragma unroll
-      for (int u = 0; u < 16; u++) acc = xadd(acc, w[u]);
-      k += 16;
-      if (k + 16 > cnt) break;
-    }
+// ------------------------------------------------------------------------
+// Exact sequential sums (kdtree.F90:655-665) without the sequence.  While a
+// running sum s stays inside one binade [2^e, 2^(e+1)) it is a multiple of
+// u = 2^(e-52), and adding a rounds a to a multiple of u whatever s is, except
+// for a tie (a an odd multiple of u/2).  So the sums up to every element are
+// s + u (prefix sums of rint(a/u)), exact in FP64 as long as they stay below
+// 2^53 u.  A workgroup takes SEQ_ST elements at a time, stops at the first that
+// ties or leaves the open binade, adds the next ones there in order, and goes
+// on.  Sums that swing about zero change their binade all the time: the run
+// in order grows while little is gained in between.
+//
+// On the lattice shock tube (1.1M particles) 1.3 ms over all levels; as chains
+// of dependent FP64 additions 5.7 ms (2.8 ns each; the two nodes of level 1 3.1
+// -> 0.48 ms, levels that split along y and z, whose sums swing, 0.6 -> 0.5).
+// ------------------------------------------------------------------------
+#define SEQ_ST 8192
+#define SEQ_BS 1024
+constexpr int SEQ_BUF = SEQ_ST + SEQ_ST / 8 + 32;  // doubles of LDS: rows of eight elements and a word of padding
+constexpr int SEQ_SW = SEQ_BS / 64 + 2;
+__device__ __forceinline__ int seq_at(int k) { return k + (k >> 3); }
+__device__ __forceinline__ int exp_of(double a) { return (int)((__double_as_longlong(a) >> 52) & 0x7ff) - 1023; }
+__device__ __forceinline__ double two_to(int e) { return __longlong_as_double((long long)(1023 + e) << 52); }
+
+// a added n times to zero, in order: within a binade the same rounded
+// increment every time (after a tie the sum is even, and stays so)
+__device__ double seq_mass(int n, double a) {
+  double s = 0.;
+  if (!(a > 1e-250 && a < 1e250)) {
+    for (int k = 0; k < n; k++) s = xadd(s, a);
+    return s;
   }
-  for (; k < cnt; k++) acc = xadd(acc, src[k]);
+  int k = 0;
+  while (k < n) {
+    s = xadd(s, a);
+    k++;
+    const int e = exp_of(s);
+    const double S = s * two_to(52 - e), t = a * two_to(52 - e);
+    if (t >= 2251799813685248.) continue;  // 2^51
+    const double fl = floor(t), fr = t - fl;
+    const long long il = (long long)fl, is = (long long)S;
+    long long m = il + (fr > 0.5 ? 1 : 0);
+    if (fr == 0.5) {
+      if (is & 1) continue;
+      m = il + (il & 1);
+    }
+    if (m == 0) break;
+    const long long c = min((long long)(n - k), ((1ll << 53) - 1 - is) / m);
+    s = (double)(is + c * m) * two_to(e - 52);
+    k += (int)c;
+  }
+  return s;
+}
+
+// additions of buf[seq_at(k)], k = k0 .. k1-1, to acc in order: rows of eight,
+// two rows read ahead (up to three past the last one: SEQ_BUF has room)
+__device__ __forceinline__ double seq_chain(double acc, const double *buf, int k0, int k1) {
+  int k = k0;
+  while (k < k1 && (k & 7)) acc = xadd(acc, buf[seq_at(k++)]);
+  const double *r = buf + seq_at(k);
+  const int nr = (k1 - k) >> 3;
+  auto read = [&](double (&d)[8], int j) {
+#pragma unroll
+    for (int u = 0; u < 8; u++) d[u] = r[9 * j + u];
+  };
+  auto add = [&](const double (&d)[8]) {
+#pragma unroll
+    for (int u = 0; u < 8; u++) acc = xadd(acc, d[u]);
+  };
+  if (nr > 0) {
+    double v[8], w[8], x[8];
+    read(v, 0); read(w, 1); read(x, 2);
+    int j = 0;
+    for (; j + 3 <= nr; j += 3) {
+      add(v); read(v, j + 3);
+      add(w); read(w, j + 4);
+      add(x); read(x, j + 5);
+    }
+    if (j < nr) add(v);
+    if (j + 1 < nr) add(w);
+    k += 8 * nr;
+  }
+  for (; k < k1; k++) acc = xadd(acc, buf[seq_at(k)]);
   return acc;
 }
 
-// Exact sequential sums (kdtree.F90:655-665) of the particles [lo, hi], by a
-// whole workgroup: x, y, z and mass to seq.  The four running sums are four
-// dependent chains in lanes 0-3 of wavefront 0; the other wavefronts stage
-// the products fac*x of the next BN_SEQ positions into LDS meanwhile.  The
-// rows are padded so that the four lanes read distinct LDS banks.
-#define BN_SEQ_LD (BN_SEQ + 20)
-constexpr int BN_SEQ_BUF = 7 * BN_SEQ_LD;  // doubles of LDS: two stages of three rows, and a row of masses
-template <int BS>
-__device__ void seq_sums(double *buf, double *seq, int lo, int hi, double pm, double fac, const double *tx,
-                         const double *ty, const double *tz) {
-  const int tid = threadIdx.x, lane = tid & 63;
-  double *mrow = buf + 6 * BN_SEQ_LD;
-  const int n = hi - lo + 1;
-  const int nst = (n + BN_SEQ - 1) / BN_SEQ;
-  auto fill = [&](int st) {
-    const int base = lo + st * BN_SEQ;
-    const int cnt = min(BN_SEQ, hi - base + 1);
-    double *dst = buf + (st & 1) * 3 * BN_SEQ_LD;
-    for (int k = tid - 64; k < cnt; k += BS - 64) {
-      dst[k] = xmul(fac, tx[base + k]);
-      dst[BN_SEQ_LD + k] = xmul(fac, ty[base + k]);
-      dst[2 * BN_SEQ_LD + k] = xmul(fac, tz[base + k]);
-    }
-  };
-  for (int k = tid; k < BN_SEQ_LD; k += BS) mrow[k] = pm;
-  if (tid >= 64) fill(0);
-  __syncthreads();
-  double acc = 0.;
-  for (int st = 0; st < nst; st++) {
-    if (tid >= 64) {
-      if (st + 1 < nst) fill(st + 1);
-    } else if (lane < 4) {
-      const int cnt = min(BN_SEQ, hi - (lo + st * BN_SEQ) + 1);
-      acc = seq_chain(acc, lane < 3 ? buf + ((st & 1) * 3 + lane) * BN_SEQ_LD : mrow, cnt);
-    }
+// the running sums of fac*ta and of the mass over the particles [lo, hi], by a
+// whole workgroup of SEQ_BS threads (buf: SEQ_BUF, sw: SEQ_SW doubles of LDS)
+__device__ void seq_axis(double *buf, double *sw, int *si, int lo, int hi, double pm, double fac, const double *ta,
+                         double &sum, double &tot) {
+  constexpr int E = SEQ_ST / SEQ_BS, NW = SEQ_BS / 64;
+  static_assert(E == 8, "the padding follows a thread's elements");
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int n = hi - lo + 1, k0 = tid * E;
+  if (tid == 0) sw[NW] = 0.;
+  if (tid == SEQ_BS - 64) sw[NW + 1] = seq_mass(n, pm);
+  int run = 1024;  // length of the next run in order: the first elements double the sum again and again
+  for (int base = 0; base < n; base += SEQ_ST) {
+    const int cnt = min(SEQ_ST, n - base);
     __syncthreads();
+    for (int k = tid; k < cnt; k += SEQ_BS) buf[seq_at(k)] = xmul(fac, ta[lo + base + k]);
+    __syncthreads();
+    int q = 0;
+    while (q < cnt) {
+      const double acc = sw[NW], A = fabs(acc);
+      int first = q;
+      if (A > 1e-250 && A < 1e250) {
+        const int e = exp_of(A);
+        const double scale = copysign(two_to(52 - e), acc), S = A * two_to(52 - e);
+        double m[E], loc = 0.;
+        unsigned stop = 0u;
+#pragma unroll
+        for (int u = 0; u < E; u++) {
+          const int k = k0 + u;
+          const bool use = k >= q && k < cnt;
+          const double t = use ? buf[seq_at(k)] * scale : 0.;
+          const double r = rint(t);
+          const bool ok = fabs(t) < 1125899906842624. && fabs(t - r) != 0.5;  // 2^50
+          m[u] = ok ? r : 0.;
+          stop |= ok ? 0u : 1u << u;
+          loc += m[u];
+        }
+        double v = loc;
+        for (int o = 1; o < 64; o <<= 1) {
+          const double y = __shfl_up(v, o, 64);
+          if (lane >= o) v += y;
+        }
+        if (lane == 63) sw[w] = v;
+        if (tid == 0) *si = cnt;
+        v = __shfl_up(v, 1, 64);  // the sum of the lanes below
+        if (lane == 0) v = 0.;
+        __syncthreads();
+        double s0 = S;
+        for (int i = 0; i < w; i++) s0 += sw[i];
+        s0 += v;
+        double s = s0;
+        int ex = cnt;
+#pragma unroll
+        for (int u = 0; u < E; u++) {
+          const int k = k0 + u;
+          s += m[u];
+          const bool out = (stop >> u & 1u) || !(s > 4503599627370496. && s < 9007199254740992.);  // 2^52, 2^53
+          if (out && k >= q && k < cnt) ex = min(ex, k);
+        }
+        if (ex < cnt) atomicMin(si, ex);
+        __syncthreads();
+        first = *si;
+        if (first > q && first - 1 >= k0 && first - 1 < k0 + E) {
+#pragma unroll
+          for (int u = 0; u < E; u++)
+            if (k0 + u < first) s0 += m[u];
+          sw[NW] = copysign(s0 * two_to(e - 52), acc);
+        }
+      }
+      __syncthreads();
+      if (first > q) run = (first - q < 1024) ? min(4 * run, SEQ_ST) : 64;
+      q = first;
+      if (q < cnt) {
+        const int end = min(cnt, q + run);
+        if (w == 0) {
+          const double a = seq_chain(sw[NW], buf, q, end);
+          if (lane == 0) sw[NW] = a;
+        }
+        q = end;
+        __syncthreads();
+      }
+    }
   }
-  if (tid < 4) seq[tid] = acc;
+  __syncthreads();
+  sum = sw[NW];
+  tot = sw[NW + 1];
   __syncthreads();
 }
 
-// the sequential sums of the nodes with a particle within delta of the plane
-__global__ void __launch_bounds__(BN_SEQ_BS) k_bn_seq(DevConst dc, BigNode *bn, int bncap, int maxch,
-                                                      const int32_t *lev, int32_t *counters, const int32_t *ch_i,
-                                                      const double *tx, const double *ty, const double *tz) {
-  __shared__ double buf[BN_SEQ_BUF];
-  __shared__ double seq[4];
+// The sequential sums of the nodes with a particle within delta of the plane.
+// The split depends on those of the split axis and the mass; the centre's
+// other coordinates stay the parallel sums' (the bound of k_bn_centre).
+__global__ void __launch_bounds__(SEQ_BS) k_bn_seq(DevConst dc, BigNode *bn, int bncap, int maxch, const int32_t *lev,
+                                                   int32_t *counters, const int32_t *ch_i, const double *tx,
+                                                   const double *ty, const double *tz) {
+  __shared__ double buf[SEQ_BUF];
+  __shared__ double sw[SEQ_SW];
+  __shared__ int si;
   const int f = blockIdx.x, tid = threadIdx.x;
   if (!bn_node(lev, bncap, maxch, f)) return;
   const int nchunk = bn[f].nchunk, chunk0 = bn[f].chunk0;
   int amb = 0;
-  for (int k = tid; k < nchunk; k += BN_SEQ_BS) amb |= ch_i[(size_t)(chunk0 + k) * 4 + 0];
+  for (int k = tid; k < nchunk; k += SEQ_BS) amb |= ch_i[(size_t)(chunk0 + k) * 4 + 0];
   amb = __syncthreads_or(amb);
   if (!amb) return;
   const int lo = bn[f].lo, hi = bn[f].hi, iaxis = bn[f].iaxis;
   const double pm = dc.pmass;
   const double dfac = (pm > 0.) ? 1. / pm : 1.;
-  seq_sums<BN_SEQ_BS>(buf, seq, lo, hi, pm, xmul(pm, dfac), tx, ty, tz);
+  double sum, tot;
+  seq_axis(buf, sw, &si, lo, hi, pm, xmul(pm, dfac), axis_arr(iaxis, tx, ty, tz), sum, tot);
   if (tid == 0) {
-    const double tot = seq[3];
-    const double D = xmul(tot, dfac);
     BigNode *b = bn + f;
-    for (int k = 0; k < 3; k++) b->com[k] = seq[k] / D;
+    b->pivot = b->com[iaxis] = sum / xmul(tot, dfac);
     b->tot = tot;
-    b->pivot = b->com[iaxis];
     atomicAdd(&counters[CNT_FALLBACK], 1);
     atomicMax(&counters[CNT_SEQMAX], hi - lo + 1);
   }
@@ -897,15 +1000,18 @@ __global__ void k_bn_finish(const BigNode *bn, int bncap, int maxch, const int32
 #define MID_RED 20    // doubles per wavefront: sums, or size, child boxes and second moments
 #define MID_WORDS (MID_MAX / 64 + 2 * MID_Q)
 
+template <bool QUADS>
 __global__ void __launch_bounds__(MID_BS) k_mid(DevConst dc, double *tx, double *ty, double *tz, double *th,
                                                 int32_t *iparts, int32_t *nd_lo, int32_t *nd_hi, phsph_kdnode *nd,
                                                 int32_t *leaf_flag, int maxlevel_indexed, int64_t nslots,
                                                 double *quads, NodeLists L) {
-  // the stages of the sequential sums, then the pairs of the partition
-  static_assert(BN_SEQ_BUF * 8 >= MID_MAX * 2, "the pairs fit the stages");
-  __shared__ double buf[BN_SEQ_BUF];
+  // the stage of the sequential sums, then the pairs of the partition
+  static_assert(SEQ_BUF * 8 >= MID_MAX * 2, "the pairs fit the stage");
+  static_assert(SEQ_BS == MID_BS, "seq_axis is run by the whole workgroup");
+  __shared__ double buf[SEQ_BUF];
   uint16_t *pairs = reinterpret_cast<uint16_t *>(buf);
-  __shared__ double seq[4];
+  __shared__ double sw[SEQ_SW];
+  __shared__ int si;
   __shared__ double red[MID_W][MID_RED];
   __shared__ int redn[MID_W];                       // particles on the left of the pivot
   __shared__ unsigned long long lew[MID_WORDS];     // bit of each particle: on the left
@@ -913,7 +1019,7 @@ __global__ void __launch_bounds__(MID_BS) k_mid(DevConst dc, double *tx, double 
   // nodes of a level: id, range, split axis; then centre, pivot, mass, split
   __shared__ int qn[2][MID_Q], ql[2][MID_Q], qh[2][MID_Q], qx[2][MID_Q];
   __shared__ int qcount[2];
-  __shared__ double qcom[MID_Q][3], qtot[MID_Q];
+  __shared__ double qpiv[MID_Q], qtot[MID_Q];
   __shared__ int qamb[MID_Q], qnl[MID_Q], qnbad[MID_Q], qcx[MID_Q][2];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   if ((int)blockIdx.x >= L.counters[CNT_NMID]) return;
@@ -982,7 +1088,7 @@ __global__ void __launch_bounds__(MID_BS) k_mid(DevConst dc, double *tx, double 
     while (true) {
       const double piv = (axis == 0) ? c0 : (axis == 1) ? c1 : c2;
       if (todo) {
-        double r2 = 0., bx[12], q[6] = {0., 0., 0., 0., 0., 0.};
+        double r2 = 0., bx[12], q[QUADS ? 6 : 1] = {0.};
         for (int k = 0; k < 3; k++) {
           bx[k] = bx[6 + k] = PH_HUGE64;
           bx[3 + k] = bx[9 + k] = -PH_HUGE64;
@@ -1008,7 +1114,7 @@ __global__ void __launch_bounds__(MID_BS) k_mid(DevConst dc, double *tx, double 
             bx[3] = left ? fmax(bx[3], x) : bx[3];    bx[9] = left ? bx[9] : fmax(bx[9], x);
             bx[4] = left ? fmax(bx[4], y) : bx[4];    bx[10] = left ? bx[10] : fmax(bx[10], y);
             bx[5] = left ? fmax(bx[5], z) : bx[5];    bx[11] = left ? bx[11] : fmax(bx[11], z);
-            if (quads) {
+            if constexpr (QUADS) {
               const double dx = x - c0, dy = y - c1, dz = z - c2;
               q[0] += pm * (dx * dx); q[1] += pm * (dx * dy); q[2] += pm * (dx * dz);
               q[3] += pm * (dy * dy); q[4] += pm * (dy * dz); q[5] += pm * (dz * dz);
@@ -1021,13 +1127,13 @@ __global__ void __launch_bounds__(MID_BS) k_mid(DevConst dc, double *tx, double 
           bx[k] = wave_all(bx[k], OpMin()); bx[6 + k] = wave_all(bx[6 + k], OpMin());
           bx[3 + k] = wave_all(bx[3 + k], OpMax()); bx[9 + k] = wave_all(bx[9 + k], OpMax());
         }
-        if (quads)
+        if constexpr (QUADS)
           for (int k = 0; k < 6; k++) q[k] = wave_all(q[k], OpAdd());
         const bool anyamb = __ballot(amb) != 0ull;
         if (lane == 0) {
           red[w][0] = r2;
           for (int k = 0; k < 12; k++) red[w][1 + k] = bx[k];
-          if (quads)
+          if constexpr (QUADS)
             for (int k = 0; k < 6; k++) red[w][13 + k] = q[k];
           redn[w] = cl;
           if (!exact && anyamb) qamb[t] = 1;
@@ -1039,11 +1145,12 @@ __global__ void __launch_bounds__(MID_BS) k_mid(DevConst dc, double *tx, double 
       for (int i = 0; i < nq; i++) {
         if (qamb[i] != 1) continue;
         any = true;
-        seq_sums<MID_BS>(buf, seq, lo0 + ql[cur][i], lo0 + qh[cur][i], pm, fac, tx, ty, tz);
+        double sum, mass;
+        seq_axis(buf, sw, &si, lo0 + ql[cur][i], lo0 + qh[cur][i], pm, fac, axis_arr(qx[cur][i], tx, ty, tz), sum,
+                 mass);
         if (tid == 0) {
-          const double D = xmul(seq[3], dfac);
-          for (int k = 0; k < 3; k++) qcom[i][k] = seq[k] / D;
-          qtot[i] = seq[3];
+          qpiv[i] = sum / xmul(mass, dfac);
+          qtot[i] = mass;
           atomicAdd(&L.counters[CNT_FALLBACK], 1);
           atomicMax(&L.counters[CNT_SEQMAX], qh[cur][i] - ql[cur][i] + 1);
         }
@@ -1052,7 +1159,9 @@ __global__ void __launch_bounds__(MID_BS) k_mid(DevConst dc, double *tx, double 
       if (!any) break;
       todo = on && qamb[t] == 1;
       if (todo) {
-        c0 = qcom[t][0]; c1 = qcom[t][1]; c2 = qcom[t][2];
+        c0 = (axis == 0) ? qpiv[t] : c0;
+        c1 = (axis == 1) ? qpiv[t] : c1;
+        c2 = (axis == 2) ? qpiv[t] : c2;
         tot = qtot[t];
         exact = true;
       }
@@ -1075,7 +1184,7 @@ __global__ void __launch_bounds__(MID_BS) k_mid(DevConst dc, double *tx, double 
           bx[3 + k] = fmax(bx[3 + k], red[i][4 + k]); bx[9 + k] = fmax(bx[9 + k], red[i][10 + k]);
         }
       }
-      if (quads && lane < 6) {
+      if (QUADS && lane < 6) {
         double q = 0.;
         for (int i = w0; i < w0 + Lw; i++) q += red[i][13 + lane];
         quads[6 * (size_t)nnode + lane] = q;
@@ -1602,7 +1711,7 @@ int tree_build(phsph_ctx *c, double *d_xyzh, int ld, int np, const int8_t *d_iph
       hipLaunchKernelGGL(k_bn_centre, dim3(gn), dim3(64), 0, s, c->dc, bn, bn_cap, maxch, lev, c->ch_red.p);
       hipLaunchKernelGGL(k_bn_amb, dim3(gch), dim3(BN_BS), 0, s, bn, chn, bn_cap, maxch, lev, c->tx.p, c->ty.p,
                          c->tz.p, c->ch_i.p);
-      hipLaunchKernelGGL(k_bn_seq, dim3(gn), dim3(BN_SEQ_BS), 0, s, c->dc, bn, bn_cap, maxch, lev, cnt_d, c->ch_i.p,
+      hipLaunchKernelGGL(k_bn_seq, dim3(gn), dim3(SEQ_BS), 0, s, c->dc, bn, bn_cap, maxch, lev, cnt_d, c->ch_i.p,
                          c->tx.p, c->ty.p, c->tz.p);
       hipLaunchKernelGGL(k_bn_size, dim3(gch), dim3(BN_BS), 0, s, c->dc, bn, chn, bn_cap, maxch, lev, c->tx.p, c->ty.p,
                          c->tz.p, c->ch_red.p, c->ch_i.p, quads ? 1 : 0);
@@ -1633,9 +1742,12 @@ int tree_build(phsph_ctx *c, double *d_xyzh, int ld, int np, const int8_t *d_iph
   }
   if (!cnt[CNT_ERR] && nmid > 0) {
     LaunchTimer lt(c, "tree_midnodes");
-    hipLaunchKernelGGL(k_mid, dim3(std::min(nmid, mid_cap)), dim3(MID_BS), 0, s, c->dc, c->tx.p, c->ty.p, c->tz.p,
-                       c->th.p, c->iparts.p, c->nd_lo.p, c->nd_hi.p, c->nd.p, c->leaf_flag.p, c->maxlevel_indexed,
-                       c->nslots, quads, lists(level + 1));
+#define MID(QQ)                                                                                                   \
+  hipLaunchKernelGGL((k_mid<QQ>), dim3(std::min(nmid, mid_cap)), dim3(MID_BS), 0, s, c->dc, c->tx.p, c->ty.p, c->tz.p, \
+                     c->th.p, c->iparts.p, c->nd_lo.p, c->nd_hi.p, c->nd.p, c->leaf_flag.p, c->maxlevel_indexed,       \
+                     c->nslots, quads, lists(level + 1))
+    if (quads) MID(true); else MID(false);
+#undef MID
   }
   if (!cnt[CNT_ERR]) {
     LaunchTimer lt(c, "tree_subtrees");
