@@ -4,9 +4,6 @@
 // pair loop with softened and point-mass gravity (force.F90:1286-2053,
 // 2909-2927).
 //
-//  * k_quads: second moments of every node about its centre of mass
-//    (kdtree.F90:724-750), one wavefront per node of at most TREE_SUB_MAX
-//    particles (the tree build forms those of larger nodes chunk by chunk).
 //  * k_hmax_replay: the reference raises a leaf's hmax (and its ancestors')
 //    whenever a density iteration relists the cell (set_hmaxcell,
 //    neigh_kdtree.f90:115-131; dens.F90:338-373).  The density kernel keeps
@@ -32,38 +29,6 @@ constexpr int GSTACK = 2048;    // (source, level) stack of the dual walk (LDS)
 constexpr int GW_MASKS = 64;    // candidates whose first-pass result is kept: 64 * GW_MASKS
 
 enum { GFL_STACK = 1, GFL_DEPTH = 2, GFL_P2P = 4, GFL_TRAJ = 8, GFL_CAND = 16, GFL_DTC = 32, GFL_NEAR = 64 };
-
-// ids 2n, 2n+1 are the children of n: a slot is a node when every ancestor
-// is an internal node (leaf_flag == 0)
-__device__ __forceinline__ bool node_valid(int n, const int32_t *__restrict__ leaf_flag) {
-  while (n > 1) {
-    n >>= 1;
-    if (leaf_flag[n] != 0) return false;
-  }
-  return true;
-}
-
-// ------------------------------------------------------------------------
-__global__ void __launch_bounds__(64)
-k_quads(DevConst dc, int64_t ncells, const phsph_kdnode *__restrict__ nd, const int32_t *__restrict__ nd_lo,
-        const int32_t *__restrict__ nd_hi, const int32_t *__restrict__ leaf_flag, const double *__restrict__ tx,
-        const double *__restrict__ ty, const double *__restrict__ tz, double *__restrict__ quads) {
-  const int64_t n = (int64_t)blockIdx.x + 1;
-  if (n > ncells || !node_valid((int)n, leaf_flag)) return;
-  if (nd_hi[n] - nd_lo[n] + 1 > TREE_SUB_MAX) return;  // formed by the tree build's large-node phase
-  const int lane = threadIdx.x;
-  const double c0 = nd[n].xcen[0], c1 = nd[n].xcen[1], c2 = nd[n].xcen[2];
-  const double pm = dc.pmass;
-  double q[6] = {0., 0., 0., 0., 0., 0.};
-  for (int p = nd_lo[n] + lane; p <= nd_hi[n]; p += 64) {
-    const double dx = tx[p] - c0, dy = ty[p] - c1, dz = tz[p] - c2;
-    q[0] += pm * (dx * dx); q[1] += pm * (dx * dy); q[2] += pm * (dx * dz);
-    q[3] += pm * (dy * dy); q[4] += pm * (dy * dz); q[5] += pm * (dz * dz);
-  }
-  for (int k = 0; k < 6; k++) q[k] = wave_sum(q[k]);
-  if (lane == 0)
-    for (int k = 0; k < 6; k++) quads[6 * n + k] = q[k];
-}
 
 __global__ void k_init_ghmax(int64_t nslots, const phsph_kdnode *__restrict__ nd,
                              unsigned long long *__restrict__ ghmax) {
@@ -904,11 +869,6 @@ int grav_tree(phsph_ctx *c) {
   if (c->nslots > ((int64_t)1 << 26)) PH_RET(c, PHSPH_ERR_CAPACITY, "maketree: too many tree nodes for self-gravity");
   PH_HIPCHECK(c, c->quads.ensure((size_t)c->nslots * 6));
   PH_HIPCHECK(c, c->ghmax.ensure((size_t)c->nslots));
-  if (c->ncells > 0) {
-    LaunchTimer lt(c, "tree_quads");
-    hipLaunchKernelGGL(k_quads, dim3((unsigned)c->ncells), dim3(64), 0, s, c->dc, c->ncells, c->nd.p, c->nd_lo.p,
-                       c->nd_hi.p, c->leaf_flag.p, c->tx.p, c->ty.p, c->tz.p, c->quads.p);
-  }
   hipLaunchKernelGGL(k_init_ghmax, dim3(nblocks(c->nslots, 256)), dim3(256), 0, s, (int64_t)c->nslots, c->nd.p,
                      c->ghmax.p);
   PH_HIPCHECK(c, hipGetLastError());

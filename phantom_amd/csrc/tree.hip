@@ -1357,11 +1357,12 @@ __device__ __forceinline__ double sub_chain(const double *row, int a0, int a1, b
   return acc;
 }
 
+template <bool QUADS>
 __global__ void __launch_bounds__(SUB_BS) k_subtrees(DevConst dc, const int32_t *small, const int32_t *smallx,
                                                      double *tx, double *ty, double *tz, double *th,
                                                      int32_t *iparts, int32_t *nd_lo, int32_t *nd_hi,
                                                      phsph_kdnode *nd, int32_t *leaf_flag, int maxlevel_indexed,
-                                                     int64_t nslots, int32_t *counters) {
+                                                     int64_t nslots, double *quads, int32_t *counters) {
   __shared__ double srow[4][SUB_ROW];  // x, y, z, h
   __shared__ int32_t sip[SUB_MAX];
   __shared__ int32_t sidx[SUB_MAX];  // partition pairs
@@ -1422,12 +1423,17 @@ __global__ void __launch_bounds__(SUB_BS) k_subtrees(DevConst dc, const int32_t 
         const int iaxis = qx[cur][t];
         const double pivot = (iaxis == 0) ? com0 : (iaxis == 1) ? com1 : com2;
         const double *sa = srow[iaxis];
-        double hmax = 0., r2max = 0.;
+        double hmax = 0., r2max = 0., qd[QUADS ? 6 : 1] = {0.};
         int act = 0, cl = 0;
   #pragma unroll 4
         for (int k = a0 + sub; k <= a1; k += L) {
           const int q = sub_at(k);
-          const double r2 = r2_exact(xsub(sx[q], com0), xsub(sy[q], com1), xsub(sz[q], com2));
+          const double dx = xsub(sx[q], com0), dy = xsub(sy[q], com1), dz = xsub(sz[q], com2);
+          const double r2 = r2_exact(dx, dy, dz);
+          if constexpr (QUADS) {
+            qd[0] += pm * (dx * dx); qd[1] += pm * (dx * dy); qd[2] += pm * (dx * dz);
+            qd[3] += pm * (dy * dy); qd[4] += pm * (dy * dz); qd[5] += pm * (dz * dz);
+          }
           r2max = (r2 > r2max) ? r2 : r2max;
           hmax = (shh[q] > hmax) ? shh[q] : hmax;
           act |= sip[k] > 0;
@@ -1438,6 +1444,8 @@ __global__ void __launch_bounds__(SUB_BS) k_subtrees(DevConst dc, const int32_t 
           hmax = fmax(hmax, __shfl_xor(hmax, o, 64));
           act |= __shfl_xor(act, o, 64);
           cl += __shfl_xor(cl, o, 64);
+          if constexpr (QUADS)
+            for (int i = 0; i < 6; i++) qd[i] += __shfl_xor(qd[i], o, 64);
         }
         const bool isleaf = npn <= PH_MINPART;
         const int il = 2 * nnode, ir = il + 1;
@@ -1453,6 +1461,8 @@ __global__ void __launch_bounds__(SUB_BS) k_subtrees(DevConst dc, const int32_t 
           e.parent = nnode / 2;
           e.idum = 0;
           nd[nnode] = e;
+          if constexpr (QUADS)
+            for (int i = 0; i < 6; i++) quads[6 * (size_t)nnode + i] = qd[i];
           nd_lo[nnode] = lo + a0;
           nd_hi[nnode] = lo + a1;
           leaf_flag[nnode] = isleaf ? ((dc.ind_timesteps && !act) ? -1 : 1) : 0;
@@ -1644,7 +1654,8 @@ int tree_build(phsph_ctx *c, double *d_xyzh, int ld, int np, const int8_t *d_iph
   PH_HIPCHECK(c, c->ch_i.ensure((size_t)maxch * 4));
   PH_HIPCHECK(c, c->ch_off.ensure((size_t)maxch * 2));
   PH_HIPCHECK(c, c->ch_red.ensure((size_t)maxch * BN_RED));
-  // under self-gravity the large nodes' second moments are formed here
+  // under self-gravity the nodes' second moments about their centres of mass
+  // (kdtree.F90:724-750) are formed here
   double *quads = nullptr;
   if (c->p.gravity) {
     PH_HIPCHECK(c, c->quads.ensure((size_t)c->nslots * 6));
@@ -1742,10 +1753,10 @@ int tree_build(phsph_ctx *c, double *d_xyzh, int ld, int np, const int8_t *d_iph
   }
   if (!cnt[CNT_ERR] && nmid > 0) {
     LaunchTimer lt(c, "tree_midnodes");
-#define MID(QQ)                                                                                                   \
-  hipLaunchKernelGGL((k_mid<QQ>), dim3(std::min(nmid, mid_cap)), dim3(MID_BS), 0, s, c->dc, c->tx.p, c->ty.p, c->tz.p, \
-                     c->th.p, c->iparts.p, c->nd_lo.p, c->nd_hi.p, c->nd.p, c->leaf_flag.p, c->maxlevel_indexed,       \
-                     c->nslots, quads, lists(level + 1))
+#define MID(QQ)                                                                                                     \
+  hipLaunchKernelGGL((k_mid<QQ>), dim3(std::min(nmid, mid_cap)), dim3(MID_BS), 0, s, c->dc, c->tx.p, c->ty.p,         \
+                     c->tz.p, c->th.p, c->iparts.p, c->nd_lo.p, c->nd_hi.p, c->nd.p, c->leaf_flag.p,                  \
+                     c->maxlevel_indexed, c->nslots, quads, lists(level + 1))
     if (quads) MID(true); else MID(false);
 #undef MID
   }
@@ -1753,9 +1764,12 @@ int tree_build(phsph_ctx *c, double *d_xyzh, int ld, int np, const int8_t *d_iph
     LaunchTimer lt(c, "tree_subtrees");
     // nodes of at most SUB_MAX particles have 512 to 1024 in an even set
     const unsigned g = (unsigned)std::min<int64_t>((int64_t)np, 64 + (int64_t)c->nlive / 384);
-    hipLaunchKernelGGL(k_subtrees, dim3(g), dim3(SUB_BS), 0, s, c->dc, c->small_n.p, c->small_x.p, c->tx.p, c->ty.p,
-                       c->tz.p, c->th.p, c->iparts.p, c->nd_lo.p, c->nd_hi.p, c->nd.p, c->leaf_flag.p,
-                       c->maxlevel_indexed, c->nslots, c->counters.p);
+#define SUBT(QQ)                                                                                                    \
+  hipLaunchKernelGGL((k_subtrees<QQ>), dim3(g), dim3(SUB_BS), 0, s, c->dc, c->small_n.p, c->small_x.p, c->tx.p,       \
+                     c->ty.p, c->tz.p, c->th.p, c->iparts.p, c->nd_lo.p, c->nd_hi.p, c->nd.p, c->leaf_flag.p,         \
+                     c->maxlevel_indexed, c->nslots, quads, c->counters.p)
+    if (quads) SUBT(true); else SUBT(false);
+#undef SUBT
   }
   PH_HIPCHECK(c, hipGetLastError());
   PH_HIPCHECK(c, hipMemcpyAsync(cnt, c->counters.p, sizeof(cnt), hipMemcpyDeviceToHost, s));
