@@ -7,7 +7,12 @@
 //  * k_group_walk: one wavefront per group of 64 active particles walks the
 //    tree breadth-parallel (64 nodes per step) and lists the candidate leaves
 //    of the whole group (stream.h).
-//  * k_dens_iter: one wavefront per group, one particle per lane.  Each lane
+//  * Dense active sets: k_dens_tile and k_dens_sums (dens_tile.hip,
+//    dens_sums.hip).
+//  * Sparse ones, and the particles that tiles hand back: k_dens_solo, one
+//    particle per wavefront, then k_dens_final.
+//  * k_dens_iter: dense sets that cannot run by tile (and the autotuner): one
+//    wavefront per group, one particle per lane.  Each lane
 //    visits the candidate leaves its particle can reach (build_list),
 //    keeps the particles within rfac*radkern*h of its own particle in a
 //    neighbour list, then runs its own Newton-Raphson

@@ -8,11 +8,12 @@
 // stress, Borve div B source subtraction, artificial resistivity, psi
 // cleaning) and one-fluid dust (sqrt(eps/(1-eps)) evolution, Delta v).
 //
-// k_flist (one wavefront per group of 64 active particles, one particle per
-// lane) collects each particle's symmetric neighbour set
+// k_flist_solo and k_flist (one particle per wavefront, or one per lane of a
+// group of 64) collect each particle's symmetric neighbour set
 // {j : q_i < R or q_j < R} (force.F90:1287) from the group's candidate leaves
 // with the same separately rounded FP64 tests as the reference; k_force (one
-// thread per particle) evaluates the pair terms over that list.  Quantities
+// thread per particle) evaluates the pair terms over that list, k_force_tile
+// (force_tile.hip) over the lists of the density tiles.  Quantities
 // of particle j that the reference recomputes per pair (rho_j, P/rho^2, wave
 // speed, MHD stress, stopping time) are evaluated once per particle by
 // k_force_prep with the same arithmetic and packed into one 128-byte record
