@@ -21,6 +21,9 @@
 //     particles: with |x_j|^2 stored, three FMA and a compare.  The list may
 //     hold more than the search sphere (the sums and the later passes make
 //     their own exact tests), so FP32 with a margin above its rounding does.
+//     Lengths there are in units of the group's search radius, so that no
+//     square leaves the FP32 range whatever the unit of length; a group whose
+//     box or neighbours' radii are 1e15 times its own goes to the list kernels.
 //     Hits are packed into the particle's list in candidate order.
 //  3. FP64 distances into registers, list to memory, Newton iterations.
 //
@@ -49,7 +52,7 @@ k_dens_tile(DevConst dc, int icall, double rfac, double lmargin, const int32_t *
   constexpr int W = TileCap<K, V>::W, NC = TileCap<K, V>::NC, LC = TileCap<K, V>::LC, NE = BIG ? 1 : LC / TILE_L;
   constexpr int LEAVES = 64 * W;  // leaves staged at a time
   __shared__ double cx[NC], cy[NC], cz[NC];  // position with the offset
-  __shared__ float cr2[NC];                  // (list radius of j)^2, rounded up
+  __shared__ float cr2[NC];                  // (list radius of j)^2 in units of the group's, rounded up
   __shared__ uint32_t cj[NC];                // tree position and offset code
   __shared__ float4 bxs[W][64];              // candidates under test: x, y, z about the centre and their square
   __shared__ uint2 brs[W][64];               // their cr2 and slot
@@ -74,7 +77,8 @@ k_dens_tile(DevConst dc, int icall, double rfac, double lmargin, const int32_t *
   const double ex = 0.5 * (gb[3] - gb[0]) * (1. + 1e-12) + 1e-300, ey = 0.5 * (gb[4] - gb[1]) * (1. + 1e-12) + 1e-300,
                ez = 0.5 * (gb[5] - gb[2]) * (1. + 1e-12) + 1e-300;
   const double rl = rfac * lmargin * dc.radkern;
-  const double rg2 = (rl * gb[6]) * (rl * gb[6]);
+  const double rg = rl * gb[6], rg2 = rg * rg;
+  const double sc = 1. / rg, sc2 = sc * sc;  // to units of the group's search radius
   const uint32_t *gc = gcand + cand_base(goff, g, capg);
   const int nleaf = gncand[g];
   const int pfirst = act[t0], plast = act[t1 - 1];
@@ -114,10 +118,15 @@ k_dens_tile(DevConst dc, int icall, double rfac, double lmargin, const int32_t *
           const double4 v = tp[j];
           x = v.x; y = v.y; z = v.z;
           offset_pos(dc, code, x, y, z);
-          if (hmax0) rj2 = (float)((rl * v.w) * (rl * v.w) * (1. + 1.2e-7));
+          double rd2 = rg2;
+          if (hmax0) {
+            const double d2 = (rl * v.w) * (rl * v.w);
+            rj2 = (float)(d2 * sc2 * (1. + 1.2e-7));
+            rd2 = fmax(rd2, d2);
+          }
           const double qx = fmax(fabs(x - bx) - ex, 0.), qy = fmax(fabs(y - by) - ey, 0.),
                        qz = fmax(fabs(z - bz) - ez, 0.);
-          in = qx * qx + qy * qy + qz * qz < fmax(rg2, (double)rj2) * (1. + 1e-9);
+          in = qx * qx + qy * qy + qz * qz < rd2 * (1. + 1e-9);
           jc = cand_pack(j, code);
         }
       }
@@ -151,6 +160,8 @@ k_dens_tile(DevConst dc, int icall, double rfac, double lmargin, const int32_t *
     const double need = (rl * hmx + 3. * smax) * (1. + 1e-9);
     bad = bad || ex + need >= dc.hdlx || ey + need >= dc.hdly || ez + need >= dc.hdlz;
   }
+  // squares of the scaled lengths stay far inside the FP32 range
+  bad = bad || !((ex + ey + ez + rl * hmx) * sc < 1e15);
   if (bad && !BIG && nc > NC && tid == 0) tl.big[atomicAdd(tl.nbig, 1)] = g;  // the large form next
   uint32_t *gcl = BIG ? tl.bcand + (size_t)b * tl.bncap : tl.cand + (size_t)g * tl.ncap;
   uint16_t *gll = BIG ? tl.blist + (size_t)b * TILE_BW * tl.blc * TILE_P : tl.list + (size_t)g * tl.lw * tl.lc * TILE_P;
@@ -187,15 +198,15 @@ k_dens_tile(DevConst dc, int icall, double rfac, double lmargin, const int32_t *
       hw = fmax(hw, __shfl_xor(hw, o, 64));
     }
     const double wx = 0.5 * (xl + xh), wy = 0.5 * (yl + yh), wz = 0.5 * (zl + zh);
-    const float fx = (float)(0.5 * (xh - xl)) * 1.000001f, fy = (float)(0.5 * (yh - yl)) * 1.000001f,
-                fz = (float)(0.5 * (zh - zl)) * 1.000001f;
-    const float rw2 = (float)((rl * hw) * (rl * hw)) * 1.00001f;
+    const float fx = (float)(0.5 * (xh - xl) * sc) * 1.000001f, fy = (float)(0.5 * (yh - yl) * sc) * 1.000001f,
+                fz = (float)(0.5 * (zh - zl) * sc) * 1.000001f;
+    const float rw2 = (float)((rl * hw * sc) * (rl * hw * sc)) * 1.00001f;
     // particle i about the centre; the margin covers the FP32 rounding of the
     // separation (a few 2^-24 of (|x_i| + |x_j|)^2, |x_j| <= |x_i| + radius)
-    const float xf = (float)(xi - wx), yf = (float)(yi - wy), zf = (float)(zi - wz);
+    const float xf = (float)((xi - wx) * sc), yf = (float)((yi - wy) * sc), zf = (float)((zi - wz) * sc);
     const float di2 = xf * xf + yf * yf + zf * zf;
-    const float far = 2.f * sqrtf(di2) + (float)(rl * hmx);
-    const float rc2 = (float)((rl * h0) * (rl * h0)) * 1.000001f;
+    const float far = 2.f * sqrtf(di2) + (float)(rl * hmx * sc);
+    const float rc2 = (float)((rl * h0 * sc) * (rl * h0 * sc)) * 1.000001f;
     const float ui = di2 - 2e-6f * far * far;
     const float mx = -2.f * xf, my = -2.f * yf, mz = -2.f * zf;
     uint16_t(*L)[TILE_P] = U.list[w];
@@ -207,11 +218,11 @@ k_dens_tile(DevConst dc, int icall, double rfac, double lmargin, const int32_t *
       bool in = false;
       float x = 0.f, y = 0.f, z = 0.f, rj2 = 0.f;
       if (s < nc) {
-        x = (float)(cx[s] - wx); y = (float)(cy[s] - wy); z = (float)(cz[s] - wz);
+        x = (float)((cx[s] - wx) * sc); y = (float)((cy[s] - wy) * sc); z = (float)((cz[s] - wz) * sc);
         rj2 = cr2[s];
         const float qx = fmaxf(fabsf(x) - fx, 0.f), qy = fmaxf(fabsf(y) - fy, 0.f), qz = fmaxf(fabsf(z) - fz, 0.f);
         const float a2 = fabsf(x) + fabsf(y) + fabsf(z);
-        in = qx * qx + qy * qy + qz * qz - 2e-6f * a2 * a2 < fmaxf(rw2, rj2);
+        in = qx * qx + qy * qy + qz * qz - 2e-6f * a2 * a2 <= fmaxf(rw2, rj2);
       }
       const unsigned long long m = __ballot(in);
       const int ns = __popcll(m);
