@@ -109,7 +109,8 @@ static inline unsigned tile_grid(int ngroups, const TileLists &tl) { return xcd_
 // estimate: one coupled Newton step for the root and its half reciprocal, the
 // residual of the root, and one step for the reciprocal (each to about one unit
 // in the last place; zero and denormal squares give about 1e-145, far below
-// any h)
+// any h).  From 1/r that step leaves (eps/r)^2, so below 1e8 eps it starts from
+// an estimate of 1/(r + eps).
 __device__ __forceinline__ void sqrt_rsqrt_sep(double r2, double eps, double &r, double &r1) {
   const double a = fmax(r2, 1e-290);
   const double y = __builtin_amdgcn_rsq(a);
@@ -120,7 +121,12 @@ __device__ __forceinline__ void sqrt_rsqrt_sep(double r2, double eps, double &r,
   const double d = fma(-g, g, a);
   r = fma(d, h, g);
   h = h + h;
-  const double e1 = fma(-(r + eps), h, 1.);
+  const double b = r + eps;
+  if (eps > 0. && r < 1e8 * eps) {
+    h = __builtin_amdgcn_rcp(b);
+    h = fma(h, fma(-b, h, 1.), h);
+  }
+  const double e1 = fma(-b, h, 1.);
   r1 = fma(h, e1, h);
 }
 
