@@ -123,6 +123,7 @@ struct phsph_ctx {
   DBuf<int32_t> tl_nc, tl_bnc;
   DBuf<double2> t_sums;      // sums of the last h iteration per active slot
   int ntg = 0, tg_max = 0;   // tile groups, particles of the largest
+  int walk_unfit = 0;        // tile groups of the last walk that are no tiles
   DBuf<int32_t> pleaf;       // tree position -> index into leaves
   DBuf<int32_t> iparts;      // inodeparts: signed 1-based original index
   DBuf<double> tx, ty, tz, th;  // treecache x, y, z, h (tree order)

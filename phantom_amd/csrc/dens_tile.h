@@ -5,7 +5,8 @@
 
 enum { DFL_CAND = 1, DFL_LIST = 2, DFL_REWALK = 4, DFL_NOCONV = 8, DFL_NEGH = 16, DFL_STACK = 32, DFL_TILE = 64,
        DFL_STACK_LO = 128 };
-constexpr int CNT_REWALK = 8;  // c->counters: particles that outgrew their lists (tiles)
+// c->counters: particles that outgrew their lists (tiles), and groups that are no tiles (tile_unfit)
+constexpr int CNT_REWALK = 8, CNT_UNFIT = 9;
 
 struct DensIn {
   const double4 *tp;  // x, y, z (treecache) and h at entry

@@ -39,7 +39,7 @@
 // the leaf sizes: a pair for which the two choices differ is then out of reach
 // (and its separation under either is beyond the search radius), and no
 // separation in reach needs a further minimum-image step.  Groups in boxes too
-// small for that go to the list kernels.
+// small for that go to the list kernels (all of a set of which most are: dens_run).
 template <int K, int V>
 __global__ void __launch_bounds__((64 * TileCap<K, V>::W)) __attribute__((amdgpu_waves_per_eu(TileCap<K, V>::WPE)))
 k_dens_tile(DevConst dc, int icall, double rfac, double lmargin, const int32_t *__restrict__ act, int ngroups,
@@ -156,12 +156,7 @@ k_dens_tile(DevConst dc, int icall, double rfac, double lmargin, const int32_t *
   if (lane == 0) { wred[w][0] = smax; wred[w][1] = hmx; }
   __syncthreads();
   for (int k = 0; k < W; k++) { smax = fmax(smax, wred[k][0]); hmx = fmax(hmx, wred[k][1]); }
-  if (dc.periodic) {
-    const double need = (rl * hmx + 3. * smax) * (1. + 1e-9);
-    bad = bad || ex + need >= dc.hdlx || ey + need >= dc.hdly || ez + need >= dc.hdlz;
-  }
-  // squares of the scaled lengths stay far inside the FP32 range
-  bad = bad || !((ex + ey + ez + rl * hmx) * sc < 1e15);
+  bad = bad || tile_unfit(dc, ex, ey, ez, rl, gb[6], hmx, smax);
   if (bad && !BIG && nc > NC && tid == 0) tl.big[atomicAdd(tl.nbig, 1)] = g;  // the large form next
   uint32_t *gcl = BIG ? tl.bcand + (size_t)b * tl.bncap : tl.cand + (size_t)g * tl.ncap;
   uint16_t *gll = BIG ? tl.blist + (size_t)b * TILE_BW * tl.blc * TILE_P : tl.list + (size_t)g * tl.lw * tl.lc * TILE_P;

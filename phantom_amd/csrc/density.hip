@@ -163,6 +163,7 @@ k_group_walk(DevConst dc, int mode, double rfac, const phsph_kdnode *__restrict_
   if (lane == 0) stk[0] = 1;
   int top = 1, nc = 0;
   bool ovf = false;
+  double smax = 0., hmx = hm;  // of the candidates (tiles)
   __syncthreads();
   while (top > 0) {
     const int take = min(top, 64);
@@ -172,8 +173,10 @@ k_group_walk(DevConst dc, int mode, double rfac, const phsph_kdnode *__restrict_
     top -= take;
     bool open = false, isleaf = false;
     int lc = 0, rc = 0;
+    double size = 0.;
     if (node > 0) {
       const phsph_kdnode e = nd[node];
+      size = e.size;
       double dx = e.xcen[0] - bx, dy = e.xcen[1] - by, dz = e.xcen[2] - bz;
       if (dc.periodic) {
         if (fabs(dx) > dc.hdlx) dx -= copysign(dc.dxbound, dx);
@@ -194,6 +197,8 @@ k_group_walk(DevConst dc, int mode, double rfac, const phsph_kdnode *__restrict_
     if (open && isleaf) {
       const int k = nc + __popcll(ml & lanemask_lt());
       if (k < gcap) gcand[gbase + k] = (uint32_t)node;
+      smax = fmax(smax, size);
+      if (hmaxn) hmx = fmax(hmx, hmaxn[node]);
     }
     nc += __popcll(ml);
     const bool push = open && !isleaf;
@@ -210,6 +215,11 @@ k_group_walk(DevConst dc, int mode, double rfac, const phsph_kdnode *__restrict_
     }
     top += npush;
     __syncthreads();
+  }
+  if (gt && !ovf) {
+    smax = wave_max(smax);
+    hmx = wave_max(hmx);
+    if (lane == 0 && tile_unfit(dc, ex, ey, ez, rfac * dc.radkern, hm, hmx, smax)) atomicAdd(&flags[CNT_UNFIT], 1);
   }
   if (lane == 0) {
     gncand[g] = ovf ? -1 : nc;
@@ -1144,8 +1154,9 @@ int walk_groups(phsph_ctx *c, int mode, double rfac, const double *d_hsrc, const
     if (!exact) PH_HIPCHECK(c, c->gcand.ensure((size_t)(ng + 1) * c->caps.gcand));
     PH_HIPCHECK(c, c->gncand.ensure(ng + 1));
     PH_HIPCHECK(c, c->gbox.ensure((size_t)(ng + 1) * GBOX));
-    int32_t zero = 0;
-    PH_HIPCHECK(c, dev_set(c, c->counters.p, &zero, sizeof(int32_t)));
+    int32_t cnt[CNT_UNFIT + 1] = {};
+    const size_t ncnt = sizeof(int32_t) * (tiles ? CNT_UNFIT + 1 : 1);
+    PH_HIPCHECK(c, dev_set(c, c->counters.p, cnt, ncnt));
 #define WALK(SS)                                                                                                \
   hipLaunchKernelGGL((k_group_walk<SS>), dim3(xcd_grid(ng)), dim3(64), 0, s, c->dc, mode, rfac, c->nd.p, d_hmaxn, \
                      c->leaf_flag.p, c->act.p, c->nact, tiles ? c->tg_t.p : nullptr, c->tx.p, c->ty.p, c->tz.p,   \
@@ -1155,17 +1166,18 @@ int walk_groups(phsph_ctx *c, int mode, double rfac, const double *d_hsrc, const
       WALK(WALK_STACK_LO);
     }
     PH_HIPCHECK(c, hipGetLastError());
-    int32_t fl = 0;
-    PH_HIPCHECK(c, hipMemcpyAsync(&fl, c->counters.p, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+    PH_HIPCHECK(c, hipMemcpyAsync(cnt, c->counters.p, ncnt, hipMemcpyDeviceToHost, s));
     PH_HIPCHECK(c, hipStreamSynchronize(s));
-    if (fl & DFL_STACK_LO) {
+    if (cnt[0] & DFL_STACK_LO) {
       LaunchTimer lt(c, mode == 0 ? "walk_density" : "walk_force");
       WALK(WALK_STACK);
       PH_HIPCHECK(c, hipGetLastError());
-      PH_HIPCHECK(c, hipMemcpyAsync(&fl, c->counters.p, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+      PH_HIPCHECK(c, hipMemcpyAsync(cnt, c->counters.p, ncnt, hipMemcpyDeviceToHost, s));
       PH_HIPCHECK(c, hipStreamSynchronize(s));
     }
 #undef WALK
+    const int32_t fl = cnt[0];
+    c->walk_unfit = cnt[CNT_UNFIT];
     if (getenv("PHSPH_DEBUG")) {
       size_t fr = 0, tot = 0;
       (void)hipMemGetInfo(&fr, &tot);
@@ -1471,13 +1483,20 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
   // lanes visit only the leaves in their own reach; from half of the
   // particles active on the tile is the faster one.  Not with a list capacity
   // below a tile's own.
-  const bool tile = 2 * (int64_t)nact >= n && c->caps.dlist >= dens_tile_list_cap(c);
-  const bool tile_tune = tile && c->tune_mode == TUNE_PENDING && nact >= TUNE_MIN_ACTIVE;
+  bool tile = 2 * (int64_t)nact >= n && c->caps.dlist >= dens_tile_list_cap(c);
   if (tile) {
     PH_HIPCHECK(c, c->tg_t.ensure((size_t)c->ntg + 1));
     hipLaunchKernelGGL(k_tile_ranges, dim3(nblocks((size_t)c->ntg + 1, 256)), dim3(256), 0, s, c->ntg, c->tg_lo.p,
                        c->act.p, nact, c->tg_t.p);
+    rc = walk_groups(c, 0, rfac * lmargin, c->th_in.p, reusable ? c->hmax0.p : nullptr, true);
+    if (rc) return rc;
+    // A periodic box with few particles along a side has no or few groups that
+    // are tiles (tile_unfit): the lists of all particles then, which also serve
+    // the force pass.  Box of 256 x 256 x 12, cubic kernel: 5.6 ms, as
+    // particles handed back by tiles 7.3.
+    tile = 2 * (int64_t)c->walk_unfit <= c->ntg;
   }
+  const bool tile_tune = tile && c->tune_mode == TUNE_PENDING && nact >= TUNE_MIN_ACTIVE;
   if (!tile || tile_tune) {
     rc = pad_groups(c);
     if (rc) return rc;
@@ -1538,11 +1557,12 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
       hipLaunchKernelGGL(k_zero_i32, dim3(nblocks(c->nleaves, 256)), dim3(256), 0, s, c->leaf_nits.p, c->nleaves, 0);
     }
     if (by_tile) {
-      rc = walk_groups(c, 0, rfac * lmargin, c->th_in.p, widen ? c->hmax0.p : nullptr, true);
-      if (rc) return rc;
+      if (tile_tune) {  // the tuner walked other groups
+        rc = walk_groups(c, 0, rfac * lmargin, c->th_in.p, widen ? c->hmax0.p : nullptr, true);
+        if (rc) return rc;
+      }
       hipLaunchKernelGGL(k_zero_i32, dim3(nblocks(n, 256)), dim3(256), 0, s, c->tmpi.p, n, 0);
       PH_HIPCHECK(c, dev_set(c, c->counters.p, &zero, sizeof(int32_t)));
-      PH_HIPCHECK(c, dev_set(c, c->counters.p + CNT_REWALK, &zero, sizeof(int32_t)));
       rc = tile_lists(c, tl);
       if (rc) return rc;
       PH_HIPCHECK(c, dev_set(c, tl.nbig, &zero, sizeof(int32_t)));

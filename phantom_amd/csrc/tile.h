@@ -54,6 +54,20 @@ __device__ __forceinline__ void offset_pos(const DevConst &dc, int code, double 
   if (sz) z = xadd(z, copysign(dc.dzbound, (double)sz));
 }
 
+// A group whose box (half extents e) is too large beside the periodic box for
+// one offset per leaf (dens_tile.hip), or beside its own search radius for FP32
+// squares: rl is the search radius in units of h, hm the group's largest h, hmx
+// that of its candidates too, smax the largest of their leaves' sizes.
+__device__ __forceinline__ bool tile_unfit(const DevConst &dc, double ex, double ey, double ez, double rl, double hm,
+                                           double hmx, double smax) {
+  bool bad = !(ex + ey + ez + rl * hmx < 1e15 * (rl * hm));
+  if (dc.periodic) {
+    const double need = (rl * hmx + 3. * smax) * (1. + 1e-9);
+    bad = bad || ex + need >= dc.hdlx || ey + need >= dc.hdly || ez + need >= dc.hdlz;
+  }
+  return bad;
+}
+
 // The lists that the density tile kernel leaves for the sums and for the force
 // pass: the candidates of each group (tree position and offset code) and, per
 // 16 particles (one wavefront), the entries of their lists as 16-bit slots of

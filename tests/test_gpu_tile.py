@@ -68,3 +68,21 @@ def test_tiles_match_oracle(name, gpu):
     if setup.get("bins") is not None:
         np.testing.assert_array_equal(g["force"]["ibin"], o["force"]["ibin"])
     g["ctx"].close()
+
+
+@pytest.mark.parametrize("kernel", [abi.KERNEL_CUBIC, abi.KERNEL_QUINTIC])
+def test_thin_box_keeps_its_lists(kernel, gpu):
+    """A periodic box with 12 particles along z, too thin for any tile: the
+    density pass makes lists of all particles, and the force pass uses them
+    (no list of its own, none for particles run again)."""
+    setup = setups.uniform_box(nx=40, ny=40, nz=12, seed=9, kernel=kernel, box=(-0.5, 0.5, -0.5, 0.5, -0.15, 0.15))
+    g = parity.run_gpu(setup)
+    kernels = [nm for nm, _ in g["ctx"].timings()]
+    g["ctx"].close()
+    assert "force" in kernels and not any(k.startswith("force_list") for k in kernels), kernels
+    o = parity.run_oracle(setup)
+    np.testing.assert_array_equal(g["nneigh"], o["dens"]["nneigh"])
+    np.testing.assert_array_equal(g["nits"], o["dens"]["nits"])
+    assert parity.rel_rms(g["xyzh"][:, 3], o["xyzh"][:, 3]) <= 1e-12
+    for c in range(3):
+        assert parity.rel_rms(g["force"]["fxyzu"][:, c], o["force"]["fxyzu"][:, c]) <= 1e-12, c
