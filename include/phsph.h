@@ -548,6 +548,19 @@ int phsph_get_particle_stats(phsph_ctx *ctx, int32_t np, int32_t *nneigh,
 int phsph_get_force_stats(phsph_ctx *ctx, int64_t *npairs);
 
 /*
+ * How the last densityiterate searched (no counterpart in the reference):
+ * `tiles` tree nodes searched by one workgroup each with their candidates in
+ * LDS (0: neighbour lists of all active particles), `large` of them in the
+ * form that has the LDS of a whole CU, `again` active particles run again by
+ * lists (with the padding of their groups), and `deep` tree walks since then
+ * of which some group needed the full node stack.  `force_tiles`: nodes whose
+ * tiles the last force call took its neighbours from (0: lists).  Any pointer
+ * may be null.
+ */
+int phsph_get_search_stats(phsph_ctx *ctx, int32_t *tiles, int32_t *large,
+                           int32_t *again, int32_t *deep, int32_t *force_tiles);
+
+/*
  * Adjoints with respect to positions.  Phantom has no adjoint: these are
  * the vector-Jacobian products of its forward sums, for gradient-based
  * uses of the hot path (relaxation of initial conditions to a target

@@ -206,7 +206,8 @@ int phsph_create(const phsph_params *p, int32_t device, phsph_ctx **out) {
   c->dc = make_devconst(*p);
   // initial list capacities and the list budget (KiB) may be set from the
   // environment, e.g. PHSPH_CAPS="gcand=64,dlist=32,flist=32,p2p=16,gnear=8,budget_kib=1":
-  // larger values avoid second search passes, smaller ones exercise them
+  // larger values avoid second search passes, smaller ones exercise them;
+  // "lists=1" has the list kernels search dense active sets too
   if (const char *env = getenv("PHSPH_CAPS")) {
     std::string spec(env);
     size_t pos = 0;
@@ -225,6 +226,7 @@ int phsph_create(const phsph_params *p, int32_t device, phsph_ctx **out) {
           else if (key == "p2p") c->caps.p2p = v;
           else if (key == "gnear") c->caps.gnear = v;
           else if (key == "budget_kib") c->list_budget = (size_t)v << 10;
+          else if (key == "lists") c->lists_only = true;
         }
       }
       pos = end + 1;
@@ -971,6 +973,21 @@ int phsph_get_particle_stats(phsph_ctx *c, int32_t np, int32_t *nneigh, int32_t 
 int phsph_get_force_stats(phsph_ctx *c, int64_t *npairs) {
   if (!c) return PHSPH_ERR_INPUT;
   if (npairs) *npairs = c->force_npairs;
+  return PHSPH_OK;
+}
+
+int phsph_get_search_stats(phsph_ctx *c, int32_t *tiles, int32_t *large, int32_t *again, int32_t *deep,
+                           int32_t *force_tiles) {
+  if (!c) return PHSPH_ERR_INPUT;
+  if (tiles) *tiles = c->stat_tiles;
+  if (again) *again = c->stat_again;
+  if (deep) *deep = c->stat_deep;
+  if (force_tiles) *force_tiles = c->stat_force_tiles;
+  if (large) {
+    *large = 0;
+    if (c->stat_tiles > 0)
+      PH_HIPCHECK(c, hipMemcpy(large, c->tg_big.p + c->stat_tiles, sizeof(int32_t), hipMemcpyDeviceToHost));
+  }
   return PHSPH_OK;
 }
 

@@ -123,7 +123,10 @@ struct phsph_ctx {
   DBuf<int32_t> tl_nc, tl_bnc;
   DBuf<double2> t_sums;      // sums of the last h iteration per active slot
   int ntg = 0, tg_max = 0;   // tile groups, particles of the largest
+  bool lists_only = false;   // no tiles (PHSPH_CAPS, for tests of the list kernels)
   int walk_unfit = 0;        // tile groups of the last walk that are no tiles
+  // phsph_get_search_stats
+  int stat_tiles = 0, stat_again = 0, stat_deep = 0, stat_force_tiles = 0;
   DBuf<int32_t> pleaf;       // tree position -> index into leaves
   DBuf<int32_t> iparts;      // inodeparts: signed 1-based original index
   DBuf<double> tx, ty, tz, th;  // treecache x, y, z, h (tree order)

@@ -1169,6 +1169,7 @@ int walk_groups(phsph_ctx *c, int mode, double rfac, const double *d_hsrc, const
     PH_HIPCHECK(c, hipMemcpyAsync(cnt, c->counters.p, ncnt, hipMemcpyDeviceToHost, s));
     PH_HIPCHECK(c, hipStreamSynchronize(s));
     if (cnt[0] & DFL_STACK_LO) {
+      c->stat_deep++;
       LaunchTimer lt(c, mode == 0 ? "walk_density" : "walk_force");
       WALK(WALK_STACK);
       PH_HIPCHECK(c, hipGetLastError());
@@ -1400,6 +1401,20 @@ __global__ void k_tile_ranges(int ntg, const int32_t *__restrict__ tg_lo, const 
   tg_t[g] = a;
 }
 
+// Active sets dense enough for tiles.  A tile's time is that of its candidates,
+// nearly the same whatever part of its particles is active (the candidates span
+// the same region), while the list kernels' grows with the active particles.
+// One substep by tiles and by lists, ms: groups of up to 64 particles, 128^3
+// box at 1/2 active 7.2 and 8.9 (cubic), 10.5 and 12.6 (quintic), 108^3 (38 a
+// group) 6.1 and 7.0, 8.7 and 9.1.  Groups of up to 80 leave a CU fewer
+// wavefronts and cost half as much again: cubic, 160^3 box at 1/2 20.4 and
+// 17.9, at 3/4 21.0 and 21.3, 1.1M tube at 1/2 6.8 and 7.0; quintic, 160^3 at
+// 3/4 33.6 and 30.2, at 1 33.3 and 33.7, tube at 0.7 11.9 and 11.7.
+static bool tile_dense(const phsph_ctx *c, int nact, int n) {
+  if (c->tg_max <= 4 * TILE_P) return 2 * (int64_t)nact >= n;
+  return 8 * (int64_t)nact >= (c->p.kernel == PHSPH_KERNEL_CUBIC ? 5 : 7) * (int64_t)n;
+}
+
 int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
   hipStream_t s = c->stream;
   const int n = c->nlive;
@@ -1448,6 +1463,7 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
   hipLaunchKernelGGL(k_zero_i32, dim3(nblocks(n, 256)), dim3(256), 0, s, c->p_nits.p, n, -1);
   hipLaunchKernelGGL(k_zero_i32, dim3(nblocks(n, 256)), dim3(256), 0, s, c->p_nneigh.p, n, -1);
   const bool dbg = getenv("PHSPH_DEBUG") != nullptr;
+  c->stat_deep = 0;
   // Particles whose h outgrows their neighbour list, or whose list does not
   // fit, are handed back and run again (alone) with a wider search or a
   // longer list.  The first search radius (units of radkern*h at entry) is
@@ -1477,13 +1493,9 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
   // while the lists of every active particle fit in the list budget
   // 12 bytes per entry: the entry and its squared separation
   while (c->caps.dlist > 16 && !list_fits(c, (size_t)list_cap(c->caps.dlist) * nact * 3)) c->caps.dlist /= 2;
-  // Dense active sets are searched by tiles (dens_tile.hip).  Every particle
-  // of the region that 64 active particles span is a candidate, so the tests
-  // grow with the inverse of the active fraction, while the list kernel's
-  // lanes visit only the leaves in their own reach; from half of the
-  // particles active on the tile is the faster one.  Not with a list capacity
-  // below a tile's own.
-  bool tile = 2 * (int64_t)nact >= n && c->caps.dlist >= dens_tile_list_cap(c);
+  // Dense active sets are searched by tiles (dens_tile.hip), if the list
+  // capacity is not below a tile's own.
+  bool tile = !c->lists_only && tile_dense(c, nact, n) && c->caps.dlist >= dens_tile_list_cap(c);
   if (tile) {
     PH_HIPCHECK(c, c->tg_t.ensure((size_t)c->ntg + 1));
     hipLaunchKernelGGL(k_tile_ranges, dim3(nblocks((size_t)c->ntg + 1, 256)), dim3(256), 0, s, c->ntg, c->tg_lo.p,
@@ -1502,6 +1514,8 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
     if (rc) return rc;
   }
   c->dlist_tile = tile;
+  c->stat_tiles = tile ? c->ntg : 0;
+  c->stat_again = 0;
   int dlist = c->caps.dlist;
   const int dlist0 = dlist;
   bool tuned_now = false, retune = false;
@@ -1632,7 +1646,7 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
     rc = compact_active(c, c->tmpi.p, n);
     if (rc) return rc;
     if (attempt == 0) {
-      c->dlist_nretry = c->nact;
+      c->dlist_nretry = c->stat_again = c->nact;
       nrewalk = by_tile ? cnt[CNT_REWALK] : c->nact;
     }
     rc = pad_groups(c);

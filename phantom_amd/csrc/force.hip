@@ -1011,6 +1011,7 @@ int force_run(phsph_ctx *c, int icall, const ForceIOArgs &a, double *dtc_out, do
   }
   if (reuse && c->nact != c->dlist_nact) reuse = false;
   c->force_reused_lists = reuse;
+  c->stat_force_tiles = (reuse && c->dlist_tile) ? c->ntg : 0;
   // node hmax of the final smoothing lengths for the h_j search radius
   const bool need_lists = !reuse || c->dlist_nretry > 0;
   if (need_lists) {

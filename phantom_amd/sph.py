@@ -37,7 +37,7 @@ EXPORTED = [
     "phsph_get_quads", "phsph_init_step", "phsph_step_predictor", "phsph_substep_sph", "phsph_step_predict_sph",
     "phsph_step_corrector", "phsph_step_reset", "phsph_get_precision", "phsph_density_vjp", "phsph_force_vjp",
     "phsph_step_vjp", "phsph_step_corrector_noalloc", "phsph_get_tree_grav", "phsph_set_tuning",
-    "phsph_get_tuning", "phsph_step_graph",
+    "phsph_get_tuning", "phsph_step_graph", "phsph_get_search_stats",
 ]
 
 _lib = None
@@ -76,6 +76,7 @@ def load_library(path=LIB_PATH):
     L.phsph_get_neighbour_stats.argtypes = [vp, P(dbl), P(dbl), P(i32), P(i32), P(i64), P(i64)]
     L.phsph_get_particle_stats.argtypes = [vp, i32, vp, vp]
     L.phsph_get_force_stats.argtypes = [vp, P(i64)]
+    L.phsph_get_search_stats.argtypes = [vp] + [P(i32)] * 5
     L.phsph_get_precision.argtypes = [vp, P(i32), P(i32)]
     L.phsph_density_vjp.argtypes = [vp, i32, vp, i32, vp, vp, vp, i32]
     L.phsph_force_vjp.argtypes = [vp, i32, vp, i32, vp, i32, vp, i32, vp, i32, vp, i32]
@@ -563,6 +564,15 @@ class Context:
         n = C.c_int64()
         self._check(self.lib.phsph_get_force_stats(self._h, C.byref(n)))
         return dict(npairs=n.value)
+
+    def get_search_stats(self):
+        """How the last densityiterate and force calls searched: tree nodes
+        searched as tiles (0: by lists), those in the large form, particles
+        run again, walks with the full stack, nodes whose tiles the force
+        used."""
+        v = [C.c_int32() for _ in range(5)]
+        self._check(self.lib.phsph_get_search_stats(self._h, *[C.byref(x) for x in v]))
+        return dict(zip(("tiles", "large", "again", "deep", "force_tiles"), (x.value for x in v)))
 
     def timings(self):
         """Kernel times (ms) of the last call, measured with HIP events."""

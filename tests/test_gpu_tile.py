@@ -41,10 +41,8 @@ CASES = {
 }
 
 
-@pytest.mark.parametrize("name", list(CASES))
-def test_tiles_match_oracle(name, gpu):
-    setup = CASES[name]()
-    print(f"\n[case {name}] n={setup['xyzh'].shape[0]}", flush=True)
+def check(setup):
+    """The setup on the GPU against the oracle; how the GPU searched."""
     g = parity.run_gpu(setup)
     o = parity.run_oracle(setup)
     act = setup["iphase"] > 0 if setup.get("iphase") is not None else np.ones(len(setup["xyzh"]), bool)
@@ -67,7 +65,16 @@ def test_tiles_match_oracle(name, gpu):
         assert parity.rel_rms(g["force"]["ddustevol"], o["force"]["ddustevol"]) <= 1e-12
     if setup.get("bins") is not None:
         np.testing.assert_array_equal(g["force"]["ibin"], o["force"]["ibin"])
+    st = g["ctx"].get_search_stats()
     g["ctx"].close()
+    return st
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_tiles_match_oracle(name, gpu):
+    setup = CASES[name]()
+    print(f"\n[case {name}] n={setup['xyzh'].shape[0]}", flush=True)
+    check(setup)
 
 
 @pytest.mark.parametrize("kernel", [abi.KERNEL_CUBIC, abi.KERNEL_QUINTIC])
@@ -86,3 +93,25 @@ def test_thin_box_keeps_its_lists(kernel, gpu):
     assert parity.rel_rms(g["xyzh"][:, 3], o["xyzh"][:, 3]) <= 1e-12
     for c in range(3):
         assert parity.rel_rms(g["force"]["fxyzu"][:, c], o["force"]["fxyzu"][:, c]) <= 1e-12, c
+
+
+def _open_levels(frac, kernel, nx, ny, nz):
+    s = setups.uniform_box(nx=nx, ny=ny, nz=nz, seed=3, kernel=kernel, isothermal=False,
+                           box=(-0.025 * nx, 0.025 * nx, -0.025 * ny, 0.025 * ny, -0.025 * nz, 0.025 * nz))
+    s["params"].periodic = 0
+    return s if frac == 1.0 else setups.with_levels(s, [(0, 1.0 - frac), (2, frac)], nbinmax=2, istepfrac=1)
+
+
+# 5760 particles: groups of up to 64; 4284: of up to 80
+DISPATCH = [(0.45, abi.KERNEL_CUBIC, (18, 16, 20), False), (0.55, abi.KERNEL_CUBIC, (18, 16, 20), True),
+            (0.55, abi.KERNEL_QUINTIC, (18, 16, 20), True), (0.55, abi.KERNEL_CUBIC, (17, 18, 14), False),
+            (0.7, abi.KERNEL_CUBIC, (17, 18, 14), True), (0.8, abi.KERNEL_QUINTIC, (17, 18, 14), False),
+            (0.95, abi.KERNEL_QUINTIC, (17, 18, 14), True), (1.0, abi.KERNEL_CUBIC, (17, 18, 14), True),
+            (1.0, abi.KERNEL_QUINTIC, (17, 18, 14), True)]
+
+
+@pytest.mark.parametrize("frac,kernel,n,tiles", DISPATCH)
+def test_active_fraction_and_kernel_choose_the_search(frac, kernel, n, tiles, gpu):
+    print(f"\n[case {frac} {kernel} {n}]", flush=True)
+    st = check(_open_levels(frac, kernel, *n))
+    assert (st["tiles"] > 0) == tiles, st
