@@ -1052,11 +1052,8 @@ void launch_dens_solo(const IterLaunch &L) {
 // is kept for the context.  Every configuration visits the same leaves in
 // the same order and writes the same lists and sums, so the outputs of the
 // last run are those of any other.
+// L.r2b has room for the configurations that store the separations.
 int tune_density_iter(phsph_ctx *c, const IterLaunch &L) {
-  // the separations buffer is needed by the configurations that store them
-  PH_HIPCHECK(c, c->nr2.ensure((size_t)list_cap(L.dlist) * L.na + 2));
-  IterLaunch L2 = L;
-  L2.r2b = c->nr2.p;
   hipEvent_t e0, e1;
   PH_HIPCHECK(c, hipEventCreate(&e0));
   PH_HIPCHECK(c, hipEventCreate(&e1));
@@ -1069,7 +1066,7 @@ int tune_density_iter(phsph_ctx *c, const IterLaunch &L) {
         for (int q : {0, 1}) {
         const ListTune t{cl, lw, r2, q};
         PH_HIPCHECK(c, hipEventRecord(e0, L.s));
-        launch_dens_iter(t, L2);
+        launch_dens_iter(t, L);
         PH_HIPCHECK(c, hipEventRecord(e1, L.s));
         PH_HIPCHECK(c, hipEventSynchronize(e1));
         float ms = 0.f;
@@ -1401,6 +1398,56 @@ __global__ void k_tile_ranges(int ntg, const int32_t *__restrict__ tg_lo, const 
   tg_t[g] = a;
 }
 
+// segments of 64 active particles, evenly spread over the active list
+__global__ void k_sample_act(int nseg, int nact, const int32_t *__restrict__ from, int32_t *__restrict__ act) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= nseg * GROUP) return;
+  act[t] = from[(int64_t)(t / GROUP) * (nact / GROUP) / nseg * GROUP + t % GROUP];
+}
+
+// The autotuner of a set that tiles search: its configurations are for the
+// particles that tiles hand back and for large force lists, so a sample of the
+// groups does, with lists that are freed again.  All groups of 8.4M particles
+// took 200 ms and left 12.9 GB with the context; the sample takes 11 ms.
+constexpr int TUNE_SAMPLE = 1 << 18;
+static int tune_beside_tiles(phsph_ctx *c, int icall, double rfac, double lmargin, bool widen, bool &overflow) {
+  hipStream_t s = c->stream;
+  const int nact = c->nact_dens, nseg = std::min(nact, TUNE_SAMPLE) / GROUP;
+  c->nact = nseg * GROUP;
+  hipLaunchKernelGGL(k_sample_act, dim3(nblocks(c->nact, 256)), dim3(256), 0, s, nseg, nact, c->act_dens.p, c->act.p);
+  int rc = pad_groups(c);
+  if (rc) return rc;
+  const int na = c->nact;
+  int dlist = c->caps.dlist;
+  while (dlist > 16 && !list_fits(c, (size_t)list_cap(dlist) * na * 3)) dlist /= 2;
+  DBuf<uint32_t> lb;
+  DBuf<double> r2b;
+  PH_HIPCHECK(c, lb.ensure((size_t)list_cap(dlist) * na + 1));
+  PH_HIPCHECK(c, r2b.ensure((size_t)list_cap(dlist) * na + 2));
+  PH_HIPCHECK(c, c->t_nl_r.ensure((size_t)na + 1));
+  PH_HIPCHECK(c, c->t_hsum_r.ensure((size_t)na + 1));
+  PH_HIPCHECK(c, c->t_hfin_r.ensure((size_t)na + 1));
+  if (widen) PH_HIPCHECK(c, c->t_nlj.ensure((size_t)na + 1));
+  rc = walk_groups(c, 0, rfac * lmargin, c->th_in.p, widen ? c->hmax0.p : nullptr);
+  if (rc) return rc;
+  hipLaunchKernelGGL(k_zero_i32, dim3(nblocks(c->nlive, 256)), dim3(256), 0, s, c->tmpi.p, c->nlive, 0);
+  int32_t fl = 0;
+  PH_HIPCHECK(c, dev_set(c, c->counters.p, &fl, sizeof(int32_t)));
+  rc = tune_density_iter(c, IterLaunch{c, s, c->ngroups, icall, rfac, na, lmargin, dlist, widen, lb.p, r2b.p,
+                                       c->t_nl_r.p, c->t_hsum_r.p, c->t_hfin_r.p});
+  if (rc) return rc;
+  PH_HIPCHECK(c, hipMemcpyAsync(&fl, c->counters.p, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+  // the tiles start from the active list and clean counts
+  PH_HIPCHECK(c, c->act.ensure((size_t)nact + 1));
+  PH_HIPCHECK(c, hipMemcpyAsync(c->act.p, c->act_dens.p, sizeof(int32_t) * nact, hipMemcpyDeviceToDevice, s));
+  hipLaunchKernelGGL(k_zero_i32, dim3(nblocks(c->nleaves, 256)), dim3(256), 0, s, c->leaf_nits.p, c->nleaves, 0);
+  hipLaunchKernelGGL(k_zero_i32, dim3(nblocks(c->nlive, 256)), dim3(256), 0, s, c->p_nits.p, c->nlive, -1);
+  PH_HIPCHECK(c, hipStreamSynchronize(s));
+  c->nact = nact;
+  overflow = (fl & DFL_LIST) != 0;
+  return PHSPH_OK;
+}
+
 // Active sets dense enough for tiles.  A tile's time is that of its candidates,
 // nearly the same whatever part of its particles is active (the candidates span
 // the same region), while the list kernels' grows with the active particles.
@@ -1508,8 +1555,7 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
     // particles handed back by tiles 7.3.
     tile = 2 * (int64_t)c->walk_unfit <= c->ntg;
   }
-  const bool tile_tune = tile && c->tune_mode == TUNE_PENDING && nact >= TUNE_MIN_ACTIVE;
-  if (!tile || tile_tune) {
+  if (!tile) {
     rc = pad_groups(c);
     if (rc) return rc;
   }
@@ -1519,10 +1565,16 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
   int dlist = c->caps.dlist;
   const int dlist0 = dlist;
   bool tuned_now = false, retune = false;
+  if (tile && c->tune_mode == TUNE_PENDING && nact >= TUNE_MIN_ACTIVE) {
+    rc = tune_beside_tiles(c, icall, rfac, lmargin, reusable, retune);
+    if (rc) return rc;
+    rc = walk_groups(c, 0, rfac * lmargin, c->th_in.p, reusable ? c->hmax0.p : nullptr, true);
+    if (rc) return rc;
+  }
   TileLists tl{};
   int nrewalk = 0;  // particles of the first attempt that outgrew their lists
   for (int attempt = 0; attempt < 12; attempt++) {
-    int na = c->nact;  // active slots, padding included
+    const int na = c->nact;  // active slots, padding included
     if (na == 0) break;
     // the first attempt writes the lists the force pass may use; retries
     // write buffers of their own so that those stay intact
@@ -1531,23 +1583,24 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
     DBuf<double> &THS = attempt == 0 ? c->t_hsum : c->t_hsum_r;
     DBuf<double> &THF = attempt == 0 ? c->t_hfin : c->t_hfin_r;
     PH_HIPCHECK(c, TNL.ensure((size_t)na + 1));
-    if (attempt == 0 && reusable) PH_HIPCHECK(c, c->t_nlj.ensure((size_t)na + 1));
+    if (attempt == 0 && reusable && !tile) PH_HIPCHECK(c, c->t_nlj.ensure((size_t)na + 1));
     PH_HIPCHECK(c, THS.ensure((size_t)na + 1));
     PH_HIPCHECK(c, THF.ensure((size_t)na + 1));
     // only the first attempt's lists serve the force pass
     const bool widen = attempt == 0 && reusable;
     const bool by_tile = tile && attempt == 0;
-    int32_t zero = 0, tfl = 0;  // tfl: list overflow seen by the autotuner
-    if (!by_tile || (tile_tune && attempt == 0)) {
+    int32_t zero = 0;
+    if (!by_tile) {
       PH_HIPCHECK(c, LB.ensure((size_t)list_cap(dlist) * na + 1));
       DBuf<double> &R2B = attempt == 0 ? c->nr2 : c->nr2_r;
-      if (c->tune.r2 || c->tune_mode == TUNE_PENDING) PH_HIPCHECK(c, R2B.ensure((size_t)list_cap(dlist) * na + 2));
+      if (c->tune.r2 || c->tune_mode == TUNE_PENDING)
+        PH_HIPCHECK(c, R2B.ensure((size_t)list_cap(dlist) * na + 2));
       rc = walk_groups(c, 0, rfac * lmargin, c->th_in.p, widen ? c->hmax0.p : nullptr);
       if (rc) return rc;
       hipLaunchKernelGGL(k_zero_i32, dim3(nblocks(n, 256)), dim3(256), 0, s, c->tmpi.p, n, 0);
       PH_HIPCHECK(c, dev_set(c, c->counters.p, &zero, sizeof(int32_t)));
       const IterLaunch L{c, s, c->ngroups, icall, rfac, na, lmargin, dlist, widen, LB.p, R2B.p, TNL.p, THS.p, THF.p};
-      if (attempt == 0 && c->tune_mode == TUNE_PENDING && (tile_tune || na >= TUNE_MIN_ACTIVE)) {
+      if (attempt == 0 && c->tune_mode == TUNE_PENDING && na >= TUNE_MIN_ACTIVE) {
         tuned_now = true;
         rc = tune_density_iter(c, L);  // times every configuration, keeps the fastest
         if (rc) return rc;
@@ -1561,20 +1614,7 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
         else launch_dens_iter(c->tune, L);
       }
     }
-    if (tile_tune && attempt == 0) {
-      // the configuration is for the particles that tiles leave to the list
-      // kernels; the tiles start from the unpadded active list again
-      PH_HIPCHECK(c, hipMemcpyAsync(&tfl, c->counters.p, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-      PH_HIPCHECK(c, hipMemcpyAsync(c->act.p, c->act_dens.p, sizeof(int32_t) * nact, hipMemcpyDeviceToDevice, s));
-      PH_HIPCHECK(c, hipStreamSynchronize(s));
-      c->nact = na = nact;
-      hipLaunchKernelGGL(k_zero_i32, dim3(nblocks(c->nleaves, 256)), dim3(256), 0, s, c->leaf_nits.p, c->nleaves, 0);
-    }
     if (by_tile) {
-      if (tile_tune) {  // the tuner walked other groups
-        rc = walk_groups(c, 0, rfac * lmargin, c->th_in.p, widen ? c->hmax0.p : nullptr, true);
-        if (rc) return rc;
-      }
       hipLaunchKernelGGL(k_zero_i32, dim3(nblocks(n, 256)), dim3(256), 0, s, c->tmpi.p, n, 0);
       PH_HIPCHECK(c, dev_set(c, c->counters.p, &zero, sizeof(int32_t)));
       rc = tile_lists(c, tl);
@@ -1623,7 +1663,7 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
     // a tuning attempt whose lists overflowed (the first call on a context
     // grows the list capacity) times unrepresentative work: tune again on
     // the next large call if that call's capacity is larger
-    if (attempt == 0 && tuned_now && ((fl | tfl) & DFL_LIST)) retune = true;
+    if (attempt == 0 && tuned_now && (fl & DFL_LIST)) retune = true;
     if (fl & DFL_NEGH) PH_RET(c, PHSPH_ERR_INPUT, "densityiterate: setting negative h from hrho");
     if (attempt == 0) {
       rewalk0 = (fl & DFL_REWALK) != 0;

@@ -7,10 +7,12 @@ Every configuration must give bit-identical outputs, so the choice never
 changes a result: each one is fixed in turn and the whole derivative chain
 (tree, density, cons2prim, force) compared bit for bit with the first; the
 oracle agreement of the tuned run is the parity tests' own."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
-from phantom_amd import setups, sph
+from phantom_amd import device, setups, sph
 from tests import parity
 
 pytestmark = pytest.mark.gpu
@@ -153,3 +155,29 @@ def test_tuned_once_when_budget_holds_capacity(gpu, monkeypatch):
     # round-off, the sums to their summation order
     assert np.max(np.abs(xyzh[:, 3] - ref["h"]) / ref["h"]) <= 1e-14
     assert parity.rel_rms(np.asarray(d["gradh"], np.float64), np.asarray(ref["gradh"], np.float64)) <= 1e-7
+
+
+def _free_bytes():
+    free, total = C.c_size_t(), C.c_size_t()
+    assert device.hip().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def test_tuning_beside_tiles_keeps_no_lists(gpu):
+    """A dense set is searched by tiles: the configurations are timed on a
+    sample, and neither that nor a later call leaves lists of all particles
+    (12 bytes an entry, 256 entries each) with the context."""
+    s = setups.uniform_box(nx=80, isothermal=False)
+    n = s["xyzh"].shape[0]
+    xyzh, vxyzu = s["xyzh"], s["vxyzu"]
+    free0 = _free_bytes()
+    ctx = sph.Context(s["params"])
+    for _ in range(2):
+        x = xyzh.copy()
+        ctx.maketree(x)
+        ctx.densityiterate(1, x, vxyzu, alphaind=s["alphaind"].copy())
+        assert ctx.get_search_stats()["tiles"] > 0 and ctx.get_tuning()["tuned"]
+    held = free0 - _free_bytes()
+    ctx.close()
+    print(f"\n  held {held / 2**30:.2f} GiB of {12 * 256 * n / 2**30:.2f} GiB that the lists would take", flush=True)
+    assert held < 12 * 256 * n * 0.75
