@@ -153,4 +153,4 @@ struct IterSums {
 void launch_dens_tile(phsph_ctx *c, int icall, double rfac, double lmargin, const double *hmax0,
                       const DensIterOut &out, const TileLists &tl);
 void launch_dens_sums(phsph_ctx *c, const TileLists &tl, bool mhd, bool mixed, const DensIn &in, const DensOut &out);
-int dens_tile_list_cap(const phsph_ctx *c);
+size_t tile_list_bytes(const phsph_ctx *c);

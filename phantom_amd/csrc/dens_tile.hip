@@ -418,11 +418,23 @@ static void tile_caps(const phsph_ctx *c, TileLists &tl) {
   tl.bncap = TileCap<K, TILE_BIG>::NC;
   tl.blc = TileCap<K, TILE_BIG>::LC;
 }
-int tile_lists(phsph_ctx *c, TileLists &tl) {
+static void tile_shape(const phsph_ctx *c, TileLists &tl) {
   const size_t ng = c->ntg;
   if (c->p.kernel == PHSPH_KERNEL_CUBIC) tile_caps<PHSPH_KERNEL_CUBIC>(c, tl);
   else tile_caps<PHSPH_KERNEL_QUINTIC>(c, tl);
   tl.bcap = (int)std::min(ng, 1024 + ng / 32);
+}
+// the memory of the lists of a context's tile groups
+size_t tile_list_bytes(const phsph_ctx *c) {
+  TileLists tl{};
+  tile_shape(c, tl);
+  const size_t group = sizeof(uint32_t) * tl.ncap + sizeof(uint16_t) * tl.lw * tl.lc * TILE_P,
+               large = sizeof(uint32_t) * tl.bncap + sizeof(uint16_t) * TILE_BW * tl.blc * TILE_P;
+  return group * c->ntg + large * tl.bcap;
+}
+int tile_lists(phsph_ctx *c, TileLists &tl) {
+  const size_t ng = c->ntg;
+  tile_shape(c, tl);
   PH_HIPCHECK(c, c->tl_cand.ensure(ng * tl.ncap));
   PH_HIPCHECK(c, c->tl_list.ensure(ng * tl.lw * tl.lc * TILE_P));
   PH_HIPCHECK(c, c->tl_nc.ensure(ng + 1));
@@ -440,9 +452,4 @@ int tile_lists(phsph_ctx *c, TileLists &tl) {
   tl.blist = c->tl_blist.p;
   tl.bnc = c->tl_bnc.p;
   return PHSPH_OK;
-}
-
-int dens_tile_list_cap(const phsph_ctx *c) {
-  return c->p.kernel == PHSPH_KERNEL_CUBIC ? TileCap<PHSPH_KERNEL_CUBIC, TILE_4>::LC
-                                           : TileCap<PHSPH_KERNEL_QUINTIC, TILE_4>::LC;
 }

@@ -1419,7 +1419,7 @@ static int tune_beside_tiles(phsph_ctx *c, int icall, double rfac, double lmargi
   if (rc) return rc;
   const int na = c->nact;
   int dlist = c->caps.dlist;
-  while (dlist > 16 && !list_fits(c, (size_t)list_cap(dlist) * na * 3)) dlist /= 2;
+  while (dlist > 16 && !list_fits(c, (size_t)list_cap(dlist) * na * 3)) dlist /= 2;  // 12 bytes an entry
   DBuf<uint32_t> lb;
   DBuf<double> r2b;
   PH_HIPCHECK(c, lb.ensure((size_t)list_cap(dlist) * na + 1));
@@ -1535,14 +1535,13 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
     rc = leaf_hmax_run(c, c->th_in.p, c->hmax0.p);
     if (rc) return rc;
   }
-  // list capacity: it grows for the particles run again (the list memory is
-  // that of the retried particles); a grown capacity is kept for later calls
-  // while the lists of every active particle fit in the list budget
-  // 12 bytes per entry: the entry and its squared separation
-  while (c->caps.dlist > 16 && !list_fits(c, (size_t)list_cap(c->caps.dlist) * nact * 3)) c->caps.dlist /= 2;
-  // Dense active sets are searched by tiles (dens_tile.hip), if the list
-  // capacity is not below a tile's own.
-  bool tile = !c->lists_only && tile_dense(c, nact, n) && c->caps.dlist >= dens_tile_list_cap(c);
+  // Dense active sets are searched by tiles (dens_tile.hip) while their lists
+  // fit in the list budget (an even set takes 320 to 390 bytes a particle with
+  // the cubic and 450 to 570 with the quintic kernel: the 16 GiB of the default
+  // hold 44M and 30M).  Boxes past the 11M and 5.6M where the list kernels'
+  // buffers shrink below a tile's list: 16.4M cubic 64 ms by tiles and 131 by
+  // lists, 7.1M quintic 31 and 57.
+  bool tile = !c->lists_only && tile_dense(c, nact, n) && tile_list_bytes(c) <= c->list_budget;
   if (tile) {
     PH_HIPCHECK(c, c->tg_t.ensure((size_t)c->ntg + 1));
     hipLaunchKernelGGL(k_tile_ranges, dim3(nblocks((size_t)c->ntg + 1, 256)), dim3(256), 0, s, c->ntg, c->tg_lo.p,
@@ -1555,7 +1554,13 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
     // particles handed back by tiles 7.3.
     tile = 2 * (int64_t)c->walk_unfit <= c->ntg;
   }
+  // 12 bytes per entry of a particle's list: the entry and its squared separation
+  auto fits = [&](int cap, int slots) { return list_fits(c, (size_t)list_cap(cap) * slots * 3); };
   if (!tile) {
+    // list capacity: it grows for the particles run again (the list memory is
+    // that of the retried particles); a grown capacity is kept for later calls
+    // while the lists of every active particle fit in the list budget
+    while (c->caps.dlist > 16 && !fits(c->caps.dlist, nact)) c->caps.dlist /= 2;
     rc = pad_groups(c);
     if (rc) return rc;
   }
@@ -1576,6 +1581,9 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
   for (int attempt = 0; attempt < 12; attempt++) {
     const int na = c->nact;  // active slots, padding included
     if (na == 0) break;
+    // the first lists of particles that tiles handed back
+    if (tile && attempt == 1)
+      while (dlist > 16 && !fits(dlist, na)) dlist /= 2;
     // the first attempt writes the lists the force pass may use; retries
     // write buffers of their own so that those stay intact
     DBuf<uint32_t> &LB = attempt == 0 ? c->nlist : c->nlist_r;
@@ -1719,7 +1727,7 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
       c->rfac_level--;
     }
   }
-  while (dlist > c->caps.dlist && !list_fits(c, (size_t)list_cap(dlist) * nact * 3)) dlist /= 2;
+  while (dlist > c->caps.dlist && !fits(dlist, nact)) dlist /= 2;
   if (dlist > c->caps.dlist) c->caps.dlist = dlist;
   // where the list budget holds the capacity, the overflow recurs on every
   // call and the tuned configuration stands

@@ -3,7 +3,8 @@ candidate leaves, density and force neighbour lists and gravity near-field
 lists overflow.  With the default list budget the library doubles its
 uniform capacities; with a 1 KiB budget it takes its exact-size paths
 (per-group candidate offsets, per-group force list capacities, per-leaf
-near-field offsets; density retries with longer lists in both), and the
+near-field offsets; density retries with longer lists), with lists=1 the list
+kernels search where tiles would, and the
 self-gravity force pass's neighbour lists overflow and run again at the
 longest list.  Either way
 it must agree with the oracle to the parity tolerances: neighbour and
@@ -20,6 +21,7 @@ from tests.test_gpu_gravity import _moving, _run_gpu as run_gpu_grav, _run_oracl
 pytestmark = pytest.mark.gpu
 
 SPECS = {"doubling": "gcand=4,dlist=16,flist=16,p2p=2,gnear=4",
+         "doubling_lists": "gcand=4,dlist=16,flist=16,p2p=2,gnear=4,lists=1",
          "exact": "gcand=4,dlist=16,flist=16,p2p=2,gnear=4,budget_kib=1"}
 
 

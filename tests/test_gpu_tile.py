@@ -115,3 +115,16 @@ def test_active_fraction_and_kernel_choose_the_search(frac, kernel, n, tiles, gp
     print(f"\n[case {frac} {kernel} {n}]", flush=True)
     st = check(_open_levels(frac, kernel, *n))
     assert (st["tiles"] > 0) == tiles, st
+
+
+# lists of 128 groups (cubic) take 2 MB, those of groups in the large form, which
+# have room for all here, 21 MiB; lists of all particles 16.9 MiB at 256 entries
+@pytest.mark.parametrize("caps,tiles", [("dlist=16", True), ("budget_kib=18432", False), ("budget_kib=32768", True),
+                                        ("lists=1", False)])
+def test_budget_of_the_tiles_own_lists(caps, tiles, gpu, monkeypatch):
+    """Tiles run while their own lists fit in the list budget, whatever the
+    capacity of the list kernels' buffers."""
+    monkeypatch.setenv("PHSPH_CAPS", caps)
+    print(f"\n[case {caps}]", flush=True)
+    st = check(_open_levels(1.0, abi.KERNEL_CUBIC, 18, 16, 20))
+    assert (st["tiles"] > 0) == tiles, st
