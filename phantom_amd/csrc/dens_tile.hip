@@ -338,8 +338,8 @@ k_dens_tile(DevConst dc, int icall, double rfac, double lmargin, const int32_t *
           if (dc.radkern * hi * (1. + 1e-12) > rcut) {  // outgrew the list: run again with a wider one
             if (sl == 0) {
               atomicOr(flags, DFL_REWALK);
-              atomicAdd(out.nrewalk, 1);
-              out.retry[p] = 1;
+              // once, also in a group that runs again in the large form
+              if (atomicExch(&out.retry[p], 1) == 0) atomicAdd(out.nrewalk, 1);
             }
             run = ok = false;
           }

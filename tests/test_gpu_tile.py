@@ -9,7 +9,7 @@ terms in another order, a few 1e-16 each)."""
 import numpy as np
 import pytest
 
-from phantom_amd import abi, setups
+from phantom_amd import abi, setups, sph
 from tests import parity
 
 pytestmark = pytest.mark.gpu
@@ -128,3 +128,34 @@ def test_budget_of_the_tiles_own_lists(caps, tiles, gpu, monkeypatch):
     print(f"\n[case {caps}]", flush=True)
     st = check(_open_levels(1.0, abi.KERNEL_CUBIC, 18, 16, 20))
     assert (st["tiles"] > 0) == tiles, st
+
+
+def test_outgrown_particles_count_once(gpu):
+    """The search radius of the next call goes by how many particles outgrew
+    their lists (more than 1/200: wider).  A group that is run again in the large
+    form, for a list that is too long, meets its outgrown particles twice: 30 of
+    8192 here, in groups with one such list each."""
+    setup = setups.uniform_box(nx=32, ny=16, nz=16, seed=8, box=(-1.0, 1.0, -0.5, 0.5, -0.5, 0.5))
+    p = setup["params"]
+    p.tolh = 2e-3  # above 1e-3 the lists do not serve the force pass and the radius goes by this count alone
+    n = setup["xyzh"].shape[0]
+    cell = np.floor((setup["xyzh"][:, :3] - [-1.0, -0.5, -0.5]) * 16.0).astype(int)
+    block, local = cell // 4, cell % 4  # nodes of 64 particles: 4 x 4 x 4 lattice cells
+    some = (block[:, 0] * 16 + block[:, 1] * 4 + block[:, 2]) % 4 == 1
+    ids = np.flatnonzero(some & (local == 1).all(axis=1))[:30]
+    keep = {tuple(b) for b in block[ids]}
+    big = [i for i in np.flatnonzero(some & (local == 2).all(axis=1)) if tuple(block[i]) in keep]
+    assert len(ids) == len(big) == 30
+    ctx = sph.Context(p)
+    xyzh = setup["xyzh"].copy()
+    for k in range(3):
+        if k == 2:
+            assert ctx.get_tuning()["search_radius"] == 1.03
+            xyzh[ids, 3] *= 0.9
+            xyzh[big, 3] *= 1.25
+        ctx.maketree(xyzh)
+        ctx.densityiterate(1, xyzh, setup["vxyzu"], alphaind=setup["alphaind"].copy())
+    st, radius = ctx.get_search_stats(), ctx.get_tuning()["search_radius"]
+    ctx.close()
+    assert st["tiles"] == 128 and st["large"] == 30 and st["again"] >= 30, st
+    assert 200 * 30 <= n < 2 * 200 * 30 and radius == 1.03
