@@ -226,6 +226,8 @@ int phsph_create(const phsph_params *p, int32_t device, phsph_ctx **out) {
           else if (key == "p2p") c->caps.p2p = v;
           else if (key == "gnear") c->caps.gnear = v;
           else if (key == "budget_kib") c->list_budget = (size_t)v << 10;
+          else if (key == "wstack") c->caps.wstack = std::max(v, 2);
+          else if (key == "tlarge") c->caps.tlarge = v;
           else if (key == "lists") c->lists_only = true;
         }
       }

@@ -74,6 +74,9 @@ struct Caps {
   int dlist = 256;   // density neighbour list per particle
   int flist = 256;   // force neighbour list per particle
   int gnear = 128;   // neighbours per particle in the self-gravity force pass
+  // limits below the kernels' own, so that tests reach what follows them
+  int wstack = 1 << 24;  // nodes of the group walk's first stack
+  int tlarge = 1 << 24;  // tile groups with room in the large form
 };
 
 // list-kernel configuration picked by the autotuner (density.hip):

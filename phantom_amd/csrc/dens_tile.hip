@@ -422,7 +422,7 @@ static void tile_shape(const phsph_ctx *c, TileLists &tl) {
   const size_t ng = c->ntg;
   if (c->p.kernel == PHSPH_KERNEL_CUBIC) tile_caps<PHSPH_KERNEL_CUBIC>(c, tl);
   else tile_caps<PHSPH_KERNEL_QUINTIC>(c, tl);
-  tl.bcap = (int)std::min(ng, 1024 + ng / 32);
+  tl.bcap = std::min((int)std::min(ng, 1024 + ng / 32), c->caps.tlarge);
 }
 // the memory of the lists of a context's tile groups
 size_t tile_list_bytes(const phsph_ctx *c) {

@@ -126,8 +126,8 @@ k_group_walk(DevConst dc, int mode, double rfac, const phsph_kdnode *__restrict_
              const double *__restrict__ tx,
              const double *__restrict__ ty, const double *__restrict__ tz, const double *__restrict__ hsrc,
              int ngroups, uint32_t *__restrict__ gcand, int32_t *__restrict__ gncand, const int64_t *goff,
-             int capg, double *__restrict__ gbox, int32_t *__restrict__ flags) {
-  __shared__ int stk[STACK];
+             int capg, int stack, double *__restrict__ gbox, int32_t *__restrict__ flags) {
+  __shared__ int stk[STACK];  // of which stack are used
   const int g = xcd_block(blockIdx.x, gridDim.x);
   if (g >= ngroups) return;
   if (STACK == WALK_STACK && gncand[g] >= 0) return;
@@ -204,7 +204,7 @@ k_group_walk(DevConst dc, int mode, double rfac, const phsph_kdnode *__restrict_
     const bool push = open && !isleaf;
     const unsigned long long mi = __ballot(push);
     const int npush = 2 * __popcll(mi);
-    if (top + npush > STACK) {
+    if (top + npush > stack) {
       ovf = true;
       break;
     }
@@ -1157,7 +1157,8 @@ int walk_groups(phsph_ctx *c, int mode, double rfac, const double *d_hsrc, const
 #define WALK(SS)                                                                                                \
   hipLaunchKernelGGL((k_group_walk<SS>), dim3(xcd_grid(ng)), dim3(64), 0, s, c->dc, mode, rfac, c->nd.p, d_hmaxn, \
                      c->leaf_flag.p, c->act.p, c->nact, tiles ? c->tg_t.p : nullptr, c->tx.p, c->ty.p, c->tz.p,   \
-                     d_hsrc, ng, c->gcand.p, c->gncand.p, goff, c->caps.gcand, c->gbox.p, c->counters.p)
+                     d_hsrc, ng, c->gcand.p, c->gncand.p, goff, c->caps.gcand,                                    \
+                     SS == WALK_STACK ? SS : std::min(SS, c->caps.wstack), c->gbox.p, c->counters.p)
     if (ng > 0) {
       LaunchTimer lt(c, mode == 0 ? "walk_density" : "walk_force");
       WALK(WALK_STACK_LO);
@@ -1614,10 +1615,13 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
         if (rc) return rc;
       } else {
         LaunchTimer lt(c, "density_iter");
-        // a wavefront per particle below half of the particles active (1/8:
-        // 2.2 times faster); on all particles the list kernel is as fast with
-        // the quintic (5.7 and 5.8 ms on 2M) and faster with the cubic kernel
-        // (10.6 and 15.4 ms on 8.4M)
+        // a wavefront per particle below half of the particles active, padding
+        // of the groups included (1/8: 2.2 times faster; substep of a 160^3 box
+        // at 0.375 16.8 ms by particles and 16.5 by groups with the cubic and
+        // 21.1 and 22.2 with the quintic kernel, of 100^3 5.3 and 5.9, 6.2 and
+        // 7.2); on all particles the list kernel is as fast with the quintic
+        // (5.7 and 5.8 ms on 2M) and faster with the cubic kernel (10.6 and 15.4
+        // ms on 8.4M)
         if (2 * (int64_t)na < n) launch_dens_solo(L);
         else launch_dens_iter(c->tune, L);
       }

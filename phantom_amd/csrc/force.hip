@@ -828,8 +828,10 @@ int cons2prim_run(phsph_ctx *c, int np, const double *xyzh, int ldx, const doubl
 // Active slots below which the lists are searched by a wavefront per particle:
 // 0.18 ms on a box of 101520 particles (0.45 by groups of 64) and 0.92 ms on a
 // 500k polytrope (3.1, waiting for the groups of its outer layers).  In an even
-// set the groups take less from about half a million on (the density search
-// by groups costs 1.3 ns a particle in a box of 8.4M, by particles 1.8).
+// set both take the same time: 0.23 and 0.23 ms on 64^3, 0.78 and 0.80 ms on
+// 80^3 particles with the cubic, 0.42 and 0.43, 1.01 and 1.16 ms with the
+// quintic kernel.  On 8.4M the density search takes 1.3 ns a particle by groups
+// and 1.8 by particles; the line lies between.
 constexpr int FLIST_SOLO_MAX = 1 << 20;
 
 // ------------------------------------------------------------------------

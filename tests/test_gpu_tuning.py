@@ -4,9 +4,10 @@ per block, squared separations stored or recomputed, one group per
 wavefront or persistent wavefronts on per-XCD work queues) and keeps the
 fastest.
 Every configuration must give bit-identical outputs, so the choice never
-changes a result: each one is fixed in turn and the whole derivative chain
-(tree, density, cons2prim, force) compared bit for bit with the first; the
-oracle agreement of the tuned run is the parity tests' own."""
+changes a result: each one is fixed in turn, on sets that are searched by lists
+(PHSPH_CAPS=lists=1: tiles would take these dense sets), and the whole
+derivative chain (tree, density, cons2prim, force) compared bit for bit with
+the first, and the first with the oracle's neighbour counts."""
 import ctypes as C
 
 import numpy as np
@@ -37,6 +38,7 @@ def _chain(setup, cfg=None, calls=1):
     c = ctx.cons2prim(xyzh, setup["vxyzu"], d["dvdx"], alphaind)
     f = ctx.force(1, xyzh, setup["vxyzu"], d["gradh"], alphaind, c["eos_vars"])
     tune = ctx.get_tuning()
+    tune["tiles"] = ctx.get_search_stats()["tiles"]
     ctx.close()
     out = dict(h=xyzh[:, 3], gradh=d["gradh"], divv=d["divcurlv"], dvdx=d["dvdx"], nneigh=nneigh, nits=nits,
                f=f["fxyzu"], dtc=f["dtcourant"], dtf=f["dtforce"])
@@ -67,15 +69,17 @@ def test_autotune_picks_fastest(case):
                                          for t in tried), flush=True)
 
 
-def test_configurations_bit_identical(case):
+def test_configurations_bit_identical(case, monkeypatch):
     name, s = case
+    monkeypatch.setenv("PHSPH_CAPS", "lists=1")
     ref, t0 = _chain(s, CONFIGS[0])
+    assert t0["tiles"] == 0
     assert not t0["tuned"] and (t0["cl"], t0["lw"], t0["r2"], t0["q"]) == CONFIGS[0]
     for cfg in CONFIGS[1:]:
         out, _ = _chain(s, cfg)
         for k in ref:
             np.testing.assert_array_equal(np.asarray(out[k]), np.asarray(ref[k]), err_msg=f"{cfg} {k}")
-    # and the tuned run against the oracle's neighbour counts
+    # and the first against the oracle's neighbour counts
     o = parity.run_oracle(s)
     np.testing.assert_array_equal(ref["nneigh"], o["dens"]["nneigh"])
 
