@@ -1579,7 +1579,8 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
   }
   TileLists tl{};
   int nrewalk = 0;  // particles of the first attempt that outgrew their lists
-  for (int attempt = 0; attempt < 12; attempt++) {
+  const int nattempt = tile ? 13 : 12;  // twelve by lists
+  for (int attempt = 0; attempt < nattempt; attempt++) {
     const int na = c->nact;  // active slots, padding included
     if (na == 0) break;
     // the first lists of particles that tiles handed back

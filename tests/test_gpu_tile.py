@@ -216,3 +216,13 @@ def test_paths(name, gpu, monkeypatch):
     assert (st["deep"] > 0) == ("wstack" in caps), st
     if name == "no_room_large":
         assert st["large"] > 1
+
+
+def test_handed_back_particles_have_every_list_attempt(gpu, monkeypatch):
+    """Lists grow from one entry to the 2048 of the twelfth attempt: smoothing
+    lengths 2.5 times too large give lists of about 1200, which no tile holds."""
+    monkeypatch.setenv("PHSPH_CAPS", "dlist=1")
+    s = _open_levels(1.0, abi.KERNEL_CUBIC, 18, 16, 20)
+    s["xyzh"][:, 3] *= 2.5
+    st = check(s)
+    assert st["tiles"] > 0 and st["again"] > 0, st
