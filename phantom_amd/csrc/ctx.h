@@ -127,7 +127,7 @@ struct phsph_ctx {
   DBuf<double2> t_sums;      // sums of the last h iteration per active slot
   int ntg = 0, tg_max = 0;   // tile groups, particles of the largest
   bool lists_only = false;   // no tiles (PHSPH_CAPS, for tests of the list kernels)
-  int walk_unfit = 0;        // tile groups of the last walk that are no tiles
+  int walk_unfit = 0, walk_uneven[2] = {0, 0};  // tile groups of the last walk that are no tiles, that are uneven
   // phsph_get_search_stats
   int stat_tiles = 0, stat_again = 0, stat_deep = 0, stat_force_tiles = 0;
   DBuf<int32_t> pleaf;       // tree position -> index into leaves

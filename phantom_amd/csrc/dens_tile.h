@@ -5,8 +5,11 @@
 
 enum { DFL_CAND = 1, DFL_LIST = 2, DFL_REWALK = 4, DFL_NOCONV = 8, DFL_NEGH = 16, DFL_STACK = 32, DFL_TILE = 64,
        DFL_STACK_LO = 128 };
-// c->counters: particles that outgrew their lists (tiles), and groups that are no tiles (tile_unfit)
-constexpr int CNT_REWALK = 8, CNT_UNFIT = 9;
+// c->counters: particles that outgrew their lists (tiles), groups that are no
+// tiles (tile_unfit), and of one group in UNEVEN_STEP those whose largest h is
+// more than 1.3 and more than 1.5 times the smallest
+constexpr int CNT_REWALK = 8, CNT_UNFIT = 9, CNT_UNEVEN = 10, CNT_WALK = 12;  // CNT_WALK: words of a walk
+constexpr int UNEVEN_STEP = 8;
 
 struct DensIn {
   const double4 *tp;  // x, y, z (treecache) and h at entry

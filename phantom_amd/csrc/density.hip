@@ -140,7 +140,7 @@ k_group_walk(DevConst dc, int mode, double rfac, const phsph_kdnode *__restrict_
     return;
   }
   double xl = PH_HUGE64, yl = PH_HUGE64, zl = PH_HUGE64, xh = -PH_HUGE64, yh = -PH_HUGE64, zh = -PH_HUGE64;
-  double hm = 0.;
+  double hm = 0., hmin = PH_HUGE64;
   for (int t = t0 + lane; t < t1; t += 64) {
     const int p = act[t];
     if (p < 0) continue;
@@ -148,6 +148,7 @@ k_group_walk(DevConst dc, int mode, double rfac, const phsph_kdnode *__restrict_
     yl = fmin(yl, ty[p]); yh = fmax(yh, ty[p]);
     zl = fmin(zl, tz[p]); zh = fmax(zh, tz[p]);
     hm = fmax(hm, hsrc[p]);
+    hmin = fmin(hmin, hsrc[p]);
   }
   xl = wave_min(xl); yl = wave_min(yl); zl = wave_min(zl);
   xh = wave_max(xh); yh = wave_max(yh); zh = wave_max(zh);
@@ -219,7 +220,14 @@ k_group_walk(DevConst dc, int mode, double rfac, const phsph_kdnode *__restrict_
   if (gt && !ovf) {
     smax = wave_max(smax);
     hmx = wave_max(hmx);
-    if (lane == 0 && tile_unfit(dc, ex, ey, ez, rfac * dc.radkern, hm, hmx, smax)) atomicAdd(&flags[CNT_UNFIT], 1);
+    hmin = wave_min(hmin);
+    if (lane == 0) {
+      if (tile_unfit(dc, ex, ey, ez, rfac * dc.radkern, hm, hmx, smax)) atomicAdd(&flags[CNT_UNFIT], 1);
+      if (g % UNEVEN_STEP == 0 && hm > 1.3 * hmin) {
+        atomicAdd(&flags[CNT_UNEVEN], 1);
+        if (hm > 1.5 * hmin) atomicAdd(&flags[CNT_UNEVEN + 1], 1);
+      }
+    }
   }
   if (lane == 0) {
     gncand[g] = ovf ? -1 : nc;
@@ -1151,8 +1159,8 @@ int walk_groups(phsph_ctx *c, int mode, double rfac, const double *d_hsrc, const
     if (!exact) PH_HIPCHECK(c, c->gcand.ensure((size_t)(ng + 1) * c->caps.gcand));
     PH_HIPCHECK(c, c->gncand.ensure(ng + 1));
     PH_HIPCHECK(c, c->gbox.ensure((size_t)(ng + 1) * GBOX));
-    int32_t cnt[CNT_UNFIT + 1] = {};
-    const size_t ncnt = sizeof(int32_t) * (tiles ? CNT_UNFIT + 1 : 1);
+    int32_t cnt[CNT_WALK] = {};
+    const size_t ncnt = sizeof(int32_t) * (tiles ? CNT_WALK : 1);
     PH_HIPCHECK(c, dev_set(c, c->counters.p, cnt, ncnt));
 #define WALK(SS)                                                                                                \
   hipLaunchKernelGGL((k_group_walk<SS>), dim3(xcd_grid(ng)), dim3(64), 0, s, c->dc, mode, rfac, c->nd.p, d_hmaxn, \
@@ -1177,6 +1185,8 @@ int walk_groups(phsph_ctx *c, int mode, double rfac, const double *d_hsrc, const
 #undef WALK
     const int32_t fl = cnt[0];
     c->walk_unfit = cnt[CNT_UNFIT];
+    c->walk_uneven[0] = cnt[CNT_UNEVEN];
+    c->walk_uneven[1] = cnt[CNT_UNEVEN + 1];
     if (getenv("PHSPH_DEBUG")) {
       size_t fr = 0, tot = 0;
       (void)hipMemGetInfo(&fr, &tot);
@@ -1554,6 +1564,19 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
     // the force pass.  Box of 256 x 256 x 12, cubic kernel: 5.6 ms, as
     // particles handed back by tiles 7.3.
     tile = 2 * (int64_t)c->walk_unfit <= c->ntg;
+    // Where h differs within most groups, as it does where particles lie at
+    // random, the lists of small h, which also hold every j whose own radius
+    // reaches them, pass a tile's length: such groups need the large form, which
+    // is slower and has room for 1024 and a thirtieth of them (the others are
+    // handed back after their search).  Above that lists of all particles.  Calls
+    // by tiles and by lists, ms: quintic, random 60k 1.9 and 3.0, 100k 3.3 and
+    // 3.2, 1M 16.0 and 10.9, disc 60k 3.8 and 3.6, 1M 26.7 and 20.8; cubic, disc
+    // 60k 1.8 and 2.6, 100k 3.3 and 2.8, 1M 11.4 and 9.2, random, a fifth of whose
+    // groups need the large form, 200k 2.1 and 3.1, 1M 7.4 and 7.4, 4M 25.1 and 23.3.
+    const int some = (c->ntg + UNEVEN_STEP - 1) / UNEVEN_STEP;
+    const bool uneven = 2 * c->walk_uneven[0] > some, very = 3 * c->walk_uneven[1] > 2 * some;
+    if (c->p.kernel == PHSPH_KERNEL_CUBIC) tile = tile && !(uneven && c->ntg > (very ? 2048 : 16384));
+    else tile = tile && !(uneven && c->ntg > 1024);
   }
   // 12 bytes per entry of a particle's list: the entry and its squared separation
   auto fits = [&](int cap, int slots) { return list_fits(c, (size_t)list_cap(cap) * slots * 3); };

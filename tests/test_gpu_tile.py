@@ -226,3 +226,14 @@ def test_handed_back_particles_have_every_list_attempt(gpu, monkeypatch):
     s["xyzh"][:, 3] *= 2.5
     st = check(s)
     assert st["tiles"] > 0 and st["again"] > 0, st
+
+
+# random positions and h: about 55 particles a group
+@pytest.mark.parametrize("kernel,n,spread,tiles", [
+    (abi.KERNEL_QUINTIC, 40000, 0.2, True), (abi.KERNEL_QUINTIC, 80000, 0.2, False),
+    (abi.KERNEL_CUBIC, 80000, 0.4, True), (abi.KERNEL_CUBIC, 160000, 0.4, False),
+    (abi.KERNEL_CUBIC, 160000, 0.16, True)])
+def test_uneven_sets_with_many_groups_go_by_lists(kernel, n, spread, tiles, gpu):
+    print(f"\n[case {kernel} {n} {spread}]", flush=True)
+    st = check(setups.random_box(n=n, seed=21, kernel=kernel, hmin_frac=1.0 - spread, hmax_frac=1.0 + spread))
+    assert (st["tiles"] > 0) == tiles, st
