@@ -1575,8 +1575,10 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
     // groups need the large form, 200k 2.1 and 3.1, 1M 7.4 and 7.4, 4M 25.1 and 23.3.
     const int some = (c->ntg + UNEVEN_STEP - 1) / UNEVEN_STEP;
     const bool uneven = 2 * c->walk_uneven[0] > some, very = 3 * c->walk_uneven[1] > 2 * some;
-    if (c->p.kernel == PHSPH_KERNEL_CUBIC) tile = tile && !(uneven && c->ntg > (very ? 2048 : 16384));
-    else tile = tile && !(uneven && c->ntg > 1024);
+    // (a step of the random cubic set whose search radius is the widest: 200k 5.3
+    // and 3.5, 1M 14.9 and 10.6)
+    const int most = (c->p.kernel != PHSPH_KERNEL_CUBIC || rfac > 1.07) ? 1024 : very ? 2048 : 16384;
+    tile = tile && !(uneven && c->ntg > most);
   }
   // 12 bytes per entry of a particle's list: the entry and its squared separation
   auto fits = [&](int cap, int slots) { return list_fits(c, (size_t)list_cap(cap) * slots * 3); };

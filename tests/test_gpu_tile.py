@@ -228,12 +228,38 @@ def test_handed_back_particles_have_every_list_attempt(gpu, monkeypatch):
     assert st["tiles"] > 0 and st["again"] > 0, st
 
 
-# random positions and h: about 55 particles a group
-@pytest.mark.parametrize("kernel,n,spread,tiles", [
-    (abi.KERNEL_QUINTIC, 40000, 0.2, True), (abi.KERNEL_QUINTIC, 80000, 0.2, False),
-    (abi.KERNEL_CUBIC, 80000, 0.4, True), (abi.KERNEL_CUBIC, 160000, 0.4, False),
-    (abi.KERNEL_CUBIC, 160000, 0.16, True)])
-def test_uneven_sets_with_many_groups_go_by_lists(kernel, n, spread, tiles, gpu):
-    print(f"\n[case {kernel} {n} {spread}]", flush=True)
-    st = check(setups.random_box(n=n, seed=21, kernel=kernel, hmin_frac=1.0 - spread, hmax_frac=1.0 + spread))
+# random positions and h, about 55 particles a group, at the widest search radius
+# (that of a context's first call)
+@pytest.mark.parametrize("kernel,n,tiles", [(abi.KERNEL_QUINTIC, 40000, True), (abi.KERNEL_QUINTIC, 80000, False),
+                                            (abi.KERNEL_CUBIC, 40000, True), (abi.KERNEL_CUBIC, 80000, False)])
+def test_uneven_sets_with_many_groups_go_by_lists(kernel, n, tiles, gpu):
+    print(f"\n[case {kernel} {n}]", flush=True)
+    st = check(setups.random_box(n=n, seed=21, kernel=kernel, hmin_frac=0.7, hmax_frac=1.3))
     assert (st["tiles"] > 0) == tiles, st
+
+
+# after three calls, at the narrowest: the h of random positions differ by 1.45
+# within a group, and h with a factor of two between neighbours by more
+@pytest.mark.parametrize("n,factor,tiles", [(80000, 1.0, True), (160000, 1.0, True), (80000, 2.0, True),
+                                            (160000, 2.0, False)])
+def test_uneven_cubic_sets_at_the_narrow_radius(n, factor, tiles, gpu):
+    print(f"\n[case {n} {factor}]", flush=True)
+    s = setups.random_box(n=n, seed=22, hmin_frac=1.0, hmax_frac=1.0)
+    ctx = sph.Context(s["params"])
+    for k in range(4):
+        if k == 3:
+            assert ctx.get_tuning()["search_radius"] == 1.03
+            s["xyzh"][::2, 3] *= factor  # above the converged h: none outgrows its list
+        xyzh = s["xyzh"].copy()
+        ctx.maketree(xyzh)
+        ctx.densityiterate(1, xyzh, s["vxyzu"], alphaind=s["alphaind"].copy())
+        if k < 3:
+            s["xyzh"][:, 3] = xyzh[:, 3]
+    st = ctx.get_search_stats()
+    nneigh, nits = ctx.get_particle_stats(n)
+    ctx.close()
+    assert (st["tiles"] > 0) == tiles, st
+    o = parity.run_oracle(s)
+    np.testing.assert_array_equal(nneigh, o["dens"]["nneigh"])
+    np.testing.assert_array_equal(nits, o["dens"]["nits"])
+    assert parity.rel_rms(xyzh[:, 3], o["xyzh"][:, 3]) <= 1e-12
