@@ -118,7 +118,9 @@ __global__ void k_walk(DevConst dc, double rfac, const phsph_kdnode *__restrict_
 // is a chain of dependent node loads, about twenty per group, so what counts is
 // how many groups a CU has in flight: 4 kB of stack allow 32, the 16 kB that
 // the widest groups need allowed 10.  8M-particle box 0.67 ms (1.53 with 16 kB).
-template <int STACK>
+// TILES: the groups are the tile groups gt of the active list; their boxes and
+// search h go to gbox, and those that are no tiles, or uneven, are counted.
+template <int STACK, bool TILES>
 __global__ void __launch_bounds__(64)
 k_group_walk(DevConst dc, int mode, double rfac, const phsph_kdnode *__restrict__ nd,
              const double *__restrict__ hmaxn, const int32_t *__restrict__ leaf_flag,
@@ -134,7 +136,7 @@ k_group_walk(DevConst dc, int mode, double rfac, const phsph_kdnode *__restrict_
   const size_t gbase = cand_base(goff, g, capg);
   const int gcap = cand_cap(goff, g, capg);
   const int lane = threadIdx.x;
-  const int t0 = gt ? gt[g] : g * GROUP, t1 = gt ? gt[g + 1] : min(nact, t0 + GROUP);
+  const int t0 = TILES ? gt[g] : g * GROUP, t1 = TILES ? gt[g + 1] : min(nact, t0 + GROUP);
   if (t0 >= t1) {  // a tile without active particles
     if (lane == 0) gncand[g] = 0;
     return;
@@ -148,12 +150,12 @@ k_group_walk(DevConst dc, int mode, double rfac, const phsph_kdnode *__restrict_
     yl = fmin(yl, ty[p]); yh = fmax(yh, ty[p]);
     zl = fmin(zl, tz[p]); zh = fmax(zh, tz[p]);
     hm = fmax(hm, hsrc[p]);
-    hmin = fmin(hmin, hsrc[p]);
+    if (TILES) hmin = fmin(hmin, hsrc[p]);
   }
   xl = wave_min(xl); yl = wave_min(yl); zl = wave_min(zl);
   xh = wave_max(xh); yh = wave_max(yh); zh = wave_max(zh);
   hm = wave_max(hm);
-  if (gbox && lane < GBOX)  // the box and search h for the tile kernels
+  if (TILES && lane < GBOX)  // the box and search h for the tile kernels
     gbox[(size_t)g * GBOX + lane] = (lane < 3) ? (lane == 0 ? xl : lane == 1 ? yl : zl)
                                    : (lane < 6) ? (lane == 3 ? xh : lane == 4 ? yh : zh) : hm;
   const double bx = 0.5 * (xl + xh), by = 0.5 * (yl + yh), bz = 0.5 * (zl + zh);
@@ -174,7 +176,7 @@ k_group_walk(DevConst dc, int mode, double rfac, const phsph_kdnode *__restrict_
     top -= take;
     bool open = false, isleaf = false;
     int lc = 0, rc = 0;
-    double size = 0.;
+    double size = 0., hn = 0.;
     if (node > 0) {
       const phsph_kdnode e = nd[node];
       size = e.size;
@@ -187,8 +189,11 @@ k_group_walk(DevConst dc, int mode, double rfac, const phsph_kdnode *__restrict_
       const double qx = fmax(fabs(dx) - ex, 0.), qy = fmax(fabs(dy) - ey, 0.), qz = fmax(fabs(dz) - ez, 0.);
       const double d2 = qx * qx + qy * qy + qz * qz;
       double rc_ = rcg;
-      if (hmaxn) rc_ = fmax(rc_, (mode == 1 ? 1. : rfac) * dc.radkern * hmaxn[node]);
-      const double s = (e.size + rc_) * (1. + 1e-10);
+      if (hmaxn) {
+        hn = hmaxn[node];
+        rc_ = fmax(rc_, (mode == 1 ? 1. : rfac) * dc.radkern * hn);
+      }
+      const double s = (size + rc_) * (1. + 1e-10);
       open = d2 < s * s;
       isleaf = leaf_flag[node] != 0;
       lc = e.leftchild;
@@ -198,8 +203,10 @@ k_group_walk(DevConst dc, int mode, double rfac, const phsph_kdnode *__restrict_
     if (open && isleaf) {
       const int k = nc + __popcll(ml & lanemask_lt());
       if (k < gcap) gcand[gbase + k] = (uint32_t)node;
-      smax = fmax(smax, size);
-      if (hmaxn) hmx = fmax(hmx, hmaxn[node]);
+      if (TILES) {
+        smax = fmax(smax, size);
+        hmx = fmax(hmx, hn);
+      }
     }
     nc += __popcll(ml);
     const bool push = open && !isleaf;
@@ -217,7 +224,7 @@ k_group_walk(DevConst dc, int mode, double rfac, const phsph_kdnode *__restrict_
     top += npush;
     __syncthreads();
   }
-  if (gt && !ovf) {
+  if (TILES && !ovf) {
     smax = wave_max(smax);
     hmx = wave_max(hmx);
     hmin = wave_min(hmin);
@@ -1163,7 +1170,9 @@ int walk_groups(phsph_ctx *c, int mode, double rfac, const double *d_hsrc, const
     const size_t ncnt = sizeof(int32_t) * (tiles ? CNT_WALK : 1);
     PH_HIPCHECK(c, dev_set(c, c->counters.p, cnt, ncnt));
 #define WALK(SS)                                                                                                \
-  hipLaunchKernelGGL((k_group_walk<SS>), dim3(xcd_grid(ng)), dim3(64), 0, s, c->dc, mode, rfac, c->nd.p, d_hmaxn, \
+  if (tiles) { WALKT(SS, true); } else { WALKT(SS, false); }
+#define WALKT(SS, TT)                                                                                           \
+  hipLaunchKernelGGL((k_group_walk<SS, TT>), dim3(xcd_grid(ng)), dim3(64), 0, s, c->dc, mode, rfac, c->nd.p, d_hmaxn, \
                      c->leaf_flag.p, c->act.p, c->nact, tiles ? c->tg_t.p : nullptr, c->tx.p, c->ty.p, c->tz.p,   \
                      d_hsrc, ng, c->gcand.p, c->gncand.p, goff, c->caps.gcand,                                    \
                      SS == WALK_STACK ? SS : std::min(SS, c->caps.wstack), c->gbox.p, c->counters.p)
@@ -1183,6 +1192,7 @@ int walk_groups(phsph_ctx *c, int mode, double rfac, const double *d_hsrc, const
       PH_HIPCHECK(c, hipStreamSynchronize(s));
     }
 #undef WALK
+#undef WALKT
     const int32_t fl = cnt[0];
     c->walk_unfit = cnt[CNT_UNFIT];
     c->walk_uneven[0] = cnt[CNT_UNEVEN];
