@@ -206,8 +206,10 @@ int phsph_create(const phsph_params *p, int32_t device, phsph_ctx **out) {
   c->dc = make_devconst(*p);
   // initial list capacities and the list budget (KiB) may be set from the
   // environment, e.g. PHSPH_CAPS="gcand=64,dlist=32,flist=32,p2p=16,gnear=8,budget_kib=1":
-  // larger values avoid second search passes, smaller ones exercise them;
-  // "lists=1" has the list kernels search dense active sets too
+  // larger values avoid second search passes, smaller ones exercise them.
+  // For tests: "lists=1" has the list kernels search dense active sets too,
+  // "wstack" and "tlarge" bound the first node stack of the group walk and the
+  // tile groups with room in the large form
   if (const char *env = getenv("PHSPH_CAPS")) {
     std::string spec(env);
     size_t pos = 0;

@@ -38,9 +38,9 @@ struct DBuf {
   }
 };
 
-// Nodes of at most this many particles are built inside one workgroup;
-// larger nodes take the chunked large-node phase (which also forms their
-// second moments under self-gravity).
+// Nodes of at most this many particles are built in LDS by one workgroup
+// (k_subtrees); larger ones are split in memory, by one workgroup or chunk by
+// chunk (tree.hip), which also forms their second moments under self-gravity.
 constexpr int TREE_SUB_MAX = 1024;
 
 // One node of the tree build's large-node phase (more particles than one

@@ -1,9 +1,9 @@
 // dens_tile.hip -- neighbour search and h-rho iteration of dense active sets:
 // one workgroup per tree node of at most 64 or 80 particles (tile.h).
 //
-// The neighbour sets, iteration counts and Newton steps are those of
-// k_dens_iter (density.hip), which remains for sparse active sets, for what
-// does not fit a tile and for the particles that are run again.
+// The neighbour sets, iteration counts and Newton steps are those of the list
+// kernels (density.hip): k_dens_solo for sparse active sets and for the particles
+// that are run again, k_dens_iter for dense sets that do not go by tile.
 #include "dens_tile.h"
 
 #include <algorithm>
@@ -27,10 +27,11 @@
 //     Hits are packed into the particle's list in candidate order.
 //  3. FP64 distances into registers, list to memory, Newton iterations.
 //
-// Bound by vector instructions: 83 % of the issue slots at 4600 per wavefront
-// of 16 particles on the 8M-particle box (5.4 ms) with an FP64 test and the
-// kernel evaluated per neighbour; 3.9 ms now (10.6 ms as a search and iteration
-// over per-lane lists).
+// Bound by vector instructions in the four-wavefront form: 90 % of the issue
+// cycles at 3600 per wavefront of 16 particles on the 8M-particle box, 3.9 ms
+// (5.4 with an FP64 test and the kernel evaluated per neighbour, 10.6 as a
+// search and iteration over per-lane lists).  The quintic five-wavefront form
+// has one workgroup on a CU (tile.h) and 28 % of them: 2.9 ms on the 1.1M tube.
 //
 // Offsets.  get_sep (kdtree.F90:1468-1501) takes a leaf's offset from the two
 // leaf centres.  Here it is taken from the group's box centre, which gives the

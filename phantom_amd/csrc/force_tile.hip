@@ -21,9 +21,12 @@ struct ForceCap {
 // bytes (MHD + dust 176) from LDS instead of eight (thirteen) 16-byte loads
 // whose 64 lanes go to 64 cache lines each.  FP64 records are staged by eight
 // lanes each, one 128-byte line per record and load.
-// Bound by FP64 vector instructions and LDS reads.  8M-particle box 4.7 ms (8.1
+// Wavefronts wait 60 to 70 % of their time (the records of a chunk and the
+// barriers around them) at two to three a SIMD; FP64 vector instructions take
+// 42 to 58 % of the issue cycles.  8M-particle box 4.7 ms (8.1
 // ms as a list kernel, which its gathers bound), 2M particles with MHD and
-// dust 5.1 ms (8.2), 1M quintic 2.6 ms (3.35), 850k mixed 0.66 ms (0.92).
+// dust 5.1 ms (8.2), 1M quintic 2.6 ms (3.35), 850k mixed 0.66 ms (0.92; the
+// mixed form reads its FP32 records into FP64 ones and is no faster than FP64).
 template <int K, int W, bool MHD, bool DUST, bool THERMAL, bool MIXED>
 __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu((ForceCap<MHD, DUST>::WPE))))
 k_force_tile(DevConst dc, int ngroups, const int32_t *__restrict__ act, TileLists tl, const int32_t *__restrict__ t_nl,

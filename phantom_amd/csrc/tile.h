@@ -33,6 +33,9 @@ enum { TILE_4 = 0, TILE_5 = 1, TILE_BIG = 2 };
 // uniform set needs 430 and 73 (cubic, search radius 1.03 R h) or 630 and 123
 // (quintic).  The limits let the LDS of a CU hold 16 (cubic, TILE_4), 15
 // (cubic, TILE_5), 12 (quintic, TILE_4) and 10 (quintic, TILE_5) wavefronts.
+// Of five wavefronts two share a SIMD, so that its registers allow half as many
+// workgroups as wavefronts: two with the cubic (109 registers) and one with the
+// quintic kernel (145; 1.2 wavefronts per SIMD measured, 3.0 with TILE_4).
 // TILE_BIG has two wavefronts that take 16 particles after 16 and keeps its
 // lists in LDS only; what does not fit that goes to the list kernels.
 template <int K, int V>

@@ -1325,7 +1325,7 @@ __global__ void __launch_bounds__(MID_BS) k_mid(DevConst dc, double *tx, double 
 // minima and the partition run across the lanes (the partition as the
 // permutation of sort_particles_in_cell, see k_bn_pcount), and the four running
 // sums are four dependent chains in the lanes, one each where there are four.
-// Latency-bound by the chains: 1.94 ms on 8.4M particles, 0.36 ms on the 1M
+// Latency-bound by the chains: 1.94 ms on 8.4M particles, 0.38 ms on the 1M
 // polytrope; one thread per node of up to 64 particles took 2.82 and 0.87 (16 to
 // 64 lanes of 256 busy, reads of nodes of equal size in one LDS bank), and one
 // launch per level 0.70 on the polytrope, whose nodes get small at three levels.
