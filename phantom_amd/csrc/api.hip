@@ -989,8 +989,10 @@ int phsph_get_search_stats(phsph_ctx *c, int32_t *tiles, int32_t *large, int32_t
   if (force_tiles) *force_tiles = c->stat_force_tiles;
   if (large) {
     *large = 0;
-    if (c->stat_tiles > 0)
+    if (c->stat_tiles > 0) {
+      PH_HIPCHECK(c, hipSetDevice(c->device));
       PH_HIPCHECK(c, hipMemcpy(large, c->tg_big.p + c->stat_tiles, sizeof(int32_t), hipMemcpyDeviceToHost));
+    }
   }
   return PHSPH_OK;
 }
