@@ -508,7 +508,7 @@ int phsph_step_graph(phsph_ctx *ctx, const phsph_step_state *state,
  * per-XCD work queues (0: one group per wavefront).  Every configuration
  * gives bit-identical results.  By default the first densityiterate of a
  * context with at least 32768 active particles times each configuration
- * once on the caller's own particles (on up to 262144 of them, spread over
+ * once on the caller's own particles (on up to 131072 of them, spread over
  * the set, where tiles search the dense set) and keeps the fastest.
  * phsph_set_tuning fixes a configuration (cl = 0 asks for a new tuning on
  * the next large call); phsph_get_tuning returns the current one, whether

@@ -1429,8 +1429,9 @@ __global__ void k_sample_act(int nseg, int nact, const int32_t *__restrict__ fro
 // The autotuner of a set that tiles search: its configurations are for the
 // particles that tiles hand back and for large force lists, so a sample of the
 // groups does, with lists that are freed again.  All groups of 8.4M particles
-// took 200 ms and left 12.9 GB with the context; the sample takes 11 ms.
-constexpr int TUNE_SAMPLE = 1 << 18;
+// took 200 ms and left 12.9 GB with the context; the sample takes 7 ms (28 ms on
+// the 1.1M tube).
+constexpr int TUNE_SAMPLE = 1 << 17;
 static int tune_beside_tiles(phsph_ctx *c, int icall, double rfac, double lmargin, bool widen, bool &overflow) {
   hipStream_t s = c->stream;
   const int nact = c->nact_dens, nseg = std::min(nact, TUNE_SAMPLE) / GROUP;
@@ -1638,14 +1639,15 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
     if (!by_tile) {
       PH_HIPCHECK(c, LB.ensure((size_t)list_cap(dlist) * na + 1));
       DBuf<double> &R2B = attempt == 0 ? c->nr2 : c->nr2_r;
-      if (c->tune.r2 || c->tune_mode == TUNE_PENDING)
-        PH_HIPCHECK(c, R2B.ensure((size_t)list_cap(dlist) * na + 2));
+      const bool tuning = attempt == 0 && c->tune_mode == TUNE_PENDING && na >= TUNE_MIN_ACTIVE;
+      const bool solo = !tuning && 2 * (int64_t)na < n;
+      if (tuning || (!solo && c->tune.r2)) PH_HIPCHECK(c, R2B.ensure((size_t)list_cap(dlist) * na + 2));
       rc = walk_groups(c, 0, rfac * lmargin, c->th_in.p, widen ? c->hmax0.p : nullptr);
       if (rc) return rc;
       hipLaunchKernelGGL(k_zero_i32, dim3(nblocks(n, 256)), dim3(256), 0, s, c->tmpi.p, n, 0);
       PH_HIPCHECK(c, dev_set(c, c->counters.p, &zero, sizeof(int32_t)));
       const IterLaunch L{c, s, c->ngroups, icall, rfac, na, lmargin, dlist, widen, LB.p, R2B.p, TNL.p, THS.p, THF.p};
-      if (attempt == 0 && c->tune_mode == TUNE_PENDING && na >= TUNE_MIN_ACTIVE) {
+      if (tuning) {
         tuned_now = true;
         rc = tune_density_iter(c, L);  // times every configuration, keeps the fastest
         if (rc) return rc;
@@ -1658,7 +1660,7 @@ int dens_run(phsph_ctx *c, int icall, const DensIOArgs &a) {
         // 7.2); on all particles the list kernel is as fast with the quintic
         // (5.7 and 5.8 ms on 2M) and faster with the cubic kernel (10.6 and 15.4
         // ms on 8.4M)
-        if (2 * (int64_t)na < n) launch_dens_solo(L);
+        if (solo) launch_dens_solo(L);
         else launch_dens_iter(c->tune, L);
       }
     }
