@@ -553,8 +553,8 @@ int phsph_get_force_stats(phsph_ctx *ctx, int64_t *npairs);
  * `tiles` tree nodes searched by one workgroup each with their candidates in
  * LDS (0: neighbour lists of all active particles), `large` of them in the
  * form that has the LDS of a whole CU, `again` active particles run again by
- * lists (with the padding of their groups), and `deep` tree walks since then
- * of which some group needed the full node stack.  `force_tiles`: nodes whose
+ * lists, and `deep` tree walks since then of which some group needed the full
+ * node stack.  `force_tiles`: nodes whose
  * tiles the last force call took its neighbours from (0: lists).  Any pointer
  * may be null.
  */
